@@ -350,7 +350,8 @@ int supersonic_attn_gfx950_mixed(
  * memory of at least supersonic_attn_gfx950_qkv_proj_workspace_size() bytes,
  * zero-filled before its first use and not written by the caller between calls
  * (split-k arrival counters, which every call leaves at zero, and the GEMM's
- * tail hand-over counts, which every call leaves pairwise equal);
+ * tail hand-over counts, which every call leaves pairwise equal; a workspace
+ * below the size leaves a k split out, but not the tail's);
  * calls sharing it must not overlap.  NULL: library-owned buffers per device
  * (grown on demand; overlapping calls on one device then race). */
 size_t supersonic_attn_gfx950_qkv_proj_workspace_size(

@@ -324,7 +324,7 @@ constexpr int kWorkspacePrefill = 1;
 constexpr int kWorkspaceProj = 2;    // scratch rows: the o_proj GEMM output (hipBLASLt path), qkv_proj normed rows
 constexpr int kWorkspaceProjLt = 3;  // hipBLASLt workspace
 constexpr int kWorkspaceSkinny = 4;  // split-k partials and arrival counters of the o_proj kernel
-constexpr int kWorkspaceGemm = 5;    // tail-split partials and flags of the hand-written GEMM
+constexpr int kWorkspaceGemm = 5;    // split partials and counts of the hand-written GEMMs
 constexpr int kWorkspaceRope = 6;    // qkv_proj_rope: per-head counters (zero between calls), then rows
 constexpr int kWorkspaceMixed = 7;   // mixed step: the prefill's claim counters (zero between calls)
 constexpr int kWorkspaceSlots = 8;

@@ -30,19 +30,30 @@ struct GemmArgs {
     size_t ws_bytes = 0;
 };
 
-constexpr size_t kGemmFlagBytes = 8192;  // tail counts, two per tile (<= 1024 tail tiles)
+// Workspace of a projection's split work: a header of counts at fixed places,
+// whatever the shape, then the partials.  Every call leaves the tail's two
+// counts of a tile equal and the arrival counters at zero, so calls of
+// different shapes can follow each other on one workspace.
+constexpr size_t kGemmFlagBytes = 8192;         // tail counts, two per tile (<= 1024 tail tiles)
+constexpr size_t kGemmArrivalBytes = 64 << 10;  // split-k arrival counters, one per tile or column block
+constexpr size_t kGemmPartOff = kGemmFlagBytes + kGemmArrivalBytes;
 // Workspace bytes of the tail split for `tail` tiles.
-inline size_t gemm_tail_bytes(int tail) { return kGemmFlagBytes + static_cast<size_t>(tail) * 8 * 32 * 64 * 16; }
-// Workspace bytes for the tail split of a GEMM of m rows and the given
-// column segments on a GPU of `cus` CUs (256 on MI355X); 0 when it has no
-// tail to split.
-inline size_t gemm_ws_bytes(int m, int nseg, const int* n, int cus = 256) {
-    int64_t nt = 0;
-    for (int s = 0; s < nseg; ++s) nt += (n[s] + 255) / 256;
-    const int64_t tiles = static_cast<int64_t>((m + 255) / 256) * nt;
-    const int tail = static_cast<int>(tiles % cus);
-    return tiles > cus && tail > 0 && 2 * tail <= cus ? gemm_tail_bytes(tail) : 0;
+inline size_t gemm_tail_bytes(int tail) { return kGemmPartOff + static_cast<size_t>(tail) * 8 * 32 * 64 * 16; }
+
+// How a GEMM runs: bm x bn tiles, the last split_tiles of them over ks slices
+// of k.  256 x 256 is gemm.hip's kernel (with its own tail split), the others
+// gemm_tile.hip's.
+struct GemmPlan {
+    int bm = 256, bn = 256, ks = 1, split_tiles = 0;
+};
+GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch = 1);
+inline size_t gemm_split_bytes(const GemmPlan& p) {
+    return p.ks > 1 ? kGemmPartOff + static_cast<size_t>(p.split_tiles) * p.ks * p.bm * p.bn * sizeof(float) : 0;
 }
+// Workspace bytes of a GEMM of m rows over k and the given column segments on
+// a GPU of 256 CUs: the tail split's or the k split's; 0 when it has neither.
+size_t gemm_ws_bytes(int m, int k, int nseg, const int* n);
+int gemm_tile(hipStream_t st, const GemmArgs& g, const GemmPlan& plan);
 
 // Launches on `st`; 0 on success.  Requires k % 8 == 0 and 16-byte aligned
 // rows (lda % 8 == 0).

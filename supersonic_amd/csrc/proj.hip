@@ -75,7 +75,7 @@ constexpr int kSkinnyCB = 1;                        // 16-column blocks per work
 constexpr int kSkinnyKP = kSkinnyWaves / kSkinnyCB;  // k parts per workgroup (one per wave group)
 constexpr int kSkinnyMaxM = 64;                     // hard limit (4 row blocks)
 constexpr int kSkinnyDefaultM = 12;                 // measured crossover with hipBLASLt
-constexpr size_t kSkinnyArrivalBytes = 64 << 10;  // counters at a fixed offset, ahead of the partials
+constexpr size_t kSkinnyArrivalBytes = kGemmArrivalBytes;
 
 
 template <typename OT, bool RES>
@@ -193,11 +193,15 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_kernel(SkinnyParams 
 // normed = bf16(x * rsqrt(mean(x^2) + eps) * (1 + w)): one 256-thread
 // workgroup per row, 8 elements (16 or 32 bytes) per thread and chunk, every
 // chunk's load issued before the reduction (k <= 8192 in one pass of
-// registers; longer rows re-read their chunks from cache).
+// registers; longer rows re-read their chunks from cache).  Also clears the
+// arrival counters of the split-k GEMM that follows: in the Q/K/V workspace
+// they sit behind the normed rows, so a call with another row count may have
+// written there.
 template <typename XT>
 __global__ __launch_bounds__(256) void input_norm_kernel(int rows, int k, float eps, const XT* x, const uint16_t* w,
-                                                         uint16_t* out) {
+                                                         uint16_t* out, unsigned* clear, int n_clear) {
     __shared__ float part[4];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n_clear; i += gridDim.x * 256) clear[i] = 0u;
     constexpr int CH = 4;  // chunks of 8 held per thread
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -431,7 +435,7 @@ size_t skinny_ws_bytes(int m, int k, int64_t wgs) {
     while (T / (ks * 2) >= kSkinnyKP * 8) ks *= 2;
     if (ks == 1 || wgs > static_cast<int64_t>(kSkinnyArrivalBytes / 4)) return 0;
     const int MB = (m + 15) / 16;
-    return kSkinnyArrivalBytes + static_cast<size_t>(wgs) * ks * kSkinnyCB * MB * 256 * sizeof(float);
+    return kGemmPartOff + static_cast<size_t>(wgs) * ks * kSkinnyCB * MB * 256 * sizeof(float);
 }
 
 // ws: the skinny_ws_bytes() region (arrival counters zero between calls), or
@@ -447,12 +451,12 @@ int launch_skinny(int dev, hipStream_t st, int batch, SkinnyParams p, uint8_t* w
     p.ks_count = ks;
     p.slice = (T + ks - 1) / ks;
     if (ks > 1) {
-        const size_t need = kSkinnyArrivalBytes + static_cast<size_t>(wgs) * ks * kSkinnyCB * MB * 256 * sizeof(float);
+        const size_t need = kGemmPartOff + static_cast<size_t>(wgs) * ks * kSkinnyCB * MB * 256 * sizeof(float);
         if (!ws) ws = static_cast<uint8_t*>(device_workspace(dev, need, kWorkspaceSkinny));
         else if (ws_bytes < need) return SUPERSONIC_ERR_WORKSPACE;
         if (!ws) return SUPERSONIC_ERR_WORKSPACE;
-        p.arrivals = reinterpret_cast<unsigned*>(ws);
-        p.part = reinterpret_cast<float*>(ws + kSkinnyArrivalBytes);
+        p.arrivals = reinterpret_cast<unsigned*>(ws + kGemmFlagBytes);
+        p.part = reinterpret_cast<float*>(ws + kGemmPartOff);
     }
     const dim3 grid(ncb, ks, batch), blk(64 * kSkinnyWaves);
     switch (MB) {
@@ -547,17 +551,30 @@ int gemm_segments(int dev, hipStream_t st, int m, int k, const void* a, int nseg
         g.n[i] = n[i];
     }
     g.epilogue = epilogue;
-    const size_t need = gemm_ws_bytes(m, nseg, n);
+    const size_t need = gemm_ws_bytes(m, k, nseg, n);
     if (need > 0) {
         if (ws) {
-            if (ws_bytes < need) return 1;
+            // a tail split's region that is missing is the caller's error; a
+            // k split without room runs its tiles whole
+            if (gemm_plan(m, k, nseg, n).bn == 256 && ws_bytes < need) return 1;
             g.ws = ws;
+            g.ws_bytes = ws_bytes;
         } else {
-            g.ws = device_workspace(dev, need, kWorkspaceGemm);  // zero-filled once; each call leaves the tail counts equal
+            g.ws = device_workspace(dev, need, kWorkspaceGemm);
+            g.ws_bytes = g.ws ? need : 0;
         }
-        g.ws_bytes = g.ws ? need : 0;
     }
     return gemm_bt(st, g);
+}
+
+// Arrival counters that the GEMM of this shape takes in the caller's region
+// (NULL: none of the caller's): their number, and where they are.
+int split_counters(int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, unsigned** at) {
+    if (!ws || use_hipblaslt()) return 0;
+    const GemmPlan plan = gemm_plan(m, k, nseg, n);
+    if (plan.ks == 1 || ws_bytes < gemm_split_bytes(plan)) return 0;
+    *at = reinterpret_cast<unsigned*>(ws + kGemmFlagBytes);
+    return plan.split_tiles;
 }
 
 bool make_layout(hipblasLtMatrixLayout_t* l, uint64_t rows, uint64_t cols, int64_t ld, int batch, int64_t stride) {
@@ -668,7 +685,7 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
             g.w_bs = static_cast<int64_t>(n) * k;
             g.o_bs = static_cast<int64_t>(m) * n;
             if (batch == 1) {
-                g.ws_bytes = gemm_ws_bytes(m, 1, &n);
+                g.ws_bytes = gemm_ws_bytes(m, k, 1, &n);
                 if (g.ws_bytes > 0) g.ws = device_workspace(dev, g.ws_bytes, kWorkspaceGemm);
                 if (!g.ws) g.ws_bytes = 0;
             }
@@ -715,7 +732,7 @@ inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255);
 // the hipBLASLt workspace.
 size_t o_proj_ws_bytes(int m, int n, int k) {
     if (m <= skinny_max_m()) return skinny_ws_bytes(m, k, (n + kSkinnyCols - 1) / kSkinnyCols);
-    if (!use_hipblaslt()) return 256 + gemm_ws_bytes(m, 1, &n);  // the GEMM adds into the hidden rows in place
+    if (!use_hipblaslt()) return 256 + gemm_ws_bytes(m, k, 1, &n);  // the GEMM adds into the hidden rows in place
     return align256(static_cast<size_t>(m) * n * 2) + kLtWorkspace;
 }
 // Workspace of the qkv entry point: the normed rows, then the streaming
@@ -724,7 +741,7 @@ size_t qkv_ws_bytes(int m, int k, int nq, int nkv) {
     const size_t normed = align256(static_cast<size_t>(m) * k * 2);
     if (m <= skinny_max_m()) return normed + skinny_ws_bytes(m, k, nq / kSkinnyCols + 2 * (nkv / kSkinnyCols));
     const int ns[3] = {nq, nkv, nkv};
-    return normed + (use_hipblaslt() ? lt_ws_bytes() : gemm_ws_bytes(m, 3, ns));
+    return normed + (use_hipblaslt() ? lt_ws_bytes() : gemm_ws_bytes(m, k, 3, ns));
 }
 }  // namespace ssa
 
@@ -851,20 +868,25 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
         normed = static_cast<uint16_t*>(device_workspace(dev, static_cast<size_t>(m) * k * 2, kWorkspaceProj));
     }
     if (!normed) return SUPERSONIC_ERR_WORKSPACE;
+    // the three matrices as one column space of the weight-streaming kernel, or
+    // as column segments of one GEMM
+    const int ns[3] = {nq, nkv, nkv};
+    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0;
+    unsigned* clear = nullptr;
+    const int n_clear = skinny ? 0 : split_counters(m, k, 3, ns, rest, rest_bytes, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {
         const dim3 grid(m), blk(256);
         if (f32)
             hipLaunchKernelGGL((input_norm_kernel<float>), grid, blk, 0, st, m, k, eps, static_cast<const float*>(hidden),
-                               static_cast<const uint16_t*>(input_norm_w), normed);
+                               static_cast<const uint16_t*>(input_norm_w), normed, clear, n_clear);
         else
             hipLaunchKernelGGL((input_norm_kernel<bf16_t>), grid, blk, 0, st, m, k, eps,
-                               static_cast<const bf16_t*>(hidden), static_cast<const uint16_t*>(input_norm_w), normed);
+                               static_cast<const bf16_t*>(hidden), static_cast<const uint16_t*>(input_norm_w), normed, clear, n_clear);
         if (hipGetLastError() != hipSuccess) return SUPERSONIC_ERR_LAUNCH;
     }
-    if (skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0) {
-        // the three matrices as one column space of the weight-streaming kernel
+    if (skinny) {
         SkinnyParams p{};
         p.x = normed;
         p.w[0] = static_cast<const uint16_t*>(q_proj_w);
@@ -887,10 +909,8 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
             if (rc) return rc;
         }
     } else {
-        // GEMM-sized: the three matrices as column segments of one GEMM
         const void* wts[3] = {q_proj_w, k_proj_w, v_proj_w};
         void* os[3] = {q_proj_out, k_out, v_out};
-        const int ns[3] = {nq, nkv, nkv};
         if (!use_hipblaslt()) {
             if (gemm_segments(dev, st, m, k, normed, 3, wts, os, ns, kGemmStore, ws ? rest : nullptr, rest_bytes) != 0)
                 return SUPERSONIC_ERR_LAUNCH;
@@ -994,21 +1014,33 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
                            reinterpret_cast<uintptr_t>(q_proj_w) | reinterpret_cast<uintptr_t>(k_proj_w) |
                            reinterpret_cast<uintptr_t>(v_proj_w) | reinterpret_cast<uintptr_t>(q_out) |
                            reinterpret_cast<uintptr_t>(k_out)) & 15) == 0;
+    // the unfused path's regions: q_proj and the raw k / v rows, then the
+    // projection's own workspace
+    uint16_t* qp = reinterpret_cast<uint16_t*>(rest);
+    uint16_t* kr = reinterpret_cast<uint16_t*>(rest + align256(static_cast<size_t>(m) * nq * 2));
+    uint16_t* vr = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(kr) + align256(static_cast<size_t>(m) * nkv * 2));
+    uint8_t* pws = reinterpret_cast<uint8_t*>(vr) + align256(static_cast<size_t>(m) * nkv * 2);
+    const size_t pws_bytes = ws + need > pws ? static_cast<size_t>(ws + need - pws) : 0;
+    const int ncb = (nq + 2 * nkv) / kSkinnyCols;
+    const bool fused = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
+                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4);
+    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0;
+    const int ns[3] = {nq, nkv, nkv};
+    unsigned* clear = nullptr;
+    const int n_clear = fused || skinny ? 0 : split_counters(m, k, 3, ns, workspace ? pws : nullptr, pws_bytes, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {
         const dim3 grid(m), blk(256);
         if (f32)
             hipLaunchKernelGGL((input_norm_kernel<float>), grid, blk, 0, st, m, k, eps, static_cast<const float*>(hidden),
-                               static_cast<const uint16_t*>(input_norm_w), normed);
+                               static_cast<const uint16_t*>(input_norm_w), normed, clear, n_clear);
         else
             hipLaunchKernelGGL((input_norm_kernel<bf16_t>), grid, blk, 0, st, m, k, eps,
-                               static_cast<const bf16_t*>(hidden), static_cast<const uint16_t*>(input_norm_w), normed);
+                               static_cast<const bf16_t*>(hidden), static_cast<const uint16_t*>(input_norm_w), normed, clear, n_clear);
         if (hipGetLastError() != hipSuccess) return SUPERSONIC_ERR_LAUNCH;
     }
-    const int ncb = (nq + 2 * nkv) / kSkinnyCols;
-    if (aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
-        Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4)) {
+    if (fused) {
         SkinnyLdsParams p{};
         p.x = normed;
         p.w[0] = static_cast<const uint16_t*>(q_proj_w);
@@ -1026,12 +1058,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
         if (hipGetLastError() != hipSuccess) return SUPERSONIC_ERR_LAUNCH;
     } else {
         // plain projections into the workspace, then one wave per (row, head)
-        uint16_t* qp = reinterpret_cast<uint16_t*>(rest);
-        uint16_t* kr = reinterpret_cast<uint16_t*>(rest + align256(static_cast<size_t>(m) * nq * 2));
-        uint16_t* vr = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(kr) + align256(static_cast<size_t>(m) * nkv * 2));
-        uint8_t* pws = reinterpret_cast<uint8_t*>(vr) + align256(static_cast<size_t>(m) * nkv * 2);
-        const size_t pws_bytes = ws + need > pws ? static_cast<size_t>(ws + need - pws) : 0;
-        if (skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0) {
+        if (skinny) {
             SkinnyParams p{};
             p.x = normed;
             p.w[0] = static_cast<const uint16_t*>(q_proj_w);
@@ -1053,7 +1080,6 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
         } else {
             const void* wts[3] = {q_proj_w, k_proj_w, v_proj_w};
             void* os[3] = {qp, kr, vr};
-            const int ns[3] = {nq, nkv, nkv};
             if (!use_hipblaslt()) {
                 if (gemm_segments(dev, st, m, k, normed, 3, wts, os, ns, kGemmStore, workspace ? pws : nullptr,
                                   pws_bytes) != 0)

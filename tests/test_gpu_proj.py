@@ -398,6 +398,83 @@ def test_decode_layer_chain_fused_projection():
         f"chain: max {d.max().item():.3e} mean {d.mean().item():.3e}"
 
 
+# Rows between the weight-streaming kernels and full chunks: every tile size of
+# the smaller-tile GEMM at its edges, whole and split along k, with columns
+# and k that end inside a tile (1000, 2056) and rows that take no 16-byte chunks (1004).
+@pytest.mark.parametrize("rows", [13, 32, 33, 65, 129, 200, 201, 257, 600, 601, 1000, 1300])
+@pytest.mark.parametrize("hidden_dim,attn_dim,hdt", [(1024, 2048, torch.bfloat16), (1000, 2056, torch.float32),
+                                                     (1004, 328, torch.bfloat16), (2560, 520, torch.float32)])
+def test_o_proj_mid_rows(rows, hidden_dim, attn_dim, hdt):
+    announce(f"o_proj mid rows={rows} {attn_dim}->{hidden_dim} {hdt}")
+    g = gen(91)
+    attn = O.randn_bf16(g, rows, attn_dim)
+    w = O.randn_bf16(g, hidden_dim, attn_dim, std=attn_dim ** -0.5)
+    hidden = O.randn_bf16(g, rows, hidden_dim)
+    ref = O.o_proj_residual(attn.float(), w, hidden)
+    ad, wd = attn.to(DEV), w.to(DEV)
+    size = K.o_proj_workspace_size(rows, hidden_dim, attn_dim)
+    got = []
+    for n in (None, size, 256):  # the library's, the caller's, one without room for a split
+        h = hidden.to(DEV).to(hdt)
+        ws = None if n is None else torch.zeros(n, dtype=torch.uint8, device=DEV)
+        for _ in range(2 if n else 1):  # twice: the counters are left at zero
+            h.copy_(hidden)
+            K.o_proj_residual(0, ad, wd, h, workspace=ws)
+        torch.cuda.synchronize()
+        got.append(h.float().cpu())
+        # two roundings: the sum's bf16 ulp and the residual add's
+        assert_ulps(got[-1], ref, 2 * ulp(torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())) + 1e-6,
+                    f"o_proj ws={n}")
+    assert torch.equal(got[0], got[1])  # the same split, slices added in order
+
+
+@pytest.mark.parametrize("rows,hid,nq,nkv", [(13, 1024, 4096, 512), (40, 1024, 520, 72), (129, 512, 1024, 256),
+                                             (300, 2048, 1024, 256), (700, 1024, 1024, 136), (1030, 512, 4096, 256)])
+def test_qkv_proj_mid_rows(rows, hid, nq, nkv):
+    """Three column segments that end inside a tile; the workspace comes from a larger call and holds its rows, so the
+    counters behind the normed rows are not zero when the call begins."""
+    announce(f"qkv mid rows={rows} {hid}->{nq}+2x{nkv}")
+    g = gen(92)
+    hidden = O.randn_bf16(g, rows, hid)
+    nw = O.randn_bf16(g, hid, std=0.1)
+    wq, wk, wv = (O.randn_bf16(g, n, hid, std=hid ** -0.5) for n in (nq, nkv, nkv))
+    refs = O.qkv_proj(hidden.float(), nw, wq, wk, wv)
+    args = [t.to(DEV) for t in (hidden, nw, wq, wk, wv)]
+    size = K.qkv_proj_workspace_size(rows, hid, nq, nkv)
+    dirty = torch.zeros(size, dtype=torch.uint8, device=DEV)
+    dirty[rows * hid * 2 + 8192:] = 1
+    for ws in (None, torch.zeros(size, dtype=torch.uint8, device=DEV), dirty):
+        outs = [torch.full((rows, w.shape[0]), float("nan"), dtype=torch.bfloat16, device=DEV) for w in (wq, wk, wv)]
+        K.qkv_proj(0, *args, *outs, workspace=ws)
+        torch.cuda.synchronize()
+        for name, out, ref in zip("qkv", outs, refs):
+            out = out.cpu()
+            big = torch.maximum(out.float().abs(), ref.float().abs())
+            # a normed element one bf16 ulp away (hardware rsqrt) moves an output by up to 2^-5 |w|, below 2^-7 here
+            assert_ulps(out, ref, 2 * ulp(big) + 2.0 ** -7, f"qkv mid {name}")
+            assert (out.float() == ref).float().mean().item() > 0.9, name
+
+
+def test_projections_share_a_workspace_over_row_counts():
+    """One o_proj workspace for calls of different row counts, a tail split among them."""
+    announce("o_proj one workspace, many row counts")
+    g = gen(93)
+    hid, adim = 4608, 512
+    w = O.randn_bf16(g, hid, adim, std=adim ** -0.5)
+    wd = w.to(DEV)
+    counts = (40, 4096, 8, 300, 40)
+    ws = torch.zeros(max(K.o_proj_workspace_size(r, hid, adim) for r in counts), dtype=torch.uint8, device=DEV)
+    for r in counts:
+        attn, hidden = O.randn_bf16(g, r, adim), O.randn_bf16(g, r, hid)
+        h = hidden.to(DEV)
+        K.o_proj_residual(0, attn.to(DEV), wd, h, workspace=ws)
+        torch.cuda.synchronize()
+        ref = O.o_proj_residual(attn.float(), w, hidden)
+        big = torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())
+        assert_ulps(h.float().cpu(), ref, 2 * ulp(big) + 1e-6, f"o_proj shared ws rows={r}")
+    assert K.wait_status() == 0
+
+
 def test_gemm_tail_expired_handover_is_reported(monkeypatch):
     """The host presets one tail tile's consumed count ahead of its produced count,
     so that tile's second k half never sees its first half, and shortens the
