@@ -254,8 +254,9 @@ int supersonic_attn_gfx950_decode_attend(
 
 /* Bytes of workspace supersonic_attn_gfx950_prefill needs for a chunk of
  * chunk_len tokens starting at chunk_start (the staged V^T rows of every
- * position, and for an fp8 cache the bf16 K rows the attention reads).  No
- * GPU call. */
+ * position, for an fp8 cache the bf16 K rows the attention reads, and for
+ * chunks of up to 8192 / kv_heads tokens the partial sums of a key split, at
+ * most 34 MB).  No GPU call. */
 size_t supersonic_attn_gfx950_prefill_workspace_size(
     int kv_dtype, size_t kv_heads, size_t head_dim, size_t chunk_len, size_t chunk_start);
 
@@ -267,7 +268,8 @@ size_t supersonic_attn_gfx950_prefill_workspace_size(
  * workspace: caller device memory of at least
  * supersonic_attn_gfx950_prefill_workspace_size() bytes (no allocation, no
  * synchronisation: the call can be captured into a HIP graph; calls sharing a
- * workspace must not overlap), or NULL for a library-owned buffer per device
+ * workspace must not overlap; without the room for a key split the chunk runs
+ * unsplit), or NULL for a library-owned buffer per device
  * (grown on demand with a device synchronisation; overlapping calls on one
  * device then race). */
 int supersonic_attn_gfx950_prefill(

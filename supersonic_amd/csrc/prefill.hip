@@ -23,6 +23,11 @@
 //   skips the MFMA work of tiles past its own last row; only tiles that cross
 //   the diagonal or the kv_len edge are masked.  Query tiles run longest
 //   first, the heads of one kv head on one XCD.
+//   Chunks of few items and many keys (a short chunk behind a long prefix) run
+//   as pieces of the items' keys, one a CU, with the query heads of a kv head
+//   packed into the 128 rows, and prefill_merge_kernel (plan_key_split): 333
+//   rows after 7001 cached tokens, 16/2 heads: 147 -> 57 us.
+#include <algorithm>
 #include <cstdlib>
 
 #include <type_traits>
@@ -42,9 +47,24 @@ struct PrefillParams {
     int vt_ld;
     int Hq, Hkv, G, S, L, off;
     float scale_log2;
-    int nqt;             // query tiles of 128 rows
+    int nqt;             // query tiles of 128 rows (of a query head; with a key split of a kv head)
     int B;               // sequences
     int n_wg;            // workgroups of the persistent grid
+    // Key split (piece 0: none).  A kv head's rows are its G query heads at S
+    // positions, R = S * G rows in all, row r = position r / G of query head
+    // kvh * G + r % G; an item's key tiles run as pieces of at most `piece`
+    // tiles, one piece a workgroup, which leave their sums here for
+    // prefill_merge_kernel, by workgroup slot: the unnormalised O in accumulator
+    // order ([slot][wave][16-dim block][lane] x 4 floats) and each row's (max, sum).
+    int piece;
+    int R;
+    int lists_log2;      // 1 << lists_log2 item lists (kv heads spread over the XCDs)
+    int W;               // workgroups of a list
+    int hpl, nb;         // kv heads of a list; items of a query tile in it, hpl * B
+    uint32_t g_mul;      // r / G = (2 r * g_mul >> 32) >> g_shift for r < 2^31:
+    int g_shift;         // g_mul = ceil(2^(31 + g_shift) / G), g_shift = ceil(log2 G)
+    float* part_o;
+    float* part_ml;
     // Dynamic schedule (NULL: the static one).  Per item list x (an XCD's, or
     // the single list) a claim counter at claims[32 x] and a finished-workgroup
     // counter at claims[32 (8 + x)], each on its own 128-byte line; both are
@@ -183,7 +203,69 @@ constexpr int kPrefillThreads = 64 * (kPrefillWaves + kCopyWaves);
 //                    weights (keys 4 g + i of the two 16-key blocks), and the A
 //                    operand (V^T) comes from two transposing LDS reads, each
 //                    giving a lane 4 consecutive keys of dim (l & 15).
-template <typename QT, int D, bool FUSED>
+// r / G by a multiplication: a division by a run-time value takes about 40
+// dependent instructions, and several of them ahead of an item's first copy
+// cost 2 us.
+__device__ __forceinline__ int div_g(const PrefillParams& p, int r) {
+    return static_cast<int>(__umulhi(2u * static_cast<uint32_t>(r), p.g_mul) >> p.g_shift);
+}
+// Item m of a list: its order index (query tiles from the last one on) and its
+// number within the query tile.
+__device__ __forceinline__ void split_item(const PrefillParams& p, int m, int& qi, int& idx) {
+    qi = m;
+    idx = 0;
+    if (p.nb > 1) {
+        qi = m / p.nb;
+        idx = m - qi * p.nb;
+    }
+}
+// 64-key tiles below the last row's causal limit of query tile qt.
+template <bool SPLIT>
+__device__ __forceinline__ int prefill_tiles(const PrefillParams& p, int qt) {
+    const int lim = min(p.L, p.off + (SPLIT ? div_g(p, min(qt * 128 + 128, p.R) - 1) + 1 : min(qt * 128 + 128, p.S)));
+    return lim > 0 ? (lim + 63) / 64 : 0;
+}
+// Pieces that n key tiles run as.
+__host__ __device__ __forceinline__ int prefill_pieces(int n, int piece) { return n > piece ? (n + piece - 1) / piece : 1; }
+
+// Slots of one list before its order index qi (query tiles from the last one
+// on), `nb` items a query tile; for the whole wave.
+__device__ __forceinline__ int prefill_slots_before(const PrefillParams& p, int qi, int nb) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+    for (int i = lane; i < qi; i += 64) n += prefill_pieces(prefill_tiles<true>(p, p.nqt - 1 - i), p.piece);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o);
+    return __builtin_amdgcn_readfirstlane(n) * nb;
+}
+// The piece in slot j of a list: order index of its query tile, its number
+// within the query tile's pieces; false past the last.
+__device__ __forceinline__ bool prefill_find_piece(const PrefillParams& p, int j, int nb, int& qi, int& at) {
+    const int lane = threadIdx.x & 63;
+    int before = 0;
+    for (int base = 0; base < p.nqt; base += 64) {
+        const int i = base + lane;
+        const int np = i < p.nqt ? prefill_pieces(prefill_tiles<true>(p, p.nqt - 1 - i), p.piece) * nb : 0;
+        int incl = np;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(incl, o);
+            incl += lane >= o ? x : 0;
+        }
+        const uint64_t hit = __ballot(before + incl > j);
+        if (hit) {
+            const int l = static_cast<int>(__builtin_ctzll(hit));
+            qi = __builtin_amdgcn_readfirstlane(base + l);
+            at = __builtin_amdgcn_readfirstlane(j - before - __shfl(incl - np, l));
+            return true;
+        }
+        before += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+    }
+    return false;
+}
+
+// SPLIT: one piece of an item a workgroup (PrefillParams::piece).
+template <typename QT, int D, bool FUSED, bool SPLIT>
 __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
     typedef typename Mfma16<QT>::op op_t;
@@ -200,14 +282,34 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     // XCD has its own item list holding the heads that share its kv heads, so
     // its L2 keeps their K/V.  Workgroup j of a list of W takes items j,
     // 2W-1-j, 2W+j, ...: a long item pairs with a short one and every
-    // workgroup gets about the same number of key tiles.
+    // workgroup gets about the same number of key tiles.  With a key split the
+    // lists hold kv heads, several XCDs to a list when there are fewer than 8.
     const int bid = blockIdx.x;
     const int hpx = p.Hq / 8;
-    const bool by_xcd = hpx > 0 && (p.Hq % 8) == 0 && (p.n_wg % 8) == 0;
-    const int j = by_xcd ? (bid >> 3) : bid;
-    const int W = by_xcd ? (p.n_wg >> 3) : p.n_wg;
+    const bool by_xcd = !SPLIT && hpx > 0 && (p.Hq % 8) == 0 && (p.n_wg % 8) == 0;
+    const int ll = p.lists_log2;
+    const int list = SPLIT ? bid & ((1 << ll) - 1) : (by_xcd ? bid & 7 : 0);
+    const int j = SPLIT ? (ll ? ((bid >> 3) << (3 - ll)) + ((bid & 7) >> ll) : bid) : (by_xcd ? (bid >> 3) : bid);
+    const int W = SPLIT ? p.W : (by_xcd ? (p.n_wg >> 3) : p.n_wg);
     const int hpi = by_xcd ? hpx : p.Hq;     // heads per item list
-    const int n_items = p.nqt * hpi * p.B;
+    const int n_items = p.nqt * (SPLIT ? p.nb : hpi * p.B);
+    // Key split: this workgroup's one piece, tiles [pt0, pt1) of item pm.
+    int pm = 0, pt0 = 0, pt1 = 0;
+    // one item, in a loop that the compiler takes for a loop: straight-line, it
+    // moves the epilogue's values across the key loop (54 spilled registers)
+    int one = 1;
+    if constexpr (SPLIT) asm volatile("" : "+s"(one));
+    if constexpr (SPLIT) {
+        int qi, at;
+        if (!prefill_find_piece(p, j, p.nb, qi, at)) return;  // the whole workgroup
+        const int n = prefill_tiles<true>(p, p.nqt - 1 - qi);
+        const int pn = prefill_pieces(n, p.piece);
+        int part, idx;
+        split_item(p, at, part, idx);
+        pm = qi * p.nb + idx;
+        pt0 = n * part / pn;
+        pt1 = n * (part + 1) / pn;
+    }
     // Dynamic schedule: the list's items are claimed one at a time from a
     // counter in list order (longest first), so workgroups that start late
     // (their CUs busy with other work when the grid was dispatched) take only
@@ -215,8 +317,8 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     // leaves it in claimed[(r + 1) & 1]; every reader is at least one
     // workgroup barrier behind the write.
     __shared__ int claimed[2];
-    const bool dyn = p.claims != nullptr;
-    unsigned* const ctr = dyn ? p.claims + 32 * (by_xcd ? (bid & 7) : 0) : nullptr;
+    const bool dyn = !SPLIT && p.claims != nullptr;
+    unsigned* const ctr = dyn ? p.claims + 32 * list : nullptr;
     auto claim_next = [&](const int slot) {
         if (wave == kPrefillWaves && (tid & 63) == 0) {
             claimed[slot] = static_cast<int>(__hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -224,20 +326,29 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
         }
     };
     // Item r of this workgroup (false past the last): 128 query rows `qt` of
-    // head h of sequence b.  The sequence of m is increasing (static schedule).
-    auto item_at = [&](const int r, int& qt, int& h, int& b) -> bool {
-        const int m = dyn ? claimed[r & 1] : ((r & 1) ? (r + 1) * W - 1 - j : r * W + j);
+    // head h (SPLIT: kv head h) of sequence b over key tiles [t0, t1).  The
+    // sequence of m is increasing (static schedule).
+    auto item_at = [&](const int r, int& qt, int& h, int& b, int& t0, int& t1) -> bool {
+        if (SPLIT && r >= one) return false;
+        const int m = SPLIT ? pm : (dyn ? claimed[r & 1] : ((r & 1) ? (r + 1) * W - 1 - j : r * W + j));
         if (m >= n_items) return false;
-        qt = p.nqt - 1 - m / (hpi * p.B);
-        const int rem = m % (hpi * p.B);
-        h = (by_xcd ? (bid & 7) * hpx : 0) + rem % hpi;
-        b = rem / hpi;
+        if constexpr (SPLIT) {
+            int qi, idx;
+            split_item(p, m, qi, idx);
+            qt = p.nqt - 1 - qi;
+            b = p.B > 1 ? idx / p.hpl : 0;
+            h = list * p.hpl + idx - b * p.hpl;
+            t0 = pt0;
+            t1 = pt1;
+        } else {
+            qt = p.nqt - 1 - m / (hpi * p.B);
+            const int rem = m % (hpi * p.B);
+            h = (by_xcd ? (bid & 7) * hpx : 0) + rem % hpi;
+            b = rem / hpi;
+            t0 = 0;
+            t1 = prefill_tiles<false>(p, qt);
+        }
         return true;
-    };
-    // 64-key tiles of query block qt: keys below the block's last row (causal).
-    auto tiles_of = [&](const int qt) -> int {
-        const int lim = min(p.L, p.off + min(qt * 128 + 128, p.S));
-        return lim > 0 ? (lim + 63) / 64 : 0;
     };
     // Tiles alternate between the two LDS stages across items: tile `it` of
     // an item that follows gt tiles goes to stage (gt + it + 1) & 1, so the
@@ -263,7 +374,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
         // c = (l & 7) ^ (4 (i & 1) + (l >> 4)) of dim 8 i + (l >> 3) (the
         // swizzle of the tile geometry); the staging buffer is zero past kv_len.
         auto issue_tile = [&](const int h, const int b, const int it, const int st) {
-            const int kvh = h / p.G;
+            const int kvh = SPLIT ? h : h / p.G;
             const uint16_t* vt_head = p.vt + (static_cast<int64_t>(b) * p.Hkv + kvh) * D * p.vt_ld;
             const int k0 = it * 64;
             const int64_t base = p.kv.row_uniform(b, kvh, k0, D) * 2;  // a tile lies inside one page
@@ -286,19 +397,19 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
         auto wait_vm0 = []() { __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8)); };
         // first tile of the first item that has keys at all
         auto issue_first = [&](int r, const int st) {
-            int qt, h, b;
-            for (; item_at(r, qt, h, b); ++r) {
-                if (tiles_of(qt) > 0) {
-                    issue_tile(h, b, 0, st);
+            int qt, h, b, t0, t1;
+            for (; item_at(r, qt, h, b, t0, t1); ++r) {
+                if (t1 > t0) {
+                    issue_tile(h, b, t0, st);
                     return;
                 }
                 if (dyn) return;  // only item r is claimed yet (and every item has tiles)
             }
         };
         issue_first(0, 1);
-        int gt = 0, qt, h, b;
-        for (int r = 0; item_at(r, qt, h, b); ++r) {
-            const int nt = tiles_of(qt);
+        int gt = 0, qt, h, b, t0, t1;
+        for (int r = 0; item_at(r, qt, h, b, t0, t1); ++r) {
+            const int nt = t1 - t0;
             // The next item is claimed as this one nears its end (at the
             // barrier of tile nt - 3, two barriers before the other copy
             // waves read the claim), so workgroups claim in the order they
@@ -312,7 +423,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
                 wait_vm0();
                 __builtin_amdgcn_s_barrier();
                 if (dyn && nt >= 3 && it == nt - 3) claim_next((r + 1) & 1);
-                if (it + 1 < nt) issue_tile(h, b, it + 1, (gt + it + 2) & 1);
+                if (it + 1 < nt) issue_tile(h, b, t0 + it + 1, (gt + it + 2) & 1);
                 else issue_first(r + 1, (gt + nt + 1) & 1);
             }
             __builtin_amdgcn_s_barrier();  // item end (the next tile needs no wait yet)
@@ -323,39 +434,44 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
             // This workgroup's claims are over (its last one failed); the
             // list's last workgroup to get here leaves both counters at zero.
             unsigned* const done = ctr + 32 * 8;
-            const unsigned wl = by_xcd ? static_cast<unsigned>(p.n_wg >> 3) : static_cast<unsigned>(p.n_wg);
-            if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == wl) {
+            if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == static_cast<unsigned>(W)) {
                 __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     };
-    // One work item = 128 query rows of one head of one sequence, run by the
-    // compute waves; gt = tiles of the workgroup's items before it.  A
-    // `return` inside ends the item, not the workgroup.
-    auto run_item = [&](const int qt, const int h, const int b, const int gt) {
+    // One work item = 128 query rows of one head (SPLIT: kv head) of one
+    // sequence, run by the compute waves over key tiles [t0, t1); gt = tiles of
+    // the workgroup's items before it.  A `return` inside ends the item, not
+    // the workgroup.
+    auto run_item = [&](const int qt, const int h, const int b, const int t0, const int t1, const int gt) {
+    // position and query head of a row
+    auto pos_of = [&](const int row) -> int { return SPLIT ? div_g(p, row) : row; };
+    auto head_of = [&](const int row, const int ps) -> int { return SPLIT ? h * p.G + row - ps * p.G : h; };
     // Opaque per item, so the compiler does not hoist lane-derived values and
     // loads (norm weights, offsets) out of the item loop, where they would
     // stay live through the key loop.
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
-    const int kvh = h / p.G;
     const int g4 = lane >> 4;
     const int q0 = qt * 128;
     const int row_w0 = q0 + 16 * wave;
     const int myrow = row_w0 + (lane & 15);
-    const bool row_ok = myrow < p.S;
-    const int S = p.S, L = p.L, off = p.off;
+    const int R = SPLIT ? p.R : p.S, L = p.L, off = p.off;
+    const bool row_ok = myrow < R;
 
-    const int ntiles = tiles_of(qt);
-    const int lim_wave = min(L, off + min(row_w0 + 16, S));
-    const int lim_row = min(L, off + myrow + 1);
+    const int ntiles = t1 - t0;
+    const int lim_wave = min(L, off + (SPLIT ? pos_of(min(row_w0 + 16, R) - 1) + 1 : min(row_w0 + 16, R)));
+    const int first_lim = off + pos_of(row_w0) + 1;  // causal limit of the wave's first row
+    const int mypos = pos_of(row_ok ? myrow : 0);
+    const int lim_row = min(L, off + (SPLIT ? mypos : myrow) + 1);  // (rows past R: anything)
+    const int64_t q_row = head_of(row_ok ? myrow : 0, mypos) * p.q_hs + static_cast<int64_t>(mypos) * p.q_rs;
 
     // ------------------------------------------------ Q^T operand (registers)
     // B operand of S^T = K Q^T: lane holds query row (lane & 15), dims 32 s + 8 g4 + j.
     op_t qb[KS];
     if constexpr (!FUSED) {
-        const uint16_t* qrow = p.q + b * p.q_bs + h * p.q_hs + static_cast<int64_t>(row_ok ? myrow : 0) * p.q_rs;
+        const uint16_t* qrow = p.q + b * p.q_bs + q_row;
 #pragma unroll
         for (int s = 0; s < KS; ++s)
             qb[s] = to_op<op_t>(row_ok ? ld16(qrow + 32 * s + 8 * g4) : u32x4_v{0u, 0u, 0u, 0u});
@@ -370,8 +486,8 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
         // it is 16.  Every global load is issued before any arithmetic.
         const int hr = p.half_rot;
         const int hs = hr / 32;                  // rotary chunks per half (0 for half_rot 16)
-        const int pos = off + (row_ok ? myrow : 0);
-        const uint16_t* qrow = p.q + h * p.q_hs + static_cast<int64_t>(row_ok ? myrow : 0) * p.q_rs;
+        const int pos = off + mypos;
+        const uint16_t* qrow = p.q + q_row;
         u32x4_v raw[KS], wv[KS], cw[KS / 2], sw[KS / 2];
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -470,10 +586,11 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
             for (int k = 0; k < NIN; ++k) {
                 const int row = row_w0 + k * RPI + rr;
                 qw[k] = cw[k] = sw[k] = u32x4_v{0u, 0u, 0u, 0u};
-                if (row < S) {
-                    qw[k] = ld16(p.q + h * p.q_hs + static_cast<int64_t>(row) * p.q_rs + 8 * c);
+                if (row < R) {
+                    const int ps = pos_of(row);
+                    qw[k] = ld16(p.q + head_of(row, ps) * p.q_hs + static_cast<int64_t>(ps) * p.q_rs + 8 * c);
                     if (rot) {
-                        const int64_t ti = static_cast<int64_t>(off + row) * hr + (8 * c < hr ? 8 * c : 8 * c - hr);
+                        const int64_t ti = static_cast<int64_t>(off + ps) * hr + (8 * c < hr ? 8 * c : 8 * c - hr);
                         cw[k] = ld16(p.cos_t + ti);
                         sw[k] = ld16(p.sin_t + ti);
                     }
@@ -560,7 +677,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     const int vrd0 = T::KBYTES + 16 * (8 * (lane & 15) + (g4 ^ vx));
     const int vrd1 = T::KBYTES + 16 * (8 * (lane & 15) + ((4 + g4) ^ vx));
     for (int it = 0; it < ntiles; ++it) {
-        const int k0 = it * 64;
+        const int k0 = (t0 + it) * 64;
         const int st = (gt + it + 1) & 1;
         __syncthreads();                // the copy waves' tile `it` has landed; stage st^1 is free again
         if (k0 >= lim_wave) continue;   // the whole tile is past this wave's rows
@@ -592,7 +709,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
 
         // Online softmax, base 2, exact running max.  Lane holds row myrow and
         // keys k0 + 16 kb + 4 g4 + i.
-        const bool need_mask = (k0 + 64 > off + row_w0 + 1) || (k0 + 64 > L);
+        const bool need_mask = (k0 + 64 > first_lim) || (k0 + 64 > L);
         if (need_mask) {
             // Only tiles crossing the diagonal or kv_len: a real branch (the
             // empty volatile asm keeps the compiler from if-converting it).
@@ -667,6 +784,23 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     __syncthreads();                    // item end (the copy waves' last barrier)
     // ------------------------------------------------ epilogue
     // O^T C layout: lane holds row myrow, dims 16 d + 4 g4 + i.
+    // the lane index afresh (mbcnt), so that no new value stays live through
+    // the key loop, which runs at the register limit
+    int ln = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    if constexpr (SPLIT) {
+        asm volatile("" : "+v"(ln));  // not computed ahead of the key loop
+        // the piece's sums as they are, for prefill_merge_kernel (with the gate
+        // epilogue here too, for items of one piece, the compiler spilled 54
+        // registers)
+        const int64_t slot = list * W + j;
+        float* po = p.part_o + (slot * kPrefillWaves + wave) * DBK * 256;
+        if (row_w0 < R) {
+#pragma unroll
+            for (int d = 0; d < DBK; ++d) *reinterpret_cast<f32x4_v*>(po + d * 256 + ln * 4) = oacc[d];
+            if (ln < 16) *reinterpret_cast<f32x2_v*>(p.part_ml + (slot * 128 + 16 * wave + ln) * 2) = f32x2_v{m_run, lacc[0]};
+        }
+        return;
+    }
     const float l_tot = lacc[0];
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
     if constexpr (!FUSED) {
@@ -686,14 +820,11 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
         // k RPI + rr, dims 8c .. 8c+7.  16-byte chunks are XOR-swizzled by
         // row, so the 16 rows of a write land in different banks.
         constexpr int LPR = D / 8, RPI = 64 / LPR, NIN = 16 / RPI, CM = LPR - 1;
-        // the lane index afresh (mbcnt), so that no new value stays live
-        // through the key loop, which runs at the register limit
-        const int ln = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
         const int c = ln % LPR, rr = ln / LPR, g4e = ln >> 4;
         u32x4_v gq[NIN];
 #pragma unroll
         for (int k = 0; k < NIN; ++k) {
-            const int row = min(row_w0 + k * RPI + rr, S - 1);
+            const int row = min(row_w0 + k * RPI + rr, R - 1);
             gq[k] = ld16(p.gate + h * p.q_hs + static_cast<int64_t>(row) * p.q_rs + 8 * c);
         }
         uint8_t* const os = lds + ((gt + ntiles) & 1) * T::STAGE + wave * 16 * D * 2;
@@ -725,7 +856,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
                 }
                 o[e] = cvt_pk<bf16_t>(r2[0], r2[1]);
             }
-            if (row < S) st16(p.out_bf16 + static_cast<int64_t>(row) * p.Hq * D + h * D + 8 * c, o);
+            if (row < R) st16(p.out_bf16 + static_cast<int64_t>(row) * p.Hq * D + h * D + 8 * c, o);
         }
     }
     };
@@ -739,13 +870,102 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     if (wave >= kPrefillWaves) {
         copy_items();
     } else {
-        int gt = 0, qt, h, b;
-        for (int r = 0; item_at(r, qt, h, b); ++r) {
-            run_item(qt, h, b, gt);
-            gt += tiles_of(qt);
+        int gt = 0, qt, h, b, t0, t1;
+        for (int r = 0; item_at(r, qt, h, b, t0, t1); ++r) {
+            run_item(qt, h, b, t0, t1, gt);
+            gt += t1 - t0;
         }
     }
 #endif
+}
+
+// Merge of a key split's pieces, and the epilogue: workgroup (item, 16-row
+// block of a compute wave), its four waves a quarter of the dims each, in the
+// layout the pieces left (16-byte accesses, lane-contiguous).  Pieces are
+// added in key order.  Bound by reading the pieces' sums (128 KB a piece at
+// D 256, at most one piece a CU).
+template <int D, bool FUSED>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
+    constexpr int DBK = D / 16, DW = DBK / 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int list = blockIdx.x & ((1 << p.lists_log2) - 1), wb = blockIdx.y;
+    const int nb = p.nb, W = p.W;
+    int qi, idx;
+    split_item(p, blockIdx.x >> p.lists_log2, qi, idx);
+    const int qt = p.nqt - 1 - qi;
+    const int np = prefill_pieces(prefill_tiles<true>(p, qt), p.piece);
+    const int row0 = qt * 128 + 16 * wb;
+    if (row0 >= p.R) return;
+    const int64_t slot0 = list * W + prefill_slots_before(p, qi, nb) + idx;
+    const float* ml = p.part_ml + (slot0 * 128 + 16 * wb + (lane & 15)) * 2;
+    const float* po = p.part_o + ((slot0 * kPrefillWaves + wb) * DBK + wave * DW) * 256 + lane * 4;
+    const int64_t step = static_cast<int64_t>(nb) * kPrefillWaves * DBK * 256;
+    f32x4_v acc[DW];
+#pragma unroll
+    for (int d = 0; d < DW; ++d) acc[d] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+    float l_tot = 0.f, mx = -1e30f;
+    // Four pieces at a time, every load issued ahead of the arithmetic (past
+    // the last piece the last one again, with no weight).
+    constexpr int NP = 4;
+    for (int i0 = 0; i0 < np; i0 += NP) {
+        f32x2_v v[NP];
+        f32x4_v o[NP][DW];
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+            const int64_t i = min(i0 + u, np - 1);
+            v[u] = *reinterpret_cast<const f32x2_v*>(ml + i * nb * 256);
+#pragma unroll
+            for (int d = 0; d < DW; ++d) o[u][d] = *reinterpret_cast<const f32x4_v*>(po + i * step + d * 256);
+        }
+        float m_new = mx;
+#pragma unroll
+        for (int u = 0; u < NP; ++u) m_new = fmaxf(m_new, v[u][0]);
+        const float a = __builtin_amdgcn_exp2f(mx - m_new);
+        mx = m_new;
+        l_tot *= a;
+#pragma unroll
+        for (int d = 0; d < DW; ++d)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[d][e] *= a;
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+            if (i0 + u >= np) break;
+            const float w = __builtin_amdgcn_exp2f(v[u][0] - m_new);
+            l_tot += v[u][1] * w;
+#pragma unroll
+            for (int d = 0; d < DW; ++d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[d][e] += o[u][d][e] * w;
+        }
+    }
+    const int row = row0 + (lane & 15), g4 = lane >> 4;
+    if (row >= p.R) return;
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    const int b = p.B > 1 ? idx / p.hpl : 0, kvh = list * p.hpl + idx - b * p.hpl;
+    const int ps = div_g(p, row), h = kvh * p.G + row - ps * p.G;
+#pragma unroll
+    for (int d = 0; d < DW; ++d) {
+        const int dim = 16 * (wave * DW + d) + 4 * g4;
+        if constexpr (!FUSED) {
+            *reinterpret_cast<f32x4_v*>(p.out_f32 + b * p.o_bs + h * p.o_hs + static_cast<int64_t>(ps) * p.o_rs + dim) =
+                f32x4_v{acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv};
+        } else {
+            const u32x2_v gw = *reinterpret_cast<const u32x2_v*>(p.gate + h * p.q_hs + static_cast<int64_t>(ps) * p.q_rs + dim);
+            u32x2_v o;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                float r2[2];
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const float a = bf16_round(acc[d][2 * e + hh] * inv);
+                    const float g = bf16_bits_to_f32(hh ? gw[e] >> 16 : gw[e] & 0xFFFFu);
+                    r2[hh] = a * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * kLog2e));
+                }
+                o[e] = cvt_pk<bf16_t>(r2[0], r2[1]);
+            }
+            *reinterpret_cast<u32x2_v*>(p.out_bf16 + (static_cast<int64_t>(ps) * p.Hq + h) * D + dim) = o;
+        }
+    }
 }
 
 // ----------------------------------------------------------------------------
@@ -989,12 +1209,14 @@ __global__ __launch_bounds__(64 * kKvStageWaves) void kv_stage_kernel(KvStagePar
 
 // Stages V^T for `B` sequences of `L` keys into the prefill workspace slot of
 // `device` and points `p` at it.  Returns hipSuccess or the failing error.
+// `part_bytes` more are kept for a key split, at *part.
 static hipError_t stage_vt(int device, hipStream_t st, const KvView& kv, int B, int Hkv, int L, int D,
-                           PrefillParams& p) {
+                           PrefillParams& p, size_t part_bytes, void** part) {
     const int ld = (L + 63) / 64 * 64;
-    const size_t bytes = static_cast<size_t>(B) * Hkv * D * ld * 2;
-    void* ws = device_workspace(device, bytes, kWorkspacePrefill);
+    const size_t bytes = (static_cast<size_t>(B) * Hkv * D * ld * 2 + 255) & ~static_cast<size_t>(255);
+    void* ws = device_workspace(device, bytes + part_bytes, kWorkspacePrefill);
     if (!ws) return hipErrorOutOfMemory;
+    *part = part_bytes ? static_cast<uint8_t*>(ws) + bytes : nullptr;
     p.vt = static_cast<const uint16_t*>(ws);
     p.vt_ld = ld;
     const dim3 grid(ld / 64, Hkv, B);
@@ -1011,24 +1233,99 @@ static hipError_t stage_vt(int device, hipStream_t st, const KvView& kv, int B, 
 // ----------------------------------------------------------------------------
 // Host side
 // ----------------------------------------------------------------------------
+// Key split: when a query head's 128-row items leave CUs without work, or with
+// one short item each, the items run as pieces over the kv heads' rows.
+constexpr int kSplitMinTiles = 4;  // key tiles a piece has at least
+static size_t prefill_part_bytes(int D, int n_wg) { return static_cast<size_t>(n_wg) * 128 * (D + 2) * sizeof(float); }
+// Chunks whose workspace holds room for a key split: at most 8192 tokens of the
+// kv heads (at 4 query heads a kv head one 128-row item a CU), and keys for
+// pieces that win more than their merge costs.
+static bool prefill_may_split(size_t S, size_t L, size_t Hkv) {
+    return S * Hkv <= 8192 && L > 2 * 64 * kSplitMinTiles;
+}
+
+// Fills in p's split (piece 0: none) for n workgroups.  The estimates are in
+// microseconds (one MI355X, D 256): a tile takes 1.25 with up to half the CUs
+// busy, and with all of them 1.4 in items of falling length but 2.0 in equal
+// pieces; a split costs 11 more (its sums to memory, and the merge).  Measured,
+// whole call, 16/4 heads: 64 rows after 8000 cached tokens 157 -> 45 us, 333
+// rows 168 -> 70, 300 after 1000 39 -> 32, 1000 after 16000 348 -> 272; left
+// whole: 1000 rows of a prompt 35.5 (split 37.6), 1500 after 1000 68.8 (75.6).
+static void plan_key_split(PrefillParams& p, int n) {
+    p.piece = 0;
+    const int lists = n % 8 ? 1 : (p.Hkv % 8 == 0 ? 8 : (8 % p.Hkv == 0 ? p.Hkv : 1));
+    p.lists_log2 = lists == 8 ? 3 : (lists == 4 ? 2 : (lists == 2 ? 1 : 0));
+    p.W = n / lists;
+    p.hpl = p.Hkv / lists;
+    p.nb = p.hpl * p.B;
+    p.g_shift = 0;
+    while ((1 << p.g_shift) < p.G) ++p.g_shift;
+    p.g_mul = static_cast<uint32_t>(((1ull << (31 + p.g_shift)) + p.G - 1) / p.G);
+    if (static_cast<int64_t>(p.S) * p.G > 0x3fffffff) return;
+    p.R = p.S * p.G;
+    const int nqt = (p.R + 127) / 128;
+    if (static_cast<int64_t>(nqt) * p.nb > p.W) return;
+    auto tiles = [&](int qt) {
+        const int64_t lim = std::min<int64_t>(p.L, static_cast<int64_t>(p.off) + (std::min(qt * 128 + 128, p.R) - 1) / p.G + 1);
+        return static_cast<int>((lim + 63) / 64);
+    };
+    auto pieces = [&](int c) {
+        int64_t t = 0;
+        for (int qt = 0; qt < nqt; ++qt) t += prefill_pieces(tiles(qt), c);
+        return t * p.nb;
+    };
+    const int longest = tiles(nqt - 1);
+    int lo = kSplitMinTiles, hi = longest;  // the least piece whose pieces fit one round
+    while (lo < hi) {
+        const int c = (lo + hi) / 2;
+        if (pieces(c) <= p.W) hi = c;
+        else lo = c + 1;
+    }
+    const double busy = std::min(1.0, static_cast<double>(p.nqt) * p.Hq * p.B / n);
+    const double busy_s = static_cast<double>(pieces(lo)) / p.W;
+    const double whole = longest * (1.25 + 0.3 * std::max(0.0, busy - 0.5));
+    const double split = lo * (1.25 + 1.5 * std::max(0.0, busy_s - 0.5)) + 11.0;
+    if (split + 2.0 < whole) {
+        p.piece = lo;
+        p.nqt = nqt;
+        p.n_wg = n;
+    }
+}
+
+template <typename QT, int D, bool FUSED>
+static hipError_t launch_prefill_d(hipStream_t st, const PrefillParams& p) {
+    const dim3 grid(static_cast<unsigned>(p.n_wg)), blk(kPrefillThreads);
+    if (!p.piece) {
+        hipLaunchKernelGGL((prefill_kernel<QT, D, FUSED, false>), grid, blk, 0, st, p);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((prefill_kernel<QT, D, FUSED, true>), grid, blk, 0, st, p);
+    const dim3 mgrid(static_cast<unsigned>(p.nqt * p.Hkv * p.B), kPrefillWaves);
+    hipLaunchKernelGGL((prefill_merge_kernel<D, FUSED>), mgrid, dim3(256), 0, st, p);
+    return hipGetLastError();
+}
+
 // Persistent grid: one workgroup per CU (a workgroup's LDS allows no second
 // one), a multiple of 8 so the XCD-aware item lists stay aligned, and never
-// more workgroups than items.
+// more workgroups than items.  part: room of part_bytes for a key split's sums,
+// or NULL for none.
 template <typename QT, bool FUSED>
-static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillParams& p) {
+static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillParams& p, void* part, size_t part_bytes) {
     const int items = p.nqt * p.Hq * p.B;
     int n = device_cu_count(device);
     if (n <= 0) n = 256;
     n = n >= 8 ? n & ~7 : n;
     p.n_wg = items < n ? items : n;
-    const dim3 grid(static_cast<unsigned>(p.n_wg));
+    p.piece = 0;
+    if (part && !p.claims && part_bytes >= prefill_part_bytes(D, n)) plan_key_split(p, n);
+    p.part_ml = static_cast<float*>(part);
+    p.part_o = p.part_ml + (part ? static_cast<size_t>(n) * 256 : 0);
     switch (D) {
-    case 64: hipLaunchKernelGGL((prefill_kernel<QT, 64, FUSED>), grid, dim3(kPrefillThreads), 0, st, p); break;
-    case 128: hipLaunchKernelGGL((prefill_kernel<QT, 128, FUSED>), grid, dim3(kPrefillThreads), 0, st, p); break;
-    case 256: hipLaunchKernelGGL((prefill_kernel<QT, 256, FUSED>), grid, dim3(kPrefillThreads), 0, st, p); break;
+    case 64: return launch_prefill_d<QT, 64, FUSED>(st, p);
+    case 128: return launch_prefill_d<QT, 128, FUSED>(st, p);
+    case 256: return launch_prefill_d<QT, 256, FUSED>(st, p);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 static float rescale_slack() {
@@ -1115,12 +1412,15 @@ int prefill_dropin(int dtype, size_t device, size_t B, size_t Hq, size_t Hkv, si
     p.o_hs = p.q_hs;
     p.o_bs = p.q_bs;
     p.B = static_cast<int>(B);
-    if (kv_len > 0 && stage_vt(static_cast<int>(device), nullptr, p.kv, static_cast<int>(B), static_cast<int>(Hkv),
-                               static_cast<int>(kv_len), static_cast<int>(D), p) != hipSuccess)
-        return 11;
     const int dev = static_cast<int>(device);
-    const hipError_t e = dtype == 0 ? launch_prefill<f16_t, false>(dev, static_cast<int>(D), nullptr, p)
-                                    : launch_prefill<bf16_t, false>(dev, static_cast<int>(D), nullptr, p);
+    void* part = nullptr;
+    const size_t part_bytes = prefill_may_split(q_len * B, kv_len, Hkv)
+                                  ? prefill_part_bytes(static_cast<int>(D), std::max(device_cu_count(dev), 256)) : 0;
+    if (kv_len > 0 && stage_vt(dev, nullptr, p.kv, static_cast<int>(B), static_cast<int>(Hkv), static_cast<int>(kv_len),
+                               static_cast<int>(D), p, part_bytes, &part) != hipSuccess)
+        return 11;
+    const hipError_t e = dtype == 0 ? launch_prefill<f16_t, false>(dev, static_cast<int>(D), nullptr, p, part, part_bytes)
+                                    : launch_prefill<bf16_t, false>(dev, static_cast<int>(D), nullptr, p, part, part_bytes);
     if (e != hipSuccess) return 11;
     if (hipDeviceSynchronize() != hipSuccess) return 12;
     return 0;
@@ -1152,7 +1452,9 @@ extern "C" size_t supersonic_attn_gfx950_prefill_workspace_size(int kv_dtype, si
     if (L > 0x7FFFFFFF || kv_heads > 4096 || head_dim > 512) return 0;
     const size_t ld = (L + 63) / 64 * 64;
     const size_t stage = kv_heads * head_dim * ld * 2;  // V^T staging
-    return kv_dtype == SUPERSONIC_KV_FP8_E4M3 ? 2 * stage : stage;  // + the bf16 K rows of an fp8 cache
+    const size_t stages = kv_dtype == SUPERSONIC_KV_FP8_E4M3 ? 2 * stage : stage;  // + the bf16 K rows of an fp8 cache
+    // + a key split's sums
+    return stages + (prefill_may_split(chunk_len, L, kv_heads) ? prefill_part_bytes(static_cast<int>(head_dim), 256) : 0);
 }
 
 namespace ssa {
@@ -1205,6 +1507,8 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
     p.eps = eps;
     p.B = 1;
     p.claims = claims;
+    void* part = nullptr;  // room for a key split's sums
+    size_t part_bytes = 0;
     // K norm + RoPE + cache append for the chunk and the V^T staging of every
     // position, in one pass
     {
@@ -1212,13 +1516,18 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
         // V^T staging, then (fp8 cache) the bf16 K rows the attention reads
         const size_t stage_bytes = static_cast<size_t>(p.Hkv) * head_dim * ld * 2;
         const size_t need = fp8 ? 2 * stage_bytes : stage_bytes;
+        // (stage_bytes is a multiple of 128)
+        if (prefill_may_split(chunk_len, p.L, kv_heads))
+            part_bytes = prefill_part_bytes(static_cast<int>(head_dim), std::max(device_cu_count(static_cast<int>(device_ordinal)), 256));
         void* ws = workspace;
         if (ws) {
             if (workspace_bytes < need) return SUPERSONIC_ERR_WORKSPACE;
+            part_bytes = std::min(part_bytes, workspace_bytes - need);
         } else {
-            ws = device_workspace(static_cast<int>(device_ordinal), need, kWorkspacePrefill);
+            ws = device_workspace(static_cast<int>(device_ordinal), need + part_bytes, kWorkspacePrefill);
         }
         if (!ws) return SUPERSONIC_ERR_WORKSPACE;
+        if (part_bytes) part = static_cast<uint8_t*>(ws) + need;
         p.vt = static_cast<const uint16_t*>(ws);
         p.vt_ld = ld;
         uint16_t* kst = fp8 ? reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(ws) + stage_bytes) : nullptr;
@@ -1261,7 +1570,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
     }
     const ProfileEvents prof = take_profile_events();
     if (prof.before) (void)hipEventRecord(prof.before, st);
-    if (launch_prefill<bf16_t, true>(static_cast<int>(device_ordinal), static_cast<int>(head_dim), st, p) != hipSuccess)
+    if (launch_prefill<bf16_t, true>(static_cast<int>(device_ordinal), static_cast<int>(head_dim), st, p, part, part_bytes) != hipSuccess)
         return SUPERSONIC_ERR_LAUNCH;
     if (prof.after) (void)hipEventRecord(prof.after, st);
     return 0;

@@ -143,6 +143,55 @@ def test_fused_prefill_matches_oracle(S, Hq, Hkv, D, rot, start):
     assert torch.equal(cache.v[0, :, start:start + S].float().cpu(), vch)
 
 
+# Chunks whose items run as pieces of their keys: single rows, rows that end inside
+# a tile and a 16-row block, query heads a kv head of 1, 2, 5 and 8, kv heads that
+# do not spread over the XCDs (3, 5), every head size, each rotary prologue.
+@pytest.mark.parametrize("S,Hq,Hkv,D,rot,start", [
+    (1, 16, 4, 256, 64, 3000), (16, 16, 2, 256, 64, 1000), (33, 8, 2, 256, 96, 2100), (129, 16, 4, 256, 64, 1531),
+    (300, 6, 3, 128, 32, 1000), (77, 5, 1, 256, 64, 4097), (64, 5, 5, 64, 32, 1600), (40, 24, 8, 256, 64, 1300),
+    (1000, 8, 2, 256, 64, 0), (200, 16, 16, 128, 128, 2500),
+])
+def test_fused_prefill_key_split(S, Hq, Hkv, D, rot, start):
+    announce(f"prefill key split S={S} Hq={Hq} Hkv={Hkv} D={D} rot={rot} start={start}")
+    c = fused_case(73, S, Hq, Hkv, D, rot, start)
+    kc = torch.zeros(1, Hkv, start + S, D, dtype=torch.bfloat16)
+    vc = torch.zeros_like(kc)
+    kc[0, :, :start], vc[0, :, :start] = c["prefix_k"], c["prefix_v"]
+    size = K.prefill_workspace_size(False, Hkv, D, S, start)
+    plain = Hkv * D * ((start + S + 63) // 64 * 64) * 2  # V^T staging alone: no room for the pieces' sums
+    assert size > plain
+    outs = []
+    for n in (None, size, plain):
+        cache = K.KvCache(kc.to(DEV), vc.to(DEV))
+        out = torch.full((S, Hq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ws = None if n is None else torch.full((n,), 255, dtype=torch.uint8, device=DEV)  # holds NaNs
+        K.fused_prefill(0, *(c[k].to(DEV) for k in ("q_proj", "k_new", "v_new", "qw", "kw", "cos", "sin")), cache, out,
+                        q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot, chunk_start=start, workspace=ws)
+        torch.cuda.synchronize()
+        outs.append(out)
+    ref, kch, _ = O.prefill_layer(c["shape"], c["q_proj"], c["k_new"], c["v_new"], c["qw"], c["kw"], c["cos"], c["sin"],
+                                  start, c["prefix_k"], c["prefix_v"])
+    for out in outs:
+        check(out, ref, TOL_BF16, "prefill key split")
+    assert torch.equal(outs[0], outs[1])
+    # the 16-bit weights round against another running max, the result to bf16: within TOL_BF16 of the whole items' too
+    check(outs[0], outs[2].float().cpu(), TOL_BF16, "split against whole")
+
+
+@pytest.mark.parametrize("dtype", [K.ScalarType.BF16, K.ScalarType.F16])
+@pytest.mark.parametrize("B,Hq,Hkv,S,L,off,D", [(2, 8, 2, 65, 2065, 2000, 128), (1, 4, 4, 130, 1500, 2000, 256),
+                                                (3, 6, 3, 20, 3020, 3000, 64), (1, 8, 1, 100, 900, 850, 256)])
+def test_prefill_dropin_key_split(dtype, B, Hq, Hkv, S, L, off, D):
+    """Batches, and keys that end before or after the causal limit."""
+    announce(f"dropin key split dtype={dtype} B={B} Hq={Hq} Hkv={Hkv} S={S} L={L} off={off} D={D}")
+    tdt = torch.bfloat16 if dtype == K.ScalarType.BF16 else torch.float16
+    g = gen(62)
+    q = torch.randn(B, Hq, S, D, generator=g).to(tdt)
+    k, v = (torch.randn(B, Hkv, L, D, generator=g).to(tdt) for _ in "kv")
+    out = dropin(q, k, v, off, dtype)
+    check(out, O.attention_prefill(q.float(), k.float(), v.float(), D ** -0.5, off), TOL_BF16, "dropin key split")
+
+
 def test_fused_prefill_paged():
     announce("fused prefill paged")
     S, Hq, Hkv, D, rot, ps = 400, 16, 2, 256, 64, 64
