@@ -50,21 +50,6 @@ struct PrefillParams {
     int nqt;             // query tiles of 128 rows (of a query head; with a key split of a kv head)
     int B;               // sequences
     int n_wg;            // workgroups of the persistent grid
-    // Key split (piece 0: none).  A kv head's rows are its G query heads at S
-    // positions, R = S * G rows in all, row r = position r / G of query head
-    // kvh * G + r % G; an item's key tiles run as pieces of at most `piece`
-    // tiles, one piece a workgroup, which leave their sums here for
-    // prefill_merge_kernel, by workgroup slot: the unnormalised O in accumulator
-    // order ([slot][wave][16-dim block][lane] x 4 floats) and each row's (max, sum).
-    int piece;
-    int R;
-    int lists_log2;      // 1 << lists_log2 item lists (kv heads spread over the XCDs)
-    int W;               // workgroups of a list
-    int hpl, nb;         // kv heads of a list; items of a query tile in it, hpl * B
-    uint32_t g_mul;      // r / G = (2 r * g_mul >> 32) >> g_shift for r < 2^31:
-    int g_shift;         // g_mul = ceil(2^(31 + g_shift) / G), g_shift = ceil(log2 G)
-    float* part_o;
-    float* part_ml;
     // Dynamic schedule (NULL: the static one).  Per item list x (an XCD's, or
     // the single list) a claim counter at claims[32 x] and a finished-workgroup
     // counter at claims[32 (8 + x)], each on its own 128-byte line; both are
@@ -83,6 +68,28 @@ struct PrefillParams {
     float eps;
     float rescale_slack;  // lazy-rescale slack in log2 units (0 = exact running max)
 };
+
+// The same with a key split (a type of its own: the other kernels' arguments
+// stay small; with these 64 bytes more every launch took 0.3 us longer).
+struct PrefillSplitParams : PrefillParams {
+    // A kv head's rows are its G query heads at S
+    // positions, R = S * G rows in all, row r = position r / G of query head
+    // kvh * G + r % G; an item's key tiles run as pieces of at most `piece`
+    // tiles, one piece a workgroup, which leave their sums here for
+    // prefill_merge_kernel, by workgroup slot: the unnormalised O in accumulator
+    // order ([slot][wave][16-dim block][lane] x 4 floats) and each row's (max, sum).
+    int piece;
+    int R;
+    int lists_log2;      // 1 << lists_log2 item lists (kv heads spread over the XCDs)
+    int W;               // workgroups of a list
+    int hpl, nb;         // kv heads of a list; items of a query tile in it, hpl * B
+    uint32_t g_mul;      // r / G = (2 r * g_mul >> 32) >> g_shift for r < 2^31:
+    int g_shift;         // g_mul = ceil(2^(31 + g_shift) / G), g_shift = ceil(log2 G)
+    float* part_o;
+    float* part_ml;
+};
+template <bool SPLIT> struct PrefillArgs { typedef PrefillParams t; };
+template <> struct PrefillArgs<true> { typedef PrefillSplitParams t; };
 
 template <typename QT> struct Mfma32;
 template <> struct Mfma32<bf16_t> {
@@ -206,12 +213,12 @@ constexpr int kPrefillThreads = 64 * (kPrefillWaves + kCopyWaves);
 // r / G by a multiplication: a division by a run-time value takes about 40
 // dependent instructions, and several of them ahead of an item's first copy
 // cost 2 us.
-__device__ __forceinline__ int div_g(const PrefillParams& p, int r) {
+__device__ __forceinline__ int div_g(const PrefillSplitParams& p, int r) {
     return static_cast<int>(__umulhi(2u * static_cast<uint32_t>(r), p.g_mul) >> p.g_shift);
 }
 // Item m of a list: its order index (query tiles from the last one on) and its
 // number within the query tile.
-__device__ __forceinline__ void split_item(const PrefillParams& p, int m, int& qi, int& idx) {
+__device__ __forceinline__ void split_item(const PrefillSplitParams& p, int m, int& qi, int& idx) {
     qi = m;
     idx = 0;
     if (p.nb > 1) {
@@ -220,32 +227,34 @@ __device__ __forceinline__ void split_item(const PrefillParams& p, int m, int& q
     }
 }
 // 64-key tiles below the last row's causal limit of query tile qt.
-template <bool SPLIT>
 __device__ __forceinline__ int prefill_tiles(const PrefillParams& p, int qt) {
-    const int lim = min(p.L, p.off + (SPLIT ? div_g(p, min(qt * 128 + 128, p.R) - 1) + 1 : min(qt * 128 + 128, p.S)));
+    const int lim = min(p.L, p.off + min(qt * 128 + 128, p.S));
     return lim > 0 ? (lim + 63) / 64 : 0;
+}
+__device__ __forceinline__ int prefill_tiles(const PrefillSplitParams& p, int qt) {
+    return (min(p.L, p.off + div_g(p, min(qt * 128 + 128, p.R) - 1) + 1) + 63) / 64;
 }
 // Pieces that n key tiles run as.
 __host__ __device__ __forceinline__ int prefill_pieces(int n, int piece) { return n > piece ? (n + piece - 1) / piece : 1; }
 
 // Slots of one list before its order index qi (query tiles from the last one
 // on), `nb` items a query tile; for the whole wave.
-__device__ __forceinline__ int prefill_slots_before(const PrefillParams& p, int qi, int nb) {
+__device__ __forceinline__ int prefill_slots_before(const PrefillSplitParams& p, int qi, int nb) {
     const int lane = threadIdx.x & 63;
     int n = 0;
-    for (int i = lane; i < qi; i += 64) n += prefill_pieces(prefill_tiles<true>(p, p.nqt - 1 - i), p.piece);
+    for (int i = lane; i < qi; i += 64) n += prefill_pieces(prefill_tiles(p, p.nqt - 1 - i), p.piece);
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o);
     return __builtin_amdgcn_readfirstlane(n) * nb;
 }
 // The piece in slot j of a list: order index of its query tile, its number
 // within the query tile's pieces; false past the last.
-__device__ __forceinline__ bool prefill_find_piece(const PrefillParams& p, int j, int nb, int& qi, int& at) {
+__device__ __forceinline__ bool prefill_find_piece(const PrefillSplitParams& p, int j, int nb, int& qi, int& at) {
     const int lane = threadIdx.x & 63;
     int before = 0;
     for (int base = 0; base < p.nqt; base += 64) {
         const int i = base + lane;
-        const int np = i < p.nqt ? prefill_pieces(prefill_tiles<true>(p, p.nqt - 1 - i), p.piece) * nb : 0;
+        const int np = i < p.nqt ? prefill_pieces(prefill_tiles(p, p.nqt - 1 - i), p.piece) * nb : 0;
         int incl = np;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -266,7 +275,7 @@ __device__ __forceinline__ bool prefill_find_piece(const PrefillParams& p, int j
 
 // SPLIT: one piece of an item a workgroup (PrefillParams::piece).
 template <typename QT, int D, bool FUSED, bool SPLIT>
-__global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams p) {
+__global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(typename PrefillArgs<SPLIT>::t p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
     typedef typename Mfma16<QT>::op op_t;
     typedef Tile<D> T;
@@ -287,12 +296,20 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     const int bid = blockIdx.x;
     const int hpx = p.Hq / 8;
     const bool by_xcd = !SPLIT && hpx > 0 && (p.Hq % 8) == 0 && (p.n_wg % 8) == 0;
-    const int ll = p.lists_log2;
-    const int list = SPLIT ? bid & ((1 << ll) - 1) : (by_xcd ? bid & 7 : 0);
-    const int j = SPLIT ? (ll ? ((bid >> 3) << (3 - ll)) + ((bid & 7) >> ll) : bid) : (by_xcd ? (bid >> 3) : bid);
-    const int W = SPLIT ? p.W : (by_xcd ? (p.n_wg >> 3) : p.n_wg);
+    int list, j, W;
+    if constexpr (SPLIT) {
+        const int ll = p.lists_log2;
+        list = bid & ((1 << ll) - 1);
+        j = ll ? ((bid >> 3) << (3 - ll)) + ((bid & 7) >> ll) : bid;
+        W = p.W;
+    } else {
+        list = by_xcd ? (bid & 7) : 0;
+        j = by_xcd ? (bid >> 3) : bid;
+        W = by_xcd ? (p.n_wg >> 3) : p.n_wg;
+    }
     const int hpi = by_xcd ? hpx : p.Hq;     // heads per item list
-    const int n_items = p.nqt * (SPLIT ? p.nb : hpi * p.B);
+    int n_items = p.nqt * hpi * p.B;
+    if constexpr (SPLIT) n_items = p.nqt * p.nb;
     // Key split: this workgroup's one piece, tiles [pt0, pt1) of item pm.
     int pm = 0, pt0 = 0, pt1 = 0;
     // one item, in a loop that the compiler takes for a loop: straight-line, it
@@ -302,7 +319,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     if constexpr (SPLIT) {
         int qi, at;
         if (!prefill_find_piece(p, j, p.nb, qi, at)) return;  // the whole workgroup
-        const int n = prefill_tiles<true>(p, p.nqt - 1 - qi);
+        const int n = prefill_tiles(p, p.nqt - 1 - qi);
         const int pn = prefill_pieces(n, p.piece);
         int part, idx;
         split_item(p, at, part, idx);
@@ -346,7 +363,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
             h = (by_xcd ? (bid & 7) * hpx : 0) + rem % hpi;
             b = rem / hpi;
             t0 = 0;
-            t1 = prefill_tiles<false>(p, qt);
+            t1 = prefill_tiles(p, qt);
         }
         return true;
     };
@@ -446,7 +463,10 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     // the workgroup.
     auto run_item = [&](const int qt, const int h, const int b, const int t0, const int t1, const int gt) {
     // position and query head of a row
-    auto pos_of = [&](const int row) -> int { return SPLIT ? div_g(p, row) : row; };
+    auto pos_of = [&](const int row) -> int {
+        if constexpr (SPLIT) return div_g(p, row);
+        else return row;
+    };
     auto head_of = [&](const int row, const int ps) -> int { return SPLIT ? h * p.G + row - ps * p.G : h; };
     // Opaque per item, so the compiler does not hoist lane-derived values and
     // loads (norm weights, offsets) out of the item loop, where they would
@@ -457,7 +477,9 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
     const int q0 = qt * 128;
     const int row_w0 = q0 + 16 * wave;
     const int myrow = row_w0 + (lane & 15);
-    const int R = SPLIT ? p.R : p.S, L = p.L, off = p.off;
+    int R = p.S;
+    if constexpr (SPLIT) R = p.R;
+    const int L = p.L, off = p.off;
     const bool row_ok = myrow < R;
 
     const int ntiles = t1 - t0;
@@ -885,7 +907,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(PrefillParams 
 // added in key order.  Bound by reading the pieces' sums (128 KB a piece at
 // D 256, at most one piece a CU).
 template <int D, bool FUSED>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillSplitParams p) {
     constexpr int DBK = D / 16, DW = DBK / 4;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int list = blockIdx.x & ((1 << p.lists_log2) - 1), wb = blockIdx.y;
@@ -893,7 +915,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     int qi, idx;
     split_item(p, blockIdx.x >> p.lists_log2, qi, idx);
     const int qt = p.nqt - 1 - qi;
-    const int np = prefill_pieces(prefill_tiles<true>(p, qt), p.piece);
+    const int np = prefill_pieces(prefill_tiles(p, qt), p.piece);
     const int row0 = qt * 128 + 16 * wb;
     if (row0 >= p.R) return;
     const int64_t slot0 = list * W + prefill_slots_before(p, qi, nb) + idx;
@@ -1251,7 +1273,7 @@ static bool prefill_may_split(size_t S, size_t L, size_t Hkv) {
 // whole call, 16/4 heads: 64 rows after 8000 cached tokens 157 -> 45 us, 333
 // rows 168 -> 70, 300 after 1000 39 -> 32, 1000 after 16000 348 -> 272; left
 // whole: 1000 rows of a prompt 35.5 (split 37.6), 1500 after 1000 68.8 (75.6).
-static void plan_key_split(PrefillParams& p, int n) {
+static void plan_key_split(PrefillSplitParams& p, int n) {
     p.piece = 0;
     const int lists = n % 8 ? 1 : (p.Hkv % 8 == 0 ? 8 : (8 % p.Hkv == 0 ? p.Hkv : 1));
     p.lists_log2 = lists == 8 ? 3 : (lists == 4 ? 2 : (lists == 2 ? 1 : 0));
@@ -1293,10 +1315,10 @@ static void plan_key_split(PrefillParams& p, int n) {
 }
 
 template <typename QT, int D, bool FUSED>
-static hipError_t launch_prefill_d(hipStream_t st, const PrefillParams& p) {
+static hipError_t launch_prefill_d(hipStream_t st, const PrefillSplitParams& p) {
     const dim3 grid(static_cast<unsigned>(p.n_wg)), blk(kPrefillThreads);
     if (!p.piece) {
-        hipLaunchKernelGGL((prefill_kernel<QT, D, FUSED, false>), grid, blk, 0, st, p);
+        hipLaunchKernelGGL((prefill_kernel<QT, D, FUSED, false>), grid, blk, 0, st, static_cast<const PrefillParams&>(p));
         return hipGetLastError();
     }
     hipLaunchKernelGGL((prefill_kernel<QT, D, FUSED, true>), grid, blk, 0, st, p);
@@ -1310,7 +1332,7 @@ static hipError_t launch_prefill_d(hipStream_t st, const PrefillParams& p) {
 // more workgroups than items.  part: room of part_bytes for a key split's sums,
 // or NULL for none.
 template <typename QT, bool FUSED>
-static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillParams& p, void* part, size_t part_bytes) {
+static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillSplitParams& p, void* part, size_t part_bytes) {
     const int items = p.nqt * p.Hq * p.B;
     int n = device_cu_count(device);
     if (n <= 0) n = 256;
@@ -1388,7 +1410,7 @@ int prefill_dropin(int dtype, size_t device, size_t B, size_t Hq, size_t Hkv, si
         if (hipDeviceSynchronize() != hipSuccess) return 12;
         return 0;
     }
-    PrefillParams p{};
+    PrefillSplitParams p{};
     p.q = static_cast<const uint16_t*>(q);
     p.q_rs = static_cast<int64_t>(D);
     p.q_hs = static_cast<int64_t>(q_len) * D;
@@ -1483,7 +1505,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
     hipStream_t st = static_cast<hipStream_t>(stream);
 
 
-    PrefillParams p{};
+    PrefillSplitParams p{};
     p.q = static_cast<const uint16_t*>(q_proj);
     p.q_bs = 0;
     p.q_hs = 2 * static_cast<int64_t>(head_dim);
