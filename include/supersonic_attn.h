@@ -344,9 +344,9 @@ int supersonic_attn_gfx950_mixed(
  * the megakernel's input norm and projections (full_attention_4b.hip:4942-4967,
  * :5019-5101) and rms_norm_rows_model + matmul_proj of prefill_engine.rs:1951-2117.
  * A norm kernel writes the normed rows once (workspace), then rows <= 12
- * (SUPERSONIC_PROJ_SKINNY_MAX_M) with q/kv_out_dim % 16 == 0 take one
- * weight-streaming launch over the three matrices; otherwise one launch of the
- * hand-written MFMA GEMM over the three matrices as column segments
+ * (SUPERSONIC_PROJ_SKINNY_MAX_M) with q/kv_out_dim % 16 == 0 and at most one
+ * 16-column block a CU take one weight-streaming launch over the three
+ * matrices; otherwise one launch of the hand-written MFMA GEMM over the three matrices as column segments
  * (SUPERSONIC_PROJ_GEMM=hipblaslt: one hipBLASLt GEMM per matrix instead).
  * hidden_dim % 8 == 0.  Asynchronous on `stream`.  workspace: caller device
  * memory of at least supersonic_attn_gfx950_qkv_proj_workspace_size() bytes,

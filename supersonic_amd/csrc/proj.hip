@@ -34,6 +34,7 @@
 #include <dlfcn.h>
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -374,6 +375,23 @@ int skinny_max_m() {
     return x < 0 ? 0 : (x > kSkinnyMaxM ? kSkinnyMaxM : x);
 }
 
+// Whether the streaming kernels' few rows go to them rather than to the tiled
+// GEMM: with at most one 16-column block a CU.  More blocks come in uneven
+// rounds, and short rows of W leave a wave too few loads in flight (one
+// MI355X, 8 rows: o_proj 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled;
+// norm + Q/K/V 1024 -> 5120, 320 blocks, 13.0 against 11.4; 2048 -> 9216, 576
+// blocks, 20.0 against 12.5; 4096 -> 10240, 640 blocks, 23.2 against 21.9).
+// A row limit or a GEMM in the environment asks for the streaming kernels.
+bool stream_columns(int dev, int64_t ncb) {
+    const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
+    return ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM");
+}
+// ... and with the QK norm and RoPE in the epilogue, which the tiled GEMM leaves
+// to a kernel of their own: also with long rows (8 rows, 4096 -> 10240: 27.6 us
+// against 27.7 tiled, 1 row 25.9 against 27.9; 2048 -> 9216: 22.6 against 17.0;
+// 1024 -> 5120: 16.5 against 14.8).
+bool stream_rope_columns(int dev, int64_t ncb, int k) { return k >= 4096 || stream_columns(dev, ncb); }
+
 bool skinny_fits(int m, int k, const void* x, const void* w) {
     return m >= 1 && m <= skinny_max_m() && k % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
            (reinterpret_cast<uintptr_t>(w) & 15) == 0;
@@ -653,7 +671,8 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
     ScopedDevice scoped(dev);
     if (batch_elems > 0 && m > 0 && n > 0) {
         const int batch = static_cast<int>(batch_elems);
-        if (k <= 0 || skinny_fits(m, k, lhs, rhs)) {
+        if (k <= 0 || (skinny_fits(m, k, lhs, rhs) &&
+                       (batch > 1 || stream_columns(dev, (n + kSkinnyCols - 1) / kSkinnyCols)))) {
             SkinnyParams p{};
             p.x = static_cast<const uint16_t*>(lhs);
             one_segment(p, rhs, out, n);
@@ -731,17 +750,19 @@ inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255);
 // partials] (rows <= the streaming limit), or the GEMM output rows followed by
 // the hipBLASLt workspace.
 size_t o_proj_ws_bytes(int m, int n, int k) {
-    if (m <= skinny_max_m()) return skinny_ws_bytes(m, k, (n + kSkinnyCols - 1) / kSkinnyCols);
-    if (!use_hipblaslt()) return 256 + gemm_ws_bytes(m, k, 1, &n);  // the GEMM adds into the hidden rows in place
+    // the streaming kernels' region or the tiled GEMM's (which adds into the
+    // hidden rows in place), whichever the call takes
+    const size_t stream = m <= skinny_max_m() ? skinny_ws_bytes(m, k, (n + kSkinnyCols - 1) / kSkinnyCols) : 0;
+    if (!use_hipblaslt()) return std::max(stream, (m > skinny_max_m() ? 256 : 0) + gemm_ws_bytes(m, k, 1, &n));
     return align256(static_cast<size_t>(m) * n * 2) + kLtWorkspace;
 }
 // Workspace of the qkv entry point: the normed rows, then the streaming
 // kernel's [counters | partials] or the hipBLASLt workspace.
 size_t qkv_ws_bytes(int m, int k, int nq, int nkv) {
     const size_t normed = align256(static_cast<size_t>(m) * k * 2);
-    if (m <= skinny_max_m()) return normed + skinny_ws_bytes(m, k, nq / kSkinnyCols + 2 * (nkv / kSkinnyCols));
     const int ns[3] = {nq, nkv, nkv};
-    return normed + (use_hipblaslt() ? lt_ws_bytes() : gemm_ws_bytes(m, k, 3, ns));
+    const size_t stream = m <= skinny_max_m() ? skinny_ws_bytes(m, k, nq / kSkinnyCols + 2 * (nkv / kSkinnyCols)) : 0;
+    return normed + (use_hipblaslt() ? std::max(stream, lt_ws_bytes()) : std::max(stream, gemm_ws_bytes(m, k, 3, ns)));
 }
 }  // namespace ssa
 
@@ -776,7 +797,7 @@ extern "C" int supersonic_attn_gfx950_o_proj_residual(size_t device_ordinal, voi
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
-    if (skinny_fits(m, k, attn, o_proj_w)) {
+    if (skinny_fits(m, k, attn, o_proj_w) && stream_columns(dev, (n + kSkinnyCols - 1) / kSkinnyCols)) {
         SkinnyParams p{};
         p.x = static_cast<const uint16_t*>(attn);
         one_segment(p, o_proj_w, hidden, n);
@@ -871,7 +892,8 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
     // the three matrices as one column space of the weight-streaming kernel, or
     // as column segments of one GEMM
     const int ns[3] = {nq, nkv, nkv};
-    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0;
+    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
+                        nkv % kSkinnyCols == 0 && stream_columns(dev, (nq + 2 * nkv) / kSkinnyCols);
     unsigned* clear = nullptr;
     const int n_clear = skinny ? 0 : split_counters(m, k, 3, ns, rest, rest_bytes, &clear);
     const ProfileEvents ev = take_profile_events();
@@ -1023,8 +1045,9 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     const size_t pws_bytes = ws + need > pws ? static_cast<size_t>(ws + need - pws) : 0;
     const int ncb = (nq + 2 * nkv) / kSkinnyCols;
     const bool fused = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
-                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4);
-    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0;
+                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4) && stream_rope_columns(dev, ncb, k);
+    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
+                        nkv % kSkinnyCols == 0 && stream_columns(dev, ncb);
     const int ns[3] = {nq, nkv, nkv};
     unsigned* clear = nullptr;
     const int n_clear = fused || skinny ? 0 : split_counters(m, k, 3, ns, workspace ? pws : nullptr, pws_bytes, &clear);

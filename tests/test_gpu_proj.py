@@ -428,7 +428,7 @@ def test_o_proj_mid_rows(rows, hidden_dim, attn_dim, hdt):
     assert torch.equal(got[0], got[1])  # the same split, slices added in order
 
 
-@pytest.mark.parametrize("rows,hid,nq,nkv", [(13, 1024, 4096, 512), (40, 1024, 520, 72), (129, 512, 1024, 256),
+@pytest.mark.parametrize("rows,hid,nq,nkv", [(1, 1024, 4096, 512), (12, 2048, 8192, 512), (13, 1024, 4096, 512), (40, 1024, 520, 72), (129, 512, 1024, 256),
                                              (300, 2048, 1024, 256), (700, 1024, 1024, 136), (1030, 512, 4096, 256)])
 def test_qkv_proj_mid_rows(rows, hid, nq, nkv):
     """Three column segments that end inside a tile; the workspace comes from a larger call and holds its rows, so the
@@ -453,6 +453,12 @@ def test_qkv_proj_mid_rows(rows, hid, nq, nkv):
             # a normed element one bf16 ulp away (hardware rsqrt) moves an output by up to 2^-5 |w|, below 2^-7 here
             assert_ulps(out, ref, 2 * ulp(big) + 2.0 ** -7, f"qkv mid {name}")
             assert (out.float() == ref).float().mean().item() > 0.9, name
+
+
+# Few rows and more column blocks than CUs: the tiled GEMM, then the norm and RoPE kernel.
+@pytest.mark.parametrize("rows,hid,Hq,Hkv", [(1, 1024, 8, 2), (12, 2048, 16, 2)])
+def test_qkv_proj_rope_many_columns(rows, hid, Hq, Hkv):
+    test_qkv_proj_rope_matches_oracle(rows, hid, Hq, Hkv, 256, 64, True)
 
 
 def test_projections_share_a_workspace_over_row_counts():
