@@ -372,7 +372,7 @@ hipError_t take_wait_error_gemm(unsigned* bits);
 // The fused entry points with their scheduling knobs (decode.hip,
 // prefill.hip): decode planned for target_wgs workgroups (0: the whole GPU),
 // prefill on the dynamic schedule when claims is not NULL (16 zeroed
-// 128-byte counter lines).
+// 128-byte counter lines), free_wgs of the CUs being its own from the start.
 int decode_native(size_t device_ordinal, void* stream, int kv_dtype, size_t batch, size_t q_heads,
                   size_t kv_heads, size_t head_dim, size_t rotary_dim, size_t max_kv_len, float eps, float scale,
                   const void* q_proj, const void* k_new, const void* v_new, const void* q_norm_w,
@@ -384,7 +384,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
                    const void* q_proj, const void* k_new, const void* v_new, const void* q_norm_w,
                    const void* k_norm_w, const void* cos_table, const void* sin_table,
                    const supersonic_kv_cache* cache, void* out, void* workspace, size_t workspace_bytes,
-                   unsigned* claims);
+                   unsigned* claims, int free_wgs = 0);
 constexpr size_t kClaimBytes = 16 * 128;
 
 // Row repack with cast and zero padding (elementwise.hip): dst row

@@ -12,7 +12,8 @@
 //      the dynamic item schedule (items claimed longest first, each as the
 //      previous one nears its end), so the workgroups that find a free CU
 //      start at once and the rest as the decode's CUs free up, taking only
-//      what is left;
+//      what is left; a chunk worth a key split (prefill.hip) runs as pieces on
+//      the CUs that the decode's c leave instead;
 //   3. the caller's stream waits for the library stream.
 // Launch order keeps the decode's CUs its own: its workgroups are dispatched
 // before the prefill's are enqueued.  c comes from the two parts' estimated
@@ -190,7 +191,7 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
         rc = prefill_native(device_ordinal, ms->aux, kv_dtype, q_heads, kv_heads, head_dim, rotary_dim,
                             chunk->chunk_len, chunk->chunk_start, eps, scale, chunk->q_proj, chunk->k_new,
                             chunk->v_new, q_norm_w, k_norm_w, cos_table, sin_table, chunk->cache, chunk->out, pws,
-                            pbytes, claims);
+                            pbytes, claims, std::max(0, device_cu_count(dev) - wgs));
     // Join even after an error, so `stream` never runs ahead of work already
     // queued on the library stream.
     if (hipEventRecord(ms->join, ms->aux) != hipSuccess || hipStreamWaitEvent(st, ms->join, 0) != hipSuccess)

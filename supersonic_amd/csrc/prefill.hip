@@ -1332,16 +1332,19 @@ static hipError_t launch_prefill_d(hipStream_t st, const PrefillSplitParams& p) 
 // more workgroups than items.  part: room of part_bytes for a key split's sums,
 // or NULL for none.
 template <typename QT, bool FUSED>
-static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillSplitParams& p, void* part, size_t part_bytes) {
+static hipError_t launch_prefill(int device, int D, hipStream_t st, PrefillSplitParams& p, void* part, size_t part_bytes,
+                                 int free_wgs = 0) {
     const int items = p.nqt * p.Hq * p.B;
     int n = device_cu_count(device);
     if (n <= 0) n = 256;
     n = n >= 8 ? n & ~7 : n;
     p.n_wg = items < n ? items : n;
     p.piece = 0;
-    if (part && !p.claims && part_bytes >= prefill_part_bytes(D, n)) plan_key_split(p, n);
+    // beside a decode (dynamic schedule) the pieces share the CUs it leaves
+    const int ns = p.claims ? std::min(free_wgs, n) & ~7 : n;
+    if (part && ns >= 8 && part_bytes >= prefill_part_bytes(D, ns)) plan_key_split(p, ns);
     p.part_ml = static_cast<float*>(part);
-    p.part_o = p.part_ml + (part ? static_cast<size_t>(n) * 256 : 0);
+    p.part_o = p.part_ml + (part ? static_cast<size_t>(ns) * 256 : 0);
     switch (D) {
     case 64: return launch_prefill_d<QT, 64, FUSED>(st, p);
     case 128: return launch_prefill_d<QT, 128, FUSED>(st, p);
@@ -1488,7 +1491,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
                    const void* q_proj, const void* k_new, const void* v_new, const void* q_norm_w,
                    const void* k_norm_w, const void* cos_table, const void* sin_table,
                    const supersonic_kv_cache* cache, void* out, void* workspace, size_t workspace_bytes,
-                   unsigned* claims) {
+                   unsigned* claims, int free_wgs) {
     if (kv_dtype != SUPERSONIC_KV_BF16 && kv_dtype != SUPERSONIC_KV_FP8_E4M3) return SUPERSONIC_ERR_DTYPE;
     const bool fp8 = kv_dtype == SUPERSONIC_KV_FP8_E4M3;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return SUPERSONIC_ERR_HEAD_DIM;
@@ -1592,7 +1595,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
     }
     const ProfileEvents prof = take_profile_events();
     if (prof.before) (void)hipEventRecord(prof.before, st);
-    if (launch_prefill<bf16_t, true>(static_cast<int>(device_ordinal), static_cast<int>(head_dim), st, p, part, part_bytes) != hipSuccess)
+    if (launch_prefill<bf16_t, true>(static_cast<int>(device_ordinal), static_cast<int>(head_dim), st, p, part, part_bytes, free_wgs) != hipSuccess)
         return SUPERSONIC_ERR_LAUNCH;
     if (prof.after) (void)hipEventRecord(prof.after, st);
     return 0;

@@ -150,3 +150,38 @@ def test_mixed_one_part_matches_the_single_calls(monkeypatch):
         del os.environ["SUPERSONIC_DECODE_DETERMINISTIC"]
     assert torch.equal(outs[0][0], outs[1][0])
     assert torch.equal(outs[0][1].k, outs[1][1].k) and torch.equal(outs[0][1].v, outs[1][1].v)
+
+
+@pytest.mark.parametrize("S,start,batch,Hq,Hkv", [(60, 2000, 3, 8, 2), (300, 3000, 20, 16, 4), (17, 5000, 1, 6, 3)])
+@pytest.mark.parametrize("own_ws", [False, True])
+def test_mixed_key_split_chunk(S, start, batch, Hq, Hkv, own_ws):
+    """A short chunk behind a long prefix runs as key pieces on the CUs that the decode leaves; both parts against the
+    single calls, twice on one workspace."""
+    announce(f"mixed key split {S}@{start} + {batch} decodes, {Hq}/{Hkv} heads, caller workspace {own_ws}")
+    D, rot = 256, 64
+    g = torch.Generator(device=DEV).manual_seed(91)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, start + S + 1, 1.0e7))
+    qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
+    lens = [100 + 37 * i for i in range(batch)]
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    kc, vc = rnd(1, Hkv, start + S, D), rnd(1, Hkv, start + S, D)
+    kd, vd = rnd(batch, Hkv, max(lens) + 1, D), rnd(batch, Hkv, max(lens) + 1, D)
+    xc = [rnd(S, Hq * 2 * D), rnd(S, Hkv * D), rnd(S, Hkv * D)]
+    xd = [rnd(batch, Hq * 2 * D), rnd(batch, Hkv * D), rnd(batch, Hkv * D)]
+    shape = dict(q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot)
+    nan = lambda n: torch.full((n, Hq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    c1, d1 = K.KvCache(kc.clone(), vc.clone()), K.KvCache(kd.clone(), vd.clone())
+    ref_c, ref_d = nan(S), nan(batch)
+    K.fused_prefill(0, *xc, qw, kw, cos, sin, c1, ref_c, chunk_start=start, **shape)
+    K.fused_decode(0, *xd, qw, kw, cos, sin, pos, d1, ref_d, max_kv_len=max(lens) + 1, **shape)
+    c2, d2 = K.KvCache(kc.clone(), vc.clone()), K.KvCache(kd.clone(), vd.clone())
+    chunk = dict(zip(("q_proj", "k_new", "v_new"), xc), cache=c2, out=nan(S), chunk_start=start)
+    dec = dict(zip(("q_proj", "k_new", "v_new"), xd), cache=d2, out=nan(batch), positions=pos, max_kv_len=max(lens) + 1)
+    ws = torch.zeros(K.mixed_workspace_size(False, Hq, Hkv, D, chunk, dec), dtype=torch.uint8, device=DEV) if own_ws else None
+    for _ in range(2):
+        K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, decode=dec, workspace=ws, **shape)
+        torch.cuda.synchronize()
+        check(chunk["out"], ref_c.float().cpu(), TOL_BF16, "mixed split chunk")
+        check(dec["out"], ref_d.float().cpu(), TOL_BF16, "mixed split decode")
+    assert torch.equal(c1.k, c2.k) and torch.equal(c1.v, c2.v) and torch.equal(d1.k, d2.k) and torch.equal(d1.v, d2.v)
