@@ -44,8 +44,8 @@ extern "C" {
 #define SUPERSONIC_ERR_SYNC 1008
 #define SUPERSONIC_ERR_RANGE 1009
 #define SUPERSONIC_ERR_CACHE 1010
-/* The device cannot co-schedule the persistent layer's grid (no cooperative
- * launch, or the grid does not fit at once). */
+/* Kept for its callers: the persistent layer no longer needs its grid
+ * co-scheduled and does not return it. */
 #define SUPERSONIC_ERR_COOPERATIVE 1011
 /* Bits of supersonic_attn_gfx950_wait_status(): a bounded wait gave up. */
 #define SUPERSONIC_WAIT_LAYER_BARRIER 1u /* persistent layer: grid barrier */
@@ -405,9 +405,10 @@ int supersonic_attn_gfx950_qkv_proj_rope(
  * hidden [batch, hidden_dim] bf16 (hidden_dtype 2) or f32 holding bf16 values
  * (1); weights as supersonic_attn_gfx950_qkv_proj / _o_proj_residual; cache,
  * positions, tables as supersonic_attn_gfx950_decode.  One workgroup per
- * compute unit, three phases separated by device-wide barriers, launched
- * cooperatively so that every workgroup of the grid is resident at once
- * (SUPERSONIC_ERR_COOPERATIVE when the device cannot do that).  Limits: batch <= 16,
+ * compute unit, three phases separated by device-wide barriers, in an ordinary
+ * launch: when other work keeps workgroups of the grid from a compute unit for
+ * some 10 ms, the kernel leaves and a lone workgroup launched behind it runs the
+ * layer (slowly, same result).  Limits: batch <= 16,
  * batch * hidden_dim <= 32768 and batch * q_heads * head_dim <= 32768,
  * hidden_dim % 16 == 0, head_dim 128/256, q_heads / kv_heads <= 4, 16-byte
  * aligned hidden and weights (otherwise SUPERSONIC_ERR_RANGE: use the
@@ -480,7 +481,7 @@ int supersonic_attn_rope_tables(size_t rotary_dim, size_t max_pos, double theta,
  * set since the last call in *bits and clears them.  A set bit means some
  * output since then is wrong, and the workspace of the call that set it must be
  * zero-filled again before reuse.  Under the documented preconditions
- * (cooperative launch, zero-filled workspaces) no wait gives up.  The
+ * (zero-filled workspaces) no wait gives up.  The
  * synchronous drop-ins check the word themselves and return their sync-failure
  * status.  SUPERSONIC_WAIT_POLLS (environment) overrides the poll bound, for
  * tests that force the give-up path. */

@@ -140,12 +140,13 @@ struct DecodeLds {
 // / gate are read and the output written with device-coherent accesses (they
 // are exchanged with other workgroups of the same kernel).
 struct NoMid {
-    __device__ void operator()() const {}
+    __device__ bool operator()() const { return true; }
 };
 
 // mid: called by every thread once, after the work item is planned and its
 // first K/V block fetched, before q / k_new / v_new / gate are read (not
-// called when the workgroup has no work item).
+// called when the workgroup has no work item); false (from every thread)
+// leaves the item undone.
 template <typename QT, bool FP8, int D, int GP, bool COH = false, typename Mid = NoMid>
 __device__ __forceinline__ void decode_split_body(const DecodeParams& p, int vbx, int vby, int vbz,
                                                   DecodeLds<D, GP>& L, const Mid& mid = Mid()) {
@@ -492,7 +493,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& p, int vbx
         // written by another phase) runs before any of the rows is read.
         if constexpr (kMid) {
             fetch(max(0, min(wave, nblk - 1)), A);
-            mid();
+            if (!mid()) return;
         }
         for (int r = wave + NW; r < rows; r += NW) {
             float x[EPL], vx[EPL], w[EPL], cs[EPL], sn[EPL];

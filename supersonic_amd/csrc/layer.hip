@@ -4,8 +4,7 @@
 // kernels/qwen36_moe_persistent/full_attn_phase.cuh:1-20, and the HIP
 // megakernel's steps A-G, kernels/full_attention_4b.hip:4842-5577).
 //
-// One workgroup per compute unit (all of them resident at once: a cooperative
-// launch), three phases
+// One workgroup per compute unit (an ordinary launch, see below), three phases
 // separated by device-wide barriers:
 //   1. input RMSNorm (applied while each workgroup stages the rows in LDS) and
 //      the Q/K/V weight stream, 16 output columns per workgroup task;
@@ -21,7 +20,6 @@
 // kernel.
 #include <algorithm>
 #include <cstdlib>
-#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -37,7 +35,7 @@ struct LayerParams {
     SkinnyLdsParams qkv;  // phase 1: three segments, NORM staging from the hidden rows
     DecodeParams dec;     // phase 2: fused decode step, ragged plan over the grid
     SkinnyLdsParams op;   // phase 3: attn -> hidden (residual in place)
-    unsigned* bar;        // barrier counters [0..2] and flags [32], [48] (another cache line), zero between calls
+    unsigned* bar;        // barrier counters [0..2], flags [32], [48] (another cache line) and [8], zero between calls
     int polls;            // bound of a barrier wait (kLayerSpin)
     // > 0: the decode step is expected to have this many work items (one
     // sequence of length max_kv_len); the last `hint` workgroups then take
@@ -48,6 +46,7 @@ struct LayerParams {
 
 constexpr int kLayerThreads = 64 * kSkinnyWaves;  // = 64 * decode_waves(4)
 constexpr int kLayerSpin = 1 << 20;               // bounded barrier wait
+constexpr int kLayerAlonePolls = 1 << 14;         // ... with workgroups missing
 
 // Every value one phase hands to the next is written and read with
 // device-coherent (sc1) accesses, so the barrier needs no cache writeback or
@@ -70,33 +69,68 @@ constexpr int kLayerSpin = 1 << 20;               // bounded barrier wait
 // per-XCD cache line.  This is what an agent-scope release / acquire pair
 // provides, without the L2 writeback and invalidate those emit.
 //
-// The launch is cooperative (every workgroup co-resident, or the launch is
-// refused), so a wait can only expire on a workspace whose counters were not
-// zero: it then sets kWaitLayerBarrier in the error word and carries on, so
-// that the kernel still exits.
+// Every workgroup arrives at barrier 0, so once it opens all of them are
+// running and no later wait can depend on one that has no CU.  The launch
+// itself does not promise that.  (A cooperative one does, through a queue of its
+// own: 17-20 us a call on this runtime: 1 sequence of 2048 tokens, 8/2 heads,
+// hidden 1024, 49.2 us a layer, 32.5 with this.)
+// Instead a wait that lasts (kLayerAlonePolls, about 10 ms) while workgroups are
+// missing from barrier 0 may be holding the CU that they need: it then closes
+// the barrier for good (flag 0 -> kFlagAlone, one compare-and-swap against the
+// last arrival's 0 -> kFlagOpen), every workgroup leaves, also those that
+// start later, and decode_layer_alone_kernel behind runs the layer.  That is
+// sound at any time before barrier 0 opens: no item is past its grid wait, so
+// the hidden rows and the cache are untouched.
+// With every workgroup arrived, a wait can only expire on a workspace whose
+// counters were not zero: it then sets kWaitLayerBarrier in the error word and
+// carries on, so that the kernel still exits.
+enum : unsigned { kFlagOpen = 1u, kFlagAlone = 2u };
+enum LayerWait { kLayerGo, kLayerLeave };
+constexpr int kLayerAloneWord = 8;  // in LayerParams::bar: the layer is left to decode_layer_alone_kernel
 constexpr int kArriveThread = kLayerThreads - 64;
-__device__ __forceinline__ void grid_arrive(unsigned* ctr, unsigned* flag, unsigned n) {
+// This workgroup's coherent stores are complete, for all of its threads.
+__device__ __forceinline__ void stores_complete() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores are complete
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
+}
+__device__ __forceinline__ void grid_arrive(unsigned* ctr, unsigned* flag, unsigned n) {
+    stores_complete();
     if (threadIdx.x == kArriveThread) {
         const unsigned prev = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == n - 1) __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (prev == n - 1) atomicCAS(flag, 0u, static_cast<unsigned>(kFlagOpen));
     }
 }
-__device__ __forceinline__ void grid_wait(unsigned* flag, int polls) {
+// Waits for `flag` (bar + 32: barrier 0's, bar + 48: barrier 1's).
+__device__ __forceinline__ LayerWait grid_wait(unsigned* bar, unsigned* flag, unsigned nwg, int polls, int& res) {
     if (threadIdx.x == 0) {
+        const int alone_polls = min(polls, kLayerAlonePolls);
+        LayerWait r = kLayerGo;
         for (int it = 0;; ++it) {
-            if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) break;
+            if (load_agent_u32(flag) == kFlagOpen) break;
+            if ((it & 63) == 63 || it >= alone_polls) {
+                const unsigned f0 = load_agent_u32(bar + 32);
+                if (f0 == kFlagAlone) {
+                    r = kLayerLeave;
+                    break;
+                }
+                if (it >= alone_polls && f0 == 0u && static_cast<int>(load_agent_u32(bar)) < static_cast<int>(nwg)) {
+                    atomicCAS(bar + 32, 0u, static_cast<unsigned>(kFlagAlone));
+                    continue;  // closed, or opened meanwhile: the next poll sees which
+                }
+            }
             if (it >= polls) {
                 wait_expired(kWaitLayerBarrier);
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
         }
+        res = r;
     }
     __syncthreads();
+    // (the next wait writes it after that barrier's arrival, which synchronises)
+    return static_cast<LayerWait>(__builtin_amdgcn_readfirstlane(res));
 }
 
 template <typename HT, bool FP8, int D>
@@ -106,13 +140,17 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
         DecodeLds<D, 4> d;
         SkinnyLds s;
     } lds;
+    __shared__ int wait_res;
     const int w = blockIdx.x;
     const unsigned nwg = gridDim.x;
     const int ncb_qkv = P.qkv.cb_end[2], ncb_op = P.op.cb_end[2];
+    const int nq = static_cast<int>(nwg) - P.hint;
+    const int shift = min(max(ncb_qkv - static_cast<int>(nwg), 0), static_cast<int>(nwg));
+    const int item = P.hint > 0 ? (w >= nq ? w - nq : P.hint + w)
+                                : (w - shift + static_cast<int>(nwg)) % static_cast<int>(nwg);
     // 1. input norm + Q/K/V projections on the first nq workgroups: column
     // blocks w, w + nq, ...; a workgroup with two left takes them together
     // (one staging of the rows, both weight streams in flight)
-    const int nq = static_cast<int>(nwg) - P.hint;
     for (int cb = w; cb < ncb_qkv && w < nq;) {
         if (cb + nq < ncb_qkv) {
             skinny_lds_body<bf16_t, false, false, true, HT, false, true, SkinnyLds, true>(P.qkv, RopeEpi{}, cb, 0,
@@ -133,35 +171,36 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
     // an item does not wait (only the readers of phase 1's output do).
     // With a hint the expected items sit on the workgroups without phase-1
     // work (any further item on the others).
-    const int shift = min(max(ncb_qkv - static_cast<int>(nwg), 0), static_cast<int>(nwg));
-    const int item = P.hint > 0 ? (w >= nq ? w - nq : P.hint + w)
-                                : (w - shift + static_cast<int>(nwg)) % static_cast<int>(nwg);
     grid_arrive(&P.bar[0], &P.bar[32], nwg);
+    LayerWait res = kLayerGo;
     bool had_item = false;
     decode_split_body<bf16_t, FP8, D, 4, true>(P.dec, item, 0, 0, lds.d, [&]() {
-        grid_wait(&P.bar[32], P.polls);
+        res = grid_wait(P.bar, &P.bar[32], nwg, P.polls, wait_res);
         had_item = true;
+        return res == kLayerGo;
     });
-    if (!had_item && w < ncb_op) {
-        // An output-projection workgroup without a decode item copies its
-        // first task's weight rows into an LDS sink while the items run, so
-        // that phase 3 finds them in this XCD's L2.  (The copies complete
-        // before it arrives at barrier 1, which waits for its loads.)
-        const int k = P.op.k;
-        const int bytes = min(kSkinnyCols, P.op.n_seg[0] - w * kSkinnyCols) * k * 2;
-        const __amdgpu_buffer_rsrc_t r =
-            uniform_rsrc(reinterpret_cast<const uint8_t*>(P.op.w[0] + static_cast<int64_t>(w) * kSkinnyCols * k), bytes);
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        for (int off = wave * 1024; off < bytes; off += kSkinnyWaves * 1024)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds.s.xs, 16,
-                                                     off + lane * 16, 0, 0, 0);
+    if (res == kLayerGo) {
+        if (!had_item && w < ncb_op) {
+            // An output-projection workgroup without a decode item copies its
+            // first task's weight rows into an LDS sink while the items run, so
+            // that phase 3 finds them in this XCD's L2.  (The copies complete
+            // before it arrives at barrier 1, which waits for its loads.)
+            const int k = P.op.k;
+            const int bytes = min(kSkinnyCols, P.op.n_seg[0] - w * kSkinnyCols) * k * 2;
+            const __amdgpu_buffer_rsrc_t r =
+                uniform_rsrc(reinterpret_cast<const uint8_t*>(P.op.w[0] + static_cast<int64_t>(w) * kSkinnyCols * k), bytes);
+            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+            for (int off = wave * 1024; off < bytes; off += kSkinnyWaves * 1024)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds.s.xs, 16,
+                                                         off + lane * 16, 0, 0, 0);
+        }
+        // Barrier 1: every workgroup arrives; those with an output-projection
+        // task wait for all of them.
+        grid_arrive(&P.bar[1], &P.bar[48], nwg);
+        if (w < ncb_op) res = grid_wait(P.bar, &P.bar[48], nwg, P.polls, wait_res);
     }
-    // Barrier 1: every workgroup arrives; those with an output-projection
-    // task wait for all of them.
-    grid_arrive(&P.bar[1], &P.bar[48], nwg);
-    if (w < ncb_op) grid_wait(&P.bar[48], P.polls);
     // 3. output projection + residual
-    for (int cb = w; cb < ncb_op; cb += nwg) {
+    for (int cb = w; cb < ncb_op && res == kLayerGo; cb += nwg) {
         skinny_lds_body<HT, true, false, false, bf16_t, true, false>(P.op, RopeEpi{}, cb, 0, lds.s);
         __syncthreads();
     }
@@ -172,6 +211,9 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
     if (threadIdx.x == 0) {
         const unsigned prev = __hip_atomic_fetch_add(&P.bar[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (prev == nwg - 1) {
+            // (a closed barrier 0 leaves the layer to decode_layer_alone_kernel)
+            if (load_agent_u32(&P.bar[32]) == kFlagAlone)
+                __hip_atomic_store(&P.bar[kLayerAloneWord], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&P.bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&P.bar[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&P.bar[32], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -179,6 +221,36 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
             __hip_atomic_store(&P.bar[2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+// The whole layer on one workgroup, after a decode_layer_kernel whose barrier 0
+// was closed (grid_wait); otherwise it only looks and leaves, which costs a
+// call 2-3 us.
+template <typename HT, bool FP8, int D>
+__global__ __launch_bounds__(kLayerThreads) void decode_layer_alone_kernel(LayerParams P) {
+    __shared__ union Lds {
+        DecodeLds<D, 4> d;
+        SkinnyLds s;
+    } lds;
+    if (load_agent_u32(&P.bar[kLayerAloneWord]) == 0u) return;
+    for (int cb = 0; cb < P.qkv.cb_end[2]; ++cb) {
+        skinny_lds_body<bf16_t, false, false, true, HT, false, true>(P.qkv, RopeEpi{}, cb, 0, lds.s);
+        __syncthreads();
+    }
+    stores_complete();
+    DecodeParams dec = P.dec;
+    dec.target = 1;  // one split a sequence and kv head
+    for (int i = 0; i < dec.B * dec.Hkv; ++i) {
+        decode_split_body<bf16_t, FP8, D, 4, true>(dec, i, 0, 0, lds.d);
+        __syncthreads();
+    }
+    stores_complete();
+    for (int cb = 0; cb < P.op.cb_end[2]; ++cb) {
+        skinny_lds_body<HT, true, false, false, bf16_t, true, false>(P.op, RopeEpi{}, cb, 0, lds.s);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&P.bar[kLayerAloneWord], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Workgroups of one layer-kernel instance resident at once, per device.
@@ -226,11 +298,6 @@ inline LayerWs layer_ws(int B, int Hq, int Hkv, int D, int max_len) {
     return w;
 }
 
-static bool plain_launch() {
-    const char* v = getenv("SUPERSONIC_LAYER_LAUNCH");
-    return v && std::strcmp(v, "plain") == 0;
-}
-
 template <typename HT, bool FP8, int D>
 static int launch_layer(int device, hipStream_t st, LayerParams& P) {
     const int grid = std::min(layer_grid<HT, FP8, D>(device), kLayerMaxGrid);
@@ -256,35 +323,9 @@ static int launch_layer(int device, hipStream_t st, LayerParams& P) {
     }
     P.polls = wait_polls(kLayerSpin);
     P.dec.merge_polls = wait_polls(kMergePoll);
-    // Cooperative launch: the runtime refuses a grid whose workgroups cannot
-    // all be resident at once, which the barriers need (as the reference's
-    // persistent kernel does, kernels/full_attention_bridge_4b.cpp:4918-4927, :4963).
-    // SUPERSONIC_LAYER_LAUNCH=plain: an ordinary launch (no co-residency
-    // guarantee; a barrier that gives up is reported by the error word).
-    if (plain_launch()) {
-        hipLaunchKernelGGL((decode_layer_kernel<HT, FP8, D>), dim3(grid), dim3(kLayerThreads), 0, st, P);
-        return hipGetLastError() == hipSuccess ? 0 : SUPERSONIC_ERR_LAUNCH;
-    }
-    void* args[] = {&P};
-    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&decode_layer_kernel<HT, FP8, D>),
-                                                    dim3(grid), dim3(kLayerThreads), args, 0, st);
-    if (e == hipErrorCooperativeLaunchTooLarge) return SUPERSONIC_ERR_COOPERATIVE;
-    return e == hipSuccess ? 0 : SUPERSONIC_ERR_LAUNCH;
-}
-
-// Whether `device` runs cooperative launches (cached per device).
-static bool cooperative_ok(int device) {
-    static std::mutex mu;
-    static std::vector<int> ok;
-    std::lock_guard<std::mutex> lock(mu);
-    if (device < 0) return false;
-    if (static_cast<size_t>(device) >= ok.size()) ok.resize(device + 1, -1);
-    if (ok[device] < 0) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess) v = 0;
-        ok[device] = v != 0;
-    }
-    return ok[device] != 0;
+    hipLaunchKernelGGL((decode_layer_kernel<HT, FP8, D>), dim3(grid), dim3(kLayerThreads), 0, st, P);
+    hipLaunchKernelGGL((decode_layer_alone_kernel<HT, FP8, D>), dim3(1), dim3(kLayerThreads), 0, st, P);
+    return hipGetLastError() == hipSuccess ? 0 : SUPERSONIC_ERR_LAUNCH;
 }
 
 hipError_t take_wait_error_layer(unsigned* bits) { return take_wait_error(bits); }
@@ -413,7 +454,6 @@ extern "C" int supersonic_attn_gfx950_decode_layer(
     o.k = static_cast<int>(adim);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int dev = static_cast<int>(device_ordinal);
-    if (!plain_launch() && !cooperative_ok(dev)) return SUPERSONIC_ERR_COOPERATIVE;
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     int rc;

@@ -201,3 +201,26 @@ def test_decode_layer_expired_barrier_is_reported(monkeypatch):
     assert K.wait_status() == 0
     ref, v_ref = oracle_layer(c)
     check_layer(c, out, cache, ref, v_ref)
+
+
+@pytest.mark.parametrize("name", ["config1", "config2_b4_ragged", "one_sequence_fp8_paged", "f32_hidden"])
+def test_decode_layer_missing_workgroups_run_alone(name, monkeypatch):
+    """The host presets barrier 0's counter below zero, as if workgroups had found no CU, and shortens the wait: the
+    barrier is closed, the lone workgroup behind the kernel runs the layer, and the result is right, nothing is
+    reported and the counters are back at zero for the next, ordinary call."""
+    kw = CASES[name]
+    announce(f"persistent decode layer, workgroups missing: {name}")
+    for held in (True, False):
+        c = layer_case(135, **kw)
+        if held:
+            ws = torch.zeros(K.decode_layer_workspace_size(c["B"], c["hid"], c["Hq"], c["Hkv"], c["D"],
+                                                           max(c["lens"]) + 1), dtype=torch.uint8, device=DEV)
+            ws[:4].view(torch.int32).fill_(-1000)
+            monkeypatch.setenv("SUPERSONIC_WAIT_POLLS", "16")
+        else:
+            monkeypatch.delenv("SUPERSONIC_WAIT_POLLS")
+        out, cache = run_layer(c, ws)
+        assert K.wait_status() == 0
+        ref, v_ref = oracle_layer(c)
+        check_layer(c, out, cache, ref, v_ref)
+        assert int(ws[:256].count_nonzero()) == 0, "barrier words not reset"
