@@ -7,9 +7,9 @@
 // 128 x 128: 0.61, 256 x 128: 0.95; with every copy served by L2 and no MFMAs
 // 0.40 / 0.45 / 0.58), and at 256 x 128 the MFMAs at the clock they leave.
 // Measured (one MI355X, 256 x 256 tiles before): o_proj 4096 -> 4096 at 32 rows
-// 91.7 -> 11.1 us, 128 rows 100 -> 16.6, 512 rows 104 -> 29.8, 1000 rows 103 ->
+// 91.7 -> 11.0 us, 128 rows 100 -> 17.0, 512 rows 104 -> 29.8, 1000 rows 103 ->
 // 40.0, 2000 rows 103 -> 63.0 (1.07 PFLOP/s), 4096 rows 127.9 -> 124.3; norm +
-// Q/K/V 4096 -> 10240 at 32 rows 95.3 -> 24, 512 rows 109 -> 58, 4096 rows
+// Q/K/V 4096 -> 10240 at 32 rows 95.3 -> 22.3, 512 rows 109 -> 58, 4096 rows
 // 325 -> 306.
 //
 // Workgroup: a BM x BN tile of out over a slice of k, four or eight compute
@@ -30,6 +30,7 @@
 // slice order (the result does not depend on the arrival order), resets the
 // counter and writes the output.  Nothing waits for another workgroup.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "gemm.hpp"
@@ -40,6 +41,7 @@ namespace ssa {
 constexpr int kTileBK = 64;
 constexpr int kTileRowB = 128;      // LDS row: 64 bf16
 constexpr int kTileCopyWaves = 4;
+constexpr int kNontemporal = 2;     // cache-policy bit of a copy
 
 struct GemmTileParams {
     const uint16_t* a;
@@ -79,7 +81,7 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
     else if constexpr (MAX > 0) wait_tiles<C, MAX - 1>(tiles);
 }
 
-template <int BM, int BN, int NST, int NW, int NC, int EPI>
+template <int BM, int BN, int NST, int NW, int EPI>
 __global__ __launch_bounds__(64 * (NW + kTileCopyWaves)) __attribute__((amdgpu_waves_per_eu(3))) void gemm_tile_kernel(GemmTileParams p) {
     constexpr int kTileWaves = NW;
     constexpr int kATile = BM * kTileRowB, kWTile = BN * kTileRowB, kStage = kATile + kWTile;
@@ -130,10 +132,10 @@ __global__ __launch_bounds__(64 * (NW + kTileCopyWaves)) __attribute__((amdgpu_w
     if (wave >= kTileWaves) {
         // ---- copy waves.  Copy instruction c of a tile moves 8 rows (1 KB):
         // rows of a for c < BM / 8, then rows of w; copy wave cw takes
-        // instructions cw, cw + NC, ...  Lane l: row l / 8, physical chunk
+        // instructions cw, cw + kTileCopyWaves, ...  Lane l: row l / 8, physical chunk
         // l % 8.  The whole offset goes in the per-lane operand (the range
         // check does not cover the scalar offset).
-        constexpr int kCopies = (BM + BN) / 8 / NC;
+        constexpr int kCopies = (BM + BN) / 8 / kTileCopyWaves;
         constexpr int kOOB = 0x7ffffff0;  // past any range: reads zero
         const int cw = wave - kTileWaves;
         const uint16_t* abase = p.a + b * p.a_bs + static_cast<int64_t>(m0) * p.lda;
@@ -141,27 +143,41 @@ __global__ __launch_bounds__(64 * (NW + kTileCopyWaves)) __attribute__((amdgpu_w
         const __amdgpu_buffer_rsrc_t ar = gemm_tile_rsrc(abase, static_cast<int64_t>(p.m - m0) * p.lda * 2);
         const __amdgpu_buffer_rsrc_t wr = gemm_tile_rsrc(wbase, static_cast<int64_t>(ns - n0) * p.k * 2);
         const int crow = lane >> 3;
-        auto issue = [&](int kt) {
+        auto issue = [&](int kt, auto once) {
             const int k0 = kt * kTileBK;
             uint8_t* st = lds + ((kt - kt0) % NST) * kStage;
 #pragma unroll
             for (int j = 0; j < kCopies; ++j) {
-                const int c = NC * j + cw;
-                const bool isa = NC * j < BM / 8;   // the same for every copy wave (NC divides BM / 8)
+                const int c = kTileCopyWaves * j + cw;
+                const bool isa = kTileCopyWaves * j < BM / 8;   // the same for every copy wave (kTileCopyWaves divides BM / 8)
                 const int row = 8 * (isa ? c : c - BM / 8) + crow;
                 const int ch = (lane & 7) ^ ((row >> 1) & 7);
                 const int off = k0 + 8 * ch < p.k ? row * static_cast<int>(isa ? p.lda : p.k) * 2 + (k0 + 8 * ch) * 2 : kOOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(isa ? ar : wr, (__attribute__((address_space(3))) void*)(st + 1024 * c),
-                                                         16, off, 0, 0, 0);
+                if (isa)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(ar, (__attribute__((address_space(3))) void*)(st + 1024 * c), 16,
+                                                             off, 0, 0, 0);
+                else if constexpr (decltype(once)::value)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(st + 1024 * c), 16,
+                                                             off, 0, 0, kNontemporal);
+                else
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(st + 1024 * c), 16,
+                                                             off, 0, 0, 0);
             }
         };
-        for (int v = 0; v < NST - 1; ++v)
-            if (kt0 + v < KT) issue(kt0 + v);
-        for (int kt = kt0; kt < KT; ++kt) {
-            wait_tiles<kCopies, NST - 2>(KT - 1 - kt);  // tile kt has landed
-            __builtin_amdgcn_s_barrier();               // ... and the stage of tile kt - 1 has been read
-            if (kt + NST - 1 < KT) issue(kt + NST - 1);
-        }
+        auto copy_tiles = [&](auto once) {
+            for (int v = 0; v < NST - 1; ++v)
+                if (kt0 + v < KT) issue(kt0 + v, once);
+            for (int kt = kt0; kt < KT; ++kt) {
+                wait_tiles<kCopies, NST - 2>(KT - 1 - kt);  // tile kt has landed
+                __builtin_amdgcn_s_barrier();               // ... and the stage of tile kt - 1 has been read
+                if (kt + NST - 1 < KT) issue(kt + NST - 1, once);
+            }
+        };
+        // One m-tile: each weight is read by one workgroup and passes the caches
+        // by (norm + Q/K/V 4096 -> 10240 at 8 rows 22.0 -> 19.7 us, 32 rows
+        // 24.0 -> 22.3; o_proj 4096 -> 4096 at 16 rows 11.0 -> 10.6).
+        if (BM <= 64 && p.mt == 1) copy_tiles(std::true_type{});
+        else copy_tiles(std::false_type{});
     } else {
         // ---- compute waves.  Operand reads: row lane % 16 of a 16-row block,
         // logical chunk 4 s + lane / 16 of k32 step s.
@@ -289,9 +305,9 @@ template <int BM, int BN, int NST, int NW>
 static int launch_tile(hipStream_t st, const GemmTileParams& p, int batch, int epilogue) {
     const dim3 grid(static_cast<unsigned>(p.full + (p.tiles - p.full) * p.ks), static_cast<unsigned>(batch)), blk(64 * (NW + kTileCopyWaves));
     switch (epilogue) {
-    case kGemmResidualBf16: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kTileCopyWaves, kGemmResidualBf16>), grid, blk, 0, st, p); break;
-    case kGemmResidualF32: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kTileCopyWaves, kGemmResidualF32>), grid, blk, 0, st, p); break;
-    default: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kTileCopyWaves, kGemmStore>), grid, blk, 0, st, p); break;
+    case kGemmResidualBf16: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kGemmResidualBf16>), grid, blk, 0, st, p); break;
+    case kGemmResidualF32: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kGemmResidualF32>), grid, blk, 0, st, p); break;
+    default: hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, NST, NW, kGemmStore>), grid, blk, 0, st, p); break;
     }
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }

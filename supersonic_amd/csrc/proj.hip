@@ -380,7 +380,7 @@ int skinny_max_m() {
 // rounds, and short rows of W leave a wave too few loads in flight (one
 // MI355X, 8 rows: o_proj 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled;
 // norm + Q/K/V 1024 -> 5120, 320 blocks, 13.0 against 11.4; 2048 -> 9216, 576
-// blocks, 20.0 against 12.5; 4096 -> 10240, 640 blocks, 23.2 against 21.9).
+// blocks, 20.0 against 12.0; 4096 -> 10240, 640 blocks, 23.2 against 19.7).
 // A row limit or a GEMM in the environment asks for the streaming kernels.
 bool stream_columns(int dev, int64_t ncb) {
     const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
