@@ -573,7 +573,7 @@ class Workloads:
                 "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                              "frac": round(ach / HBM_PEAK_GBS, 4),
                              "traffic": measured_traffic("qkv"),  # the projection kernel's bytes (the norm kernel: 128 KB)
-                             "kernel": "input_norm_kernel + skinny_lds_kernel (3 segments), events around both",
+                             "kernel": "input_norm_kernel + gemm_tile_kernel (3 segments), events around both",
                              "bytes_per_launch": kern_bytes}}
 
     def qkv_rope(self):
@@ -610,7 +610,7 @@ class Workloads:
                 "ms_per_step": step_ms, "kernel_ms": kern_ms, "bytes": kern_bytes,
                 "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                              "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": measured_traffic("qkv_rope"),
-                             "kernel": "input_norm_kernel + skinny_lds_kernel (fused norm/RoPE epilogue), events around both",
+                             "kernel": "input_norm_kernel + gemm_tile_kernel + qk_norm_rope_kernel, events around all three",
                              "bytes_per_launch": kern_bytes}}
 
     def layer_graph(self):
@@ -675,7 +675,7 @@ class Workloads:
                 K.decode_layer(0, hidden, nw, wq, wk, wv, qw, kw, wo, cos, sin, pos, cache, lws, q_heads=Hq,
                                kv_heads=Hkv, head_dim=D, rotary_dim=rot, max_kv_len=L + 1, stream=st)
             pers_ms = timed_on_stream(persistent)
-            # the same kernel through an ordinary launch (no co-residency guarantee)
+            # once more with the variable that used to ask for the ordinary launch (no effect now)
             os.environ["SUPERSONIC_LAYER_LAUNCH"] = "plain"
             try:
                 plain_ms = timed_on_stream(persistent)

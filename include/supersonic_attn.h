@@ -154,8 +154,9 @@ int supersonic_qwen35_hip_split_qgate(
  * rhs [batch, n, k], out [batch, m, n], bf16 only (the projections, o_proj
  * included, of prefill_engine.rs:356-414).  Replaces
  * kernels/full_attention_bridge_4b.cpp:3683-3704 (kernel full_attention_4b.hip:2513-2575),
- * bound at prefill_ffi.rs:782-792.  m <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M): HBM-streaming MFMA kernel; larger m:
- * the hand-written tiled MFMA GEMM (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt).
+ * bound at prefill_ffi.rs:782-792.  m <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M) and at
+ * most one 16-column block a CU: HBM-streaming MFMA kernel; otherwise the
+ * hand-written tiled MFMA GEMM (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt).
  * Status: 272 bad dtype, 270 launch, 271 sync. */
 int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(
     int dtype, size_t device_ordinal, size_t batch_elems, int m, int n, int k,
@@ -375,10 +376,10 @@ int supersonic_attn_gfx950_qkv_proj(
  * all bf16; cache (NULL: none) is a bf16 cache view that receives k_out / v_out
  * of row r at slot positions[r] of sequence r.  The outputs feed
  * supersonic_attn_gfx950_decode_attend (q, gate, kv_lens = positions + 1).
- * Rows <= 12 with rows * hidden_dim <= 32768 and head_dim 128/256: one
- * weight-streaming launch whose epilogue normalises and rotates each head as
- * its last column block completes; otherwise the projections, then one wave
- * per (row, head).  workspace: at least
+ * Rows <= 12 with rows * hidden_dim <= 32768, head_dim 128/256 and at most one
+ * 16-column block a CU: one weight-streaming launch whose epilogue normalises
+ * and rotates each head as its last column block completes; otherwise the
+ * projections, then one wave per (row, head).  workspace: at least
  * supersonic_attn_gfx950_qkv_proj_rope_workspace_size() bytes, zero-filled
  * before first use (per-head arrival counters left at zero by every call),
  * or NULL for a library-owned buffer.  Status: SUPERSONIC_ERR_CACHE for an
@@ -433,8 +434,8 @@ int supersonic_attn_gfx950_decode_layer(
  * (hidden_dtype 2, the prefill engine's hidden) or f32 holding bf16 values
  * (hidden_dtype 1, the megakernel's hidden_f32).  Replaces the megakernel's
  * step G (full_attention_4b.hip:5481-5577) and matmul_proj + residual_add of
- * prefill_engine.rs:2308-2334.  rows <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M, at most 64) with attn_dim % 8 == 0: one
- * HBM-streaming MFMA kernel with the residual fused; otherwise the hand-written
+ * prefill_engine.rs:2308-2334.  rows <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M, at most 64) with attn_dim % 8 == 0 and at
+ * most one 16-column block a CU: one HBM-streaming MFMA kernel with the residual fused; otherwise the hand-written
  * MFMA GEMM with the residual add in its epilogue, in place
  * (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt and a residual kernel).
  * Asynchronous on `stream`.  workspace: split-k partials and arrival counters,

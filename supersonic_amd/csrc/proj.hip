@@ -380,17 +380,17 @@ int skinny_max_m() {
 // rounds, and short rows of W leave a wave too few loads in flight (one
 // MI355X, 8 rows: o_proj 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled;
 // norm + Q/K/V 1024 -> 5120, 320 blocks, 13.0 against 11.4; 2048 -> 9216, 576
-// blocks, 20.0 against 12.0; 4096 -> 10240, 640 blocks, 23.2 against 19.7).
+// blocks, 20.0 against 12.0; 4096 -> 10240, 640 blocks, 23.2 against 19.7).  So
+// too with the QK norm and RoPE in the streaming kernel's epilogue, which the
+// tiled GEMM leaves to a kernel of their own (1 / 8 / 12 rows: 4096 -> 10240
+// 25.7 / 27.6 / 35.5 against 24.3 / 25.4 / 26.0; 2048 -> 9216 21.4 / 23.0 / 24.1
+// against 17.4 / 18.2 / 18.3; 1024 -> 5120 15.7 / 16.5 / 17.7 against 14.7 /
+// 14.6 / 15.1).
 // A row limit or a GEMM in the environment asks for the streaming kernels.
 bool stream_columns(int dev, int64_t ncb) {
     const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
     return ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM");
 }
-// ... and with the QK norm and RoPE in the epilogue, which the tiled GEMM leaves
-// to a kernel of their own: also with long rows (8 rows, 4096 -> 10240: 27.6 us
-// against 27.7 tiled, 1 row 25.9 against 27.9; 2048 -> 9216: 22.6 against 17.0;
-// 1024 -> 5120: 16.5 against 14.8).
-bool stream_rope_columns(int dev, int64_t ncb, int k) { return k >= 4096 || stream_columns(dev, ncb); }
 
 bool skinny_fits(int m, int k, const void* x, const void* w) {
     return m >= 1 && m <= skinny_max_m() && k % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
@@ -1045,7 +1045,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     const size_t pws_bytes = ws + need > pws ? static_cast<size_t>(ws + need - pws) : 0;
     const int ncb = (nq + 2 * nkv) / kSkinnyCols;
     const bool fused = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
-                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4) && stream_rope_columns(dev, ncb, k);
+                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4) && stream_columns(dev, ncb);
     const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
                         nkv % kSkinnyCols == 0 && stream_columns(dev, ncb);
     const int ns[3] = {nq, nkv, nkv};
