@@ -456,7 +456,7 @@ def test_qkv_proj_mid_rows(rows, hid, nq, nkv):
 
 
 # Few rows and more column blocks than CUs: the tiled GEMM, then the norm and RoPE kernel.
-@pytest.mark.parametrize("rows,hid,Hq,Hkv", [(1, 1024, 8, 2), (12, 2048, 16, 2)])
+@pytest.mark.parametrize("rows,hid,Hq,Hkv", [(1, 1024, 8, 2), (12, 2048, 16, 2), (12, 4096, 16, 4)])
 def test_qkv_proj_rope_many_columns(rows, hid, Hq, Hkv):
     test_qkv_proj_rope_matches_oracle(rows, hid, Hq, Hkv, 256, 64, True)
 
