@@ -544,7 +544,7 @@ class Workloads:
         ach = o_flops / (res["oproj_ms"] * 1e-3) / 1e12
         res["roofline"] = {"bound": "mfma", "achieved": round(ach, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                            "frac": round(ach / BF16_PEAK_TFLOPS, 4), "traffic": measured_traffic("gemm_oproj"),
-                           "kernel": "gemm_bt_kernel (o_proj + residual epilogue)"}
+                           "kernel": "gemm_tile_kernel (256 x 128, o_proj + residual epilogue)"}
         return res
 
     def qkv(self):
