@@ -1,5 +1,6 @@
-// bf16 GEMM out = a . w^T for the prefill-sized projections (rows > the
-// weight-streaming limit): the reference's matmul_rhs_transposed_tiled
+// bf16 GEMM out = a . w^T for the prefill-sized projections: the plan of every
+// tiled product (gemm_plan) and its 256 x 256 kernel; the smaller tiles are
+// gemm_tile.hip's.  The reference's matmul_rhs_transposed_tiled
 // (kernels/full_attention_4b.hip:2513-2575) and the hipBLASLt calls the
 // projection entry points used before, as one MFMA kernel for gfx950.
 //
