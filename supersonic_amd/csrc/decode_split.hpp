@@ -8,6 +8,7 @@
 
 #include "common.hpp"
 #include "kv_view.hpp"
+#include "ragged_plan.hpp"
 
 namespace ssa {
 
@@ -179,9 +180,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& p, int vbx
     int split, kvh, b, chunk, n_b, len;
     int64_t pre_b;
     if (p.ragged) {
-        // Every workgroup plans the same way from the lengths: chunk =
-        // ceil(total * Hkv / target) rounded up to 16 (at least min_chunk),
-        // sequence b gets n_b = max(1, ceil(len_b / chunk)) splits per kv
+        // Every workgroup plans the same way from the lengths: the chunk is
+        // ragged_chunk's, sequence b gets n_b = max(1, ceil(len_b / chunk)) splits per kv
         // head, each of them ceil(len_b / n_b) tokens (rounded up to 16), items
         // are ordered (b, kv head, split), and workgroup i takes item i (past
         // the last item it has nothing to do).
@@ -197,36 +197,26 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& p, int vbx
             for (int b0 = 0; b0 < p.B; b0 += 64) tot += len_of(b0 + lane);
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) tot += __shfl_xor(tot, o);
-            // Per-sequence rounding can push the item count past the target
-            // (a second, mostly idle round): grow the chunk in proportion
-            // until the items fit (a few passes; uniform lengths need none).
-            int64_t c = (tot * p.Hkv + p.target - 1) / p.target;
-            c = max((c + 15) / 16 * 16, static_cast<int64_t>(p.min_chunk));
-            bool fits = false;
-            for (int pass = 0; pass < 5; ++pass) {
-                int64_t items = 0;
-                for (int b0 = 0; b0 < p.B; b0 += 64) {
-                    const int bi = b0 + lane;
-                    const int64_t l = len_of(bi);
-                    items += bi < p.B ? max(static_cast<int64_t>(1), (l + c - 1) / c) : 0;
-                }
+            const int ch = ragged_chunk(
+                tot, p.Hkv, p.target, p.min_chunk, p.strict != 0,
+                [&](int64_t c) {
+                    int64_t items = 0;
+                    for (int b0 = 0; b0 < p.B; b0 += 64) {
+                        const int bi = b0 + lane;
+                        const int64_t l = len_of(bi);
+                        items += bi < p.B ? max(static_cast<int64_t>(1), (l + c - 1) / c) : 0;
+                    }
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) items += __shfl_xor(items, o);
-                items *= p.Hkv;
-                fits = items <= p.target;
-                if (fits || pass == 4) break;
-                c = (c * items + p.target - 1) / p.target;
-                c = (c + 15) / 16 * 16;
-            }
-            if (p.strict && !fits) {
-                // four growth steps did not get there: one split per sequence
-                int64_t mx = 0;
-                for (int b0 = 0; b0 < p.B; b0 += 64) mx = max(mx, static_cast<int64_t>(len_of(b0 + lane)));
+                    for (int o = 1; o < 64; o <<= 1) items += __shfl_xor(items, o);
+                    return items * p.Hkv;
+                },
+                [&]() {
+                    int64_t mx = 0;
+                    for (int b0 = 0; b0 < p.B; b0 += 64) mx = max(mx, static_cast<int64_t>(len_of(b0 + lane)));
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) mx = max(mx, __shfl_xor(mx, o));
-                c = max(c, (mx + 15) / 16 * 16);
-            }
-            const int ch = static_cast<int>(c);
+                    for (int o = 1; o < 64; o <<= 1) mx = max(mx, __shfl_xor(mx, o));
+                    return mx;
+                });
             if (lane == 0) plan_s[0] = -1;
             const int w = vbx;
             int run = 0, run_n = 0;  // items and splits of the sequences before b0

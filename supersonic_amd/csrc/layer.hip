@@ -310,15 +310,8 @@ static int launch_layer(int device, hipStream_t st, LayerParams& P) {
     if (P.dec.B == 1 && P.layer_len > 0) {
         // the device plan for one sequence of the expected length
         const int64_t l = P.layer_len, Hkv = P.dec.Hkv;
-        int64_t c = (l * Hkv + grid - 1) / grid;
-        c = std::max((c + 15) / 16 * 16, static_cast<int64_t>(P.dec.min_chunk));
-        for (int pass = 0; pass < 4; ++pass) {
-            const int64_t items = std::max<int64_t>(1, (l + c - 1) / c) * Hkv;
-            if (items <= grid) break;
-            c = (c * items + grid - 1) / grid;
-            c = (c + 15) / 16 * 16;
-        }
-        const int64_t items = std::max<int64_t>(1, (l + c - 1) / c) * Hkv;
+        auto items_of = [&](int64_t c) { return std::max<int64_t>(1, (l + c - 1) / c) * Hkv; };
+        const int64_t items = items_of(ragged_chunk(l, P.dec.Hkv, grid, P.dec.min_chunk, true, items_of, [&]() { return l; }));
         if (2 * items <= grid) P.hint = static_cast<int>(items);
     }
     P.polls = wait_polls(kLayerSpin);
