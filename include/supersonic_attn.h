@@ -407,9 +407,9 @@ int supersonic_attn_gfx950_qkv_proj_rope(
  * (1); weights as supersonic_attn_gfx950_qkv_proj / _o_proj_residual; cache,
  * positions, tables as supersonic_attn_gfx950_decode.  One workgroup per
  * compute unit, three phases separated by device-wide barriers, in an ordinary
- * launch: when other work keeps workgroups of the grid from a compute unit for
- * some 10 ms, the kernel leaves and a lone workgroup launched behind it runs the
- * layer (slowly, same result).  Limits: batch <= 16,
+ * launch: workgroups that other work keeps from a compute unit are not waited
+ * for, those that run take over their parts (two layers may run on two streams,
+ * each with a workspace of its own).  Limits: batch <= 16,
  * batch * hidden_dim <= 32768 and batch * q_heads * head_dim <= 32768,
  * hidden_dim % 16 == 0, head_dim 128/256, q_heads / kv_heads <= 4, 16-byte
  * aligned hidden and weights (otherwise SUPERSONIC_ERR_RANGE: use the

@@ -174,7 +174,9 @@ __device__ __forceinline__ void decode_split_body(const DecodeParams& p, int vbx
     float (&ml_s)[NW][GP][2] = L.ml_s;
     int& next_blk = L.next_blk;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int tid = threadIdx.x;
+    if constexpr (kMid) asm volatile("" : "+v"(tid));  // nothing of it is kept across the caller's other phases
+    const int lane = tid & 63, wave = tid >> 6;
     // Work item (b, kv head, split), chunk length, and the partial rows of
     // sequence b: pre_b splits before it, n_b of its own per head.
     int split, kvh, b, chunk, n_b, len;

@@ -35,7 +35,8 @@ struct LayerParams {
     SkinnyLdsParams qkv;  // phase 1: three segments, NORM staging from the hidden rows
     DecodeParams dec;     // phase 2: fused decode step, ragged plan over the grid
     SkinnyLdsParams op;   // phase 3: attn -> hidden (residual in place)
-    unsigned* bar;        // barrier counters [0..2], flags [32], [48] (another cache line) and [8], zero between calls
+    unsigned* bar;        // barrier counters [0..2] and flags [32], [48] (another cache line), zero between calls
+    unsigned* ids;        // [grid] who has which part (IdState), zero between calls
     int polls;            // bound of a barrier wait (kLayerSpin)
     // > 0: the decode step is expected to have this many work items (one
     // sequence of length max_kv_len); the last `hint` workgroups then take
@@ -46,7 +47,8 @@ struct LayerParams {
 
 constexpr int kLayerThreads = 64 * kSkinnyWaves;  // = 64 * decode_waves(4)
 constexpr int kLayerSpin = 1 << 20;               // bounded barrier wait
-constexpr int kLayerAlonePolls = 1 << 14;         // ... with workgroups missing
+constexpr int kLayerMissingPolls = 64;            // ... after which missing workgroups' parts are taken over (40 us)
+constexpr int kLayerMaxGrid = 1024;               // workspace bound on the grid (partial rows, ids)
 
 // Every value one phase hands to the next is written and read with
 // device-coherent (sc1) accesses, so the barrier needs no cache writeback or
@@ -69,25 +71,46 @@ constexpr int kLayerAlonePolls = 1 << 14;         // ... with workgroups missing
 // per-XCD cache line.  This is what an agent-scope release / acquire pair
 // provides, without the L2 writeback and invalidate those emit.
 //
-// Every workgroup arrives at barrier 0, so once it opens all of them are
-// running and no later wait can depend on one that has no CU.  The launch
-// itself does not promise that.  (A cooperative one does, through a queue of its
-// own: 17-20 us a call on this runtime: 1 sequence of 2048 tokens, 8/2 heads,
-// hidden 1024, 49.2 us a layer, 32.5 with this.)
-// Instead a wait that lasts (kLayerAlonePolls, about 10 ms) while workgroups are
-// missing from barrier 0 may be holding the CU that they need: it then closes
-// the barrier for good (flag 0 -> kFlagAlone, one compare-and-swap against the
-// last arrival's 0 -> kFlagOpen), every workgroup leaves, also those that
-// start later, and decode_layer_alone_kernel behind runs the layer.  That is
-// sound at any time before barrier 0 opens: no item is past its grid wait, so
-// the hidden rows and the cache are untouched.
-// With every workgroup arrived, a wait can only expire on a workspace whose
-// counters were not zero: it then sets kWaitLayerBarrier in the error word and
-// carries on, so that the kernel still exits.
-enum : unsigned { kFlagOpen = 1u, kFlagAlone = 2u };
-enum LayerWait { kLayerGo, kLayerLeave };
-constexpr int kLayerAloneWord = 8;  // in LayerParams::bar: the layer is left to decode_layer_alone_kernel
+// The launch does not promise that every workgroup of the grid is running, and
+// no wait depends on one that is not.  (A cooperative launch does promise it,
+// through a queue of its own: 17-20 us a call on this runtime.)  The layer's
+// work comes in one part an id, 0 .. grid - 1: the column blocks, decode item
+// and output columns above.  A workgroup takes the id of its index as it
+// starts, with an atomic whose round trip runs beside the weight stream and
+// whose result is needed before the first store.  Where a wait lasts
+// (kLayerMissingPolls) while arrivals are missing from barrier 0, the waiting
+// workgroup takes an id that no workgroup has started yet, runs its part of
+// phase 1, arrives for it, and later runs its decode item and output columns
+// behind its own.  A workgroup that finds its id taken leaves.  So whatever
+// the number of workgroups that find a CU (two layers on two streams hold a
+// part of the CUs each), those that did go on: every id is in the hands of a
+// running workgroup before barrier 0 opens, and decode items never wait for
+// each other.  1 sequence of 2048 tokens, 8/2 heads, hidden 1024: 48.8 us a
+// layer with the cooperative launch, 32.5 with an ordinary one and a kernel
+// behind it for the case that workgroups are missing, 29.4 with this (29.3
+// without any of it); such layers on two streams 39.4 us each with
+// the cooperative launch, 17.9 with this.
+// A wait only expires on a workspace whose counters were not zero: it then sets
+// kWaitLayerBarrier in the error word and carries on, so that the kernel still
+// exits.
+enum IdState : unsigned { kIdFree = 0u, kIdTaken = 1u, kIdProjected = 2u };  // projected: phase 1 done
+enum LayerWait { kLayerGo, kLayerMissing };
 constexpr int kArriveThread = kLayerThreads - 64;
+struct LayerShared {
+    int mine;                        // this workgroup got the id it is working on
+    int res;                         // grid_wait's and take_over's result
+    int first, unfinished;           // take_over's scan
+    uint16_t taken[kLayerMaxGrid];   // [1 ..]: ids taken over
+};
+// Whether this workgroup has its id, known by the time the outputs go out.
+struct OwnId {
+    unsigned before;  // the id's state before it was taken (kArriveThread)
+    int& mine;
+    __device__ void park() const {
+        if (threadIdx.x == kArriveThread) mine = before == kIdFree;
+    }
+    __device__ bool open() const { return __builtin_amdgcn_readfirstlane(mine) != 0; }
+};
 // This workgroup's coherent stores are complete, for all of its threads.
 __device__ __forceinline__ void stores_complete() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -95,162 +118,225 @@ __device__ __forceinline__ void stores_complete() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
 }
+// Counts one id in; stores_complete() comes first.
 __device__ __forceinline__ void grid_arrive(unsigned* ctr, unsigned* flag, unsigned n) {
-    stores_complete();
     if (threadIdx.x == kArriveThread) {
         const unsigned prev = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == n - 1) atomicCAS(flag, 0u, static_cast<unsigned>(kFlagOpen));
+        if (prev == n - 1) __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
-// Waits for `flag` (bar + 32: barrier 0's, bar + 48: barrier 1's).
-__device__ __forceinline__ LayerWait grid_wait(unsigned* bar, unsigned* flag, unsigned nwg, int polls, int& res) {
+// Waits for barrier `which` (0 or 1).  kLayerMissing: it lasted while arrivals
+// were missing from barrier 0.  spent: polls of the waits that ended so, in all.
+__device__ __forceinline__ LayerWait grid_wait(const LayerParams& P, int which, unsigned nwg, int& spent,
+                                               LayerShared& sh) {
     if (threadIdx.x == 0) {
-        const int alone_polls = min(polls, kLayerAlonePolls);
-        LayerWait r = kLayerGo;
+        unsigned* const ctr = P.bar + which;
+        unsigned* const flag = P.bar + 32 + 16 * which;
+        const int patience = spent ? 8 : min(P.polls, kLayerMissingPolls);
+        auto missing = [&](unsigned* c) { return static_cast<int>(load_agent_u32(c)) < static_cast<int>(nwg); };
+        // a wait expires after P.polls polls once every arrival has been counted
+        // for kLayerMissingPolls of them (the flag follows the count)
+        int r = 0, late = 0;
         for (int it = 0;; ++it) {
-            if (load_agent_u32(flag) == kFlagOpen) break;
-            if ((it & 63) == 63 || it >= alone_polls) {
-                const unsigned f0 = load_agent_u32(bar + 32);
-                if (f0 == kFlagAlone) {
-                    r = kLayerLeave;
-                    break;
-                }
-                if (it >= alone_polls && f0 == 0u && static_cast<int>(load_agent_u32(bar)) < static_cast<int>(nwg)) {
-                    atomicCAS(bar + 32, 0u, static_cast<unsigned>(kFlagAlone));
-                    continue;  // closed, or opened meanwhile: the next poll sees which
-                }
+            if (load_agent_u32(flag) != 0u) break;
+            if (it >= patience && spent < kLayerSpin && load_agent_u32(P.bar + 32) == 0u && missing(P.bar)) {
+                r = it + 1;
+                break;
             }
-            if (it >= polls) {
+            if (it >= P.polls && !missing(ctr)) ++late;
+            if (late >= kLayerMissingPolls || it >= kLayerSpin || spent >= kLayerSpin) {
                 wait_expired(kWaitLayerBarrier);
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
         }
-        res = r;
+        sh.res = r;
     }
     __syncthreads();
-    // (the next wait writes it after that barrier's arrival, which synchronises)
-    return static_cast<LayerWait>(__builtin_amdgcn_readfirstlane(res));
+    // (the next writer of res is behind another barrier)
+    const int r = __builtin_amdgcn_readfirstlane(sh.res);
+    spent += r;
+    return r ? kLayerMissing : kLayerGo;
+}
+// Takes the next id after w that no workgroup has started; -1: there is none
+// (or another workgroup was faster).  With every id's phase 1 done, barrier 0 opens
+// whatever its counter says.
+__device__ __forceinline__ int take_over(const LayerParams& P, int w, int nwg, LayerShared& sh) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sh.first = nwg;
+        sh.unfinished = 0;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nwg; i += kLayerThreads) {
+        const int v = w + i < nwg ? w + i : w + i - nwg;
+        const unsigned s = load_agent_u32(P.ids + v);
+        if (s == kIdFree) atomicMin(&sh.first, i);
+        if (s != kIdProjected) sh.unfinished = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int v = -1;
+        if (sh.first < nwg) {
+            v = w + sh.first < nwg ? w + sh.first : w + sh.first - nwg;
+            if (atomicCAS(P.ids + v, static_cast<unsigned>(kIdFree), static_cast<unsigned>(kIdTaken)) != kIdFree) v = -1;
+        } else if (!sh.unfinished) {
+            __hip_atomic_store(P.bar + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        sh.res = v;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(sh.res);
+}
+
+// The kernel's arguments, read again where they are asked for: kept in scalar
+// registers around the loops below they spill (259 of them, and 39 vector
+// registers with them; 59 and none so).
+__device__ __forceinline__ const LayerParams& layer_args() {
+    typedef const __attribute__((address_space(4))) LayerParams* Kernarg;
+    uint64_t a = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+    asm volatile("" : "+s"(a));
+    return *(const LayerParams*)reinterpret_cast<Kernarg>(a);
 }
 
 template <typename HT, bool FP8, int D>
-__global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams P) {
+__global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams) {
     static_assert(decode_waves(4) * 64 == kLayerThreads, "one workgroup shape for every phase");
-    __shared__ union Lds {
-        DecodeLds<D, 4> d;
-        SkinnyLds s;
+    // (sh first: LDS below 64 KB is reached with an immediate offset)
+    __shared__ struct {
+        LayerShared sh;
+        union {
+            DecodeLds<D, 4> d;
+            SkinnyLds s;
+        };
     } lds;
-    __shared__ int wait_res;
+    LayerShared& sh = lds.sh;
+    const LayerParams& P = layer_args();
     const int w = blockIdx.x;
     const unsigned nwg = gridDim.x;
     const int ncb_qkv = P.qkv.cb_end[2], ncb_op = P.op.cb_end[2];
     const int nq = static_cast<int>(nwg) - P.hint;
     const int shift = min(max(ncb_qkv - static_cast<int>(nwg), 0), static_cast<int>(nwg));
-    const int item = P.hint > 0 ? (w >= nq ? w - nq : P.hint + w)
-                                : (w - shift + static_cast<int>(nwg)) % static_cast<int>(nwg);
-    // 1. input norm + Q/K/V projections on the first nq workgroups: column
-    // blocks w, w + nq, ...; a workgroup with two left takes them together
-    // (one staging of the rows, both weight streams in flight)
-    for (int cb = w; cb < ncb_qkv && w < nq;) {
-        if (cb + nq < ncb_qkv) {
-            skinny_lds_body<bf16_t, false, false, true, HT, false, true, SkinnyLds, true>(P.qkv, RopeEpi{}, cb, 0,
-                                                                                           lds.s, cb + nq);
-            cb += 2 * nq;
-        } else {
-            skinny_lds_body<bf16_t, false, false, true, HT, false, true>(P.qkv, RopeEpi{}, cb, 0, lds.s);
-            cb += nq;
+    auto item_of = [&](int v) {
+        return P.hint > 0 ? (v >= nq ? v - nq : P.hint + v)
+                          : (v - shift + static_cast<int>(nwg)) % static_cast<int>(nwg);
+    };
+    // Ahead of every load, so that no later wait has to count it.
+    OwnId own{kIdFree, sh.mine};
+    if (threadIdx.x == kArriveThread)
+        own.before = atomicCAS(P.ids + w, static_cast<unsigned>(kIdFree), static_cast<unsigned>(kIdTaken));
+    int n_ids = 1, n_items = 0;      // ids of this workgroup, and those whose decode item is done
+    bool has_op = w < ncb_op;
+    int spent = 0;
+    for (int v = w;;) {
+        const LayerParams& P = layer_args();
+        if (v >= 0) {
+            // 1. input norm + Q/K/V projections on the first nq ids: column
+            // blocks v, v + nq, ...; with two left they run together
+            // (one staging of the rows, both weight streams in flight)
+            const SkinnyLdsParams qkv = P.qkv;
+            for (int cb = v; cb < ncb_qkv && v < nq;) {
+                if (cb + nq < ncb_qkv) {
+                    skinny_lds_body<bf16_t, false, false, true, HT, false, true, SkinnyLds, true>(
+                        qkv, RopeEpi{}, cb, 0, lds.s, cb + nq, own);
+                    cb += 2 * nq;
+                } else {
+                    skinny_lds_body<bf16_t, false, false, true, HT, false, true, SkinnyLds, false>(
+                        qkv, RopeEpi{}, cb, 0, lds.s, -1, own);
+                    cb += nq;
+                }
+                __syncthreads();
+            }
+            own.park();
+            stores_complete();
+            if (!own.open()) break;
+            own.before = kIdFree;
+            if (threadIdx.x == kArriveThread)
+                __hip_atomic_store(P.ids + v, static_cast<unsigned>(kIdProjected), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            grid_arrive(&P.bar[0], &P.bar[32], nwg);
         }
-        __syncthreads();
-    }
-    // 2. attention step (every workgroup plans the same ragged split).  The
-    // work items go first to the workgroups that ran one phase-1 task (the
-    // first ncb_qkv - nwg ran two), so the items start with their plan and
-    // first K/V block (the cache does not depend on phase 1) while phase 1
-    // finishes.  The workgroup arrives at barrier 0 first, then plans its item
-    // and fetches its first block, and only then waits; a workgroup without
-    // an item does not wait (only the readers of phase 1's output do).
-    // With a hint the expected items sit on the workgroups without phase-1
-    // work (any further item on the others).
-    grid_arrive(&P.bar[0], &P.bar[32], nwg);
-    LayerWait res = kLayerGo;
-    bool had_item = false;
-    decode_split_body<bf16_t, FP8, D, 4, true>(P.dec, item, 0, 0, lds.d, [&]() {
-        res = grid_wait(P.bar, &P.bar[32], nwg, P.polls, wait_res);
-        had_item = true;
-        return res == kLayerGo;
-    });
-    if (res == kLayerGo) {
-        if (!had_item && w < ncb_op) {
-            // An output-projection workgroup without a decode item copies its
-            // first task's weight rows into an LDS sink while the items run, so
-            // that phase 3 finds them in this XCD's L2.  (The copies complete
-            // before it arrives at barrier 1, which waits for its loads.)
-            const int k = P.op.k;
-            const int bytes = min(kSkinnyCols, P.op.n_seg[0] - w * kSkinnyCols) * k * 2;
-            const __amdgpu_buffer_rsrc_t r =
-                uniform_rsrc(reinterpret_cast<const uint8_t*>(P.op.w[0] + static_cast<int64_t>(w) * kSkinnyCols * k), bytes);
-            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-            for (int off = wave * 1024; off < bytes; off += kSkinnyWaves * 1024)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds.s.xs, 16,
-                                                         off + lane * 16, 0, 0, 0);
+        // 2. attention step (every workgroup plans the same ragged split).  The
+        // work items go first to the ids with one phase-1 task (the
+        // first ncb_qkv - nwg have two), so the items start with their plan and
+        // first K/V block (the cache does not depend on phase 1) while phase 1
+        // finishes.  The workgroup arrives at barrier 0 first, then plans its item
+        // and fetches its first block, and only then waits; without
+        // an item it does not wait (only the readers of phase 1's output do).
+        // With a hint the expected items sit on the ids without phase-1
+        // work (any further item on the others).
+        LayerWait res = kLayerGo;
+        for (; n_items < n_ids; ++n_items) {
+            const LayerParams& P = layer_args();
+            const int u = n_items == 0 ? w : __builtin_amdgcn_readfirstlane(sh.taken[n_items]);
+            const DecodeParams dec = P.dec;
+            bool had_item = false;
+            decode_split_body<bf16_t, FP8, D, 4, true>(dec, item_of(u), 0, 0, lds.d, [&]() {
+                res = grid_wait(P, 0, nwg, spent, sh);
+                had_item = true;
+                return res == kLayerGo;
+            });
+            // (the body's way out depends on its plan, in LDS: say that it is one for all lanes)
+            res = static_cast<LayerWait>(__builtin_amdgcn_readfirstlane(res));
+            had_item = __builtin_amdgcn_readfirstlane(had_item) != 0;
+            if (res != kLayerGo) break;
+            if (!had_item && u < ncb_op) {
+                // An output-projection workgroup without a decode item copies its
+                // first task's weight rows into an LDS sink while the items run, so
+                // that phase 3 finds them in this XCD's L2.  (The copies complete
+                // before it arrives at barrier 1, which waits for its loads.)
+                const int k = P.op.k;
+                const int bytes = min(kSkinnyCols, P.op.n_seg[0] - u * kSkinnyCols) * k * 2;
+                const __amdgpu_buffer_rsrc_t r =
+                    uniform_rsrc(reinterpret_cast<const uint8_t*>(P.op.w[0] + static_cast<int64_t>(u) * kSkinnyCols * k), bytes);
+                const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+                for (int off = wave * 1024; off < bytes; off += kSkinnyWaves * 1024)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds.s.xs, 16,
+                                                             off + lane * 16, 0, 0, 0);
+            }
+            // Barrier 1: every id arrives; the workgroups with an
+            // output-projection task wait for all of them.
+            stores_complete();
+            grid_arrive(&P.bar[1], &P.bar[48], nwg);
         }
-        // Barrier 1: every workgroup arrives; those with an output-projection
-        // task wait for all of them.
-        grid_arrive(&P.bar[1], &P.bar[48], nwg);
-        if (w < ncb_op) res = grid_wait(P.bar, &P.bar[48], nwg, P.polls, wait_res);
+        if (res == kLayerGo && has_op) res = grid_wait(P, 1, nwg, spent, sh);
+        if (res == kLayerGo) {
+            // 3. output projection + residual
+            for (int i = 0; i < n_ids; ++i) {
+                const int u = i == 0 ? w : __builtin_amdgcn_readfirstlane(sh.taken[i]);
+                for (int cb = u; cb < ncb_op; cb += nwg) {
+                    const SkinnyLdsParams op = layer_args().op;
+                    skinny_lds_body<HT, true, false, false, bf16_t, true, false>(op, RopeEpi{}, cb, 0, lds.s);
+                    __syncthreads();
+                }
+            }
+            break;
+        }
+        v = take_over(P, w, static_cast<int>(nwg), sh);
+        if (v >= 0) {
+            if (threadIdx.x == 0) sh.taken[n_ids] = static_cast<uint16_t>(v);  // (read behind stores_complete)
+            ++n_ids;
+            has_op |= v < ncb_op;
+        }
     }
-    // 3. output projection + residual
-    for (int cb = w; cb < ncb_op && res == kLayerGo; cb += nwg) {
-        skinny_lds_body<HT, true, false, false, bf16_t, true, false>(P.op, RopeEpi{}, cb, 0, lds.s);
-        __syncthreads();
-    }
-    // The last workgroup to finish resets every counter and flag: each
+    // The last workgroup to finish resets every counter, flag and id: each
     // workgroup counts itself in here after its last arrival and its last
     // poll, so nothing reads or bumps them any more in this call, whether or
     // not a wait gave up.
-    if (threadIdx.x == 0) {
-        const unsigned prev = __hip_atomic_fetch_add(&P.bar[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == nwg - 1) {
-            // (a closed barrier 0 leaves the layer to decode_layer_alone_kernel)
-            if (load_agent_u32(&P.bar[32]) == kFlagAlone)
-                __hip_atomic_store(&P.bar[kLayerAloneWord], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&P.bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&P.bar[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&P.bar[32], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&P.bar[48], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&P.bar[2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < 64) {
+        unsigned prev = 0;
+        if (threadIdx.x == 0) prev = __hip_atomic_fetch_add(&P.bar[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(prev) == nwg - 1) {
+            auto zero = [](unsigned* p) { __hip_atomic_store(p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+            if (threadIdx.x == 0) {
+                zero(&P.bar[0]);
+                zero(&P.bar[1]);
+                zero(&P.bar[32]);
+                zero(&P.bar[48]);
+                zero(&P.bar[2]);
+            }
+            for (int i = threadIdx.x; i < static_cast<int>(nwg); i += 64) zero(P.ids + i);
         }
     }
-}
-
-// The whole layer on one workgroup, after a decode_layer_kernel whose barrier 0
-// was closed (grid_wait); otherwise it only looks and leaves, which costs a
-// call 2-3 us.
-template <typename HT, bool FP8, int D>
-__global__ __launch_bounds__(kLayerThreads) void decode_layer_alone_kernel(LayerParams P) {
-    __shared__ union Lds {
-        DecodeLds<D, 4> d;
-        SkinnyLds s;
-    } lds;
-    if (load_agent_u32(&P.bar[kLayerAloneWord]) == 0u) return;
-    for (int cb = 0; cb < P.qkv.cb_end[2]; ++cb) {
-        skinny_lds_body<bf16_t, false, false, true, HT, false, true>(P.qkv, RopeEpi{}, cb, 0, lds.s);
-        __syncthreads();
-    }
-    stores_complete();
-    DecodeParams dec = P.dec;
-    dec.target = 1;  // one split a sequence and kv head
-    for (int i = 0; i < dec.B * dec.Hkv; ++i) {
-        decode_split_body<bf16_t, FP8, D, 4, true>(dec, i, 0, 0, lds.d);
-        __syncthreads();
-    }
-    stores_complete();
-    for (int cb = 0; cb < P.op.cb_end[2]; ++cb) {
-        skinny_lds_body<HT, true, false, false, bf16_t, true, false>(P.op, RopeEpi{}, cb, 0, lds.s);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        __hip_atomic_store(&P.bar[kLayerAloneWord], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Workgroups of one layer-kernel instance resident at once, per device.
@@ -271,14 +357,13 @@ static int layer_grid(int device) {
     return cap[device];
 }
 
-constexpr int kLayerMaxGrid = 1024;           // workspace bound on the grid (partial rows)
 constexpr size_t kLayerBarBytes = 256;
 constexpr size_t kLayerArrivalBytes = 64 << 10;
 
 inline size_t al256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 struct LayerWs {
-    size_t bar, arrivals, part_o, part_ml, q_proj, k_new, v_new, attn, total;
+    size_t bar, ids, arrivals, part_o, part_ml, q_proj, k_new, v_new, attn, total;
 };
 
 inline LayerWs layer_ws(int B, int Hq, int Hkv, int D, int max_len) {
@@ -287,7 +372,8 @@ inline LayerWs layer_ws(int B, int Hq, int Hkv, int D, int max_len) {
     const size_t rows = (static_cast<size_t>((kLayerMaxGrid + Hkv - 1) / Hkv) + B) * Hq;
     LayerWs w{};
     w.bar = 0;
-    w.arrivals = kLayerBarBytes;
+    w.ids = kLayerBarBytes;
+    w.arrivals = w.ids + kLayerMaxGrid * sizeof(unsigned);
     w.part_o = w.arrivals + kLayerArrivalBytes;
     w.part_ml = w.part_o + al256(rows * D * 4);
     w.q_proj = w.part_ml + al256(rows * 2 * 4);
@@ -317,7 +403,6 @@ static int launch_layer(int device, hipStream_t st, LayerParams& P) {
     P.polls = wait_polls(kLayerSpin);
     P.dec.merge_polls = wait_polls(kMergePoll);
     hipLaunchKernelGGL((decode_layer_kernel<HT, FP8, D>), dim3(grid), dim3(kLayerThreads), 0, st, P);
-    hipLaunchKernelGGL((decode_layer_alone_kernel<HT, FP8, D>), dim3(1), dim3(kLayerThreads), 0, st, P);
     return hipGetLastError() == hipSuccess ? 0 : SUPERSONIC_ERR_LAUNCH;
 }
 
@@ -378,6 +463,7 @@ extern "C" int supersonic_attn_gfx950_decode_layer(
     uint16_t* v_new = reinterpret_cast<uint16_t*>(ws + L.v_new);
     uint16_t* attn = reinterpret_cast<uint16_t*>(ws + L.attn);
     P.bar = reinterpret_cast<unsigned*>(ws + L.bar);
+    P.ids = reinterpret_cast<unsigned*>(ws + L.ids);
     P.layer_len = static_cast<int>(max_kv_len);
     // phase 1
     SkinnyLdsParams& q = P.qkv;

@@ -4,6 +4,8 @@
 // (layer.hip).
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "kv_view.hpp"
 
@@ -128,11 +130,19 @@ struct SkinnyLds : SkinnyLdsBase {
 // device-coherent accesses (data exchanged with other workgroups of the same
 // kernel).  PAIR (plain store epilogue only): a second column block cb2 (or
 // none when cb2 < 0) shares the staged rows, and both blocks' weight loads are
-// in flight together, so two blocks cost little more than one.
+// in flight together, so two blocks cost little more than one.  gate: park()
+// is called by every thread ahead of the barrier before the outputs, open()
+// behind it (the same for every thread): whether this workgroup stores them.
+struct AlwaysOpen {
+    __device__ void park() const {}
+    __device__ bool open() const { return true; }
+};
 template <typename OT, bool RES, bool ROPE, bool NORM = false, typename XT = bf16_t, bool COH_IN = false,
-          bool COH_OUT = false, typename LdsT = SkinnyLds, bool PAIR = false, int STEPS = kSkinnySteps>
+          bool COH_OUT = false, typename LdsT = SkinnyLds, bool PAIR = false, int STEPS = kSkinnySteps,
+          typename Gate = AlwaysOpen>
 __device__ __forceinline__ void skinny_lds_body(const SkinnyLdsParams& p, const RopeEpi& e, int cb, int b,
-                                                LdsT& L, int cb2 = -1) {
+                                                LdsT& L, int cb2 = -1, const Gate& gate = Gate()) {
+    static_assert(!ROPE || std::is_same<Gate, AlwaysOpen>::value, "the gate covers the plain epilogue");
     static_assert(!PAIR || (!RES && !ROPE), "pairs take the plain store epilogue");
     uint16_t (&xs)[kXsMax + 16 * 8] = L.xs;
     float (&red)[kSkinnyWaves][256] = L.red;
@@ -290,8 +300,10 @@ __device__ __forceinline__ void skinny_lds_body(const SkinnyLdsParams& p, const 
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[wave][(4 * (lane >> 4) + i) * 16 + col] = acc[i];
+    gate.park();
     __syncthreads();
     if constexpr (!ROPE) {
+        if (!gate.open()) return;
         if (tid < 256) {
             const int row = tid >> 4, c = cbs * 16 + (tid & 15);
             if (row < m && c < n) {

@@ -205,9 +205,9 @@ def test_decode_layer_expired_barrier_is_reported(monkeypatch):
 
 @pytest.mark.parametrize("name", ["config1", "config2_b4_ragged", "one_sequence_fp8_paged", "f32_hidden"])
 def test_decode_layer_missing_workgroups_run_alone(name, monkeypatch):
-    """The host presets barrier 0's counter below zero, as if workgroups had found no CU, and shortens the wait: the
-    barrier is closed, the lone workgroup behind the kernel runs the layer, and the result is right, nothing is
-    reported and the counters are back at zero for the next, ordinary call."""
+    """The host presets barrier 0's counter below zero, as if workgroups had found no CU, and shortens the wait: those
+    that run take over what no workgroup has started, open the barrier once every part is projected, and the result is
+    right, nothing is reported and the counters are back at zero for the next, ordinary call."""
     kw = CASES[name]
     announce(f"persistent decode layer, workgroups missing: {name}")
     for held in (True, False):
@@ -224,3 +224,61 @@ def test_decode_layer_missing_workgroups_run_alone(name, monkeypatch):
         ref, v_ref = oracle_layer(c)
         check_layer(c, out, cache, ref, v_ref)
         assert int(ws[:256].count_nonzero()) == 0, "barrier words not reset"
+
+
+# (sequence, kv head) pairs and round lengths, so that the taken-over parts hold whole items of every kind
+BESIDE = {
+    "config1": CASES["config1"],
+    "8x4": dict(B=8, Hq=16, Hkv=4, D=256, rot=64, hid=4096, lens=[2048] * 8),
+    "16x4": dict(B=16, Hq=8, Hkv=4, D=256, rot=64, hid=2048, lens=[1024] * 16),
+    "16x4_ragged_fp8_paged": dict(B=16, Hq=8, Hkv=4, D=256, rot=64, hid=1024, fp8=True, page=64,
+                                  lens=[(137 * i * i) % 1900 for i in range(16)]),
+    "d128": CASES["d128"],
+}
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("name", list(BESIDE))
+def test_decode_layer_beside_other_work(name, layers, monkeypatch):
+    """One layer, or one on each of two streams, that do not find every compute unit free: a decode of a long sequence
+    holds 64 of them for some 100 us at a time.  The workgroups that run take over the parts of those that do not."""
+    kw = BESIDE[name]
+    announce(f"persistent decode layer beside other work: {name}, {layers} layers")
+    c = layer_case(136, **kw)
+    ref, v_ref = oracle_layer(c)
+    size = K.decode_layer_workspace_size(c["B"], c["hid"], c["Hq"], c["Hkv"], c["D"], max(c["lens"]) + 1)
+    runs = []
+    for _ in range(layers):
+        if c["page"]:
+            k, v, ks, vs, c["bt"] = paged(c)
+            cache = K.KvCache(dev(k), dev(v), dev(ks), dev(vs), block_table=c["bt"].to(DEV))
+        else:
+            cache = K.KvCache(dev(c["k"]), dev(c["v"]), dev(c["ks"]), dev(c["vs"]))
+        runs.append((c["hidden"].to(c["hidden_dtype"]).to(DEV), cache,
+                     torch.zeros(size, dtype=torch.uint8, device=DEV), torch.cuda.Stream()))
+    w = [dev(c[k]) for k in ("nw", "wq", "wk", "wv", "qw", "kw", "wo", "cos", "sin")]
+    pos = torch.tensor(c["lens"], dtype=torch.int32, device=DEV)
+    long = 65536  # 4 kv heads of 256: 4 MB for each of 64 workgroups
+    lk = torch.zeros(1, 4, long, 256, dtype=torch.bfloat16, device=DEV)
+    lq, lkv = torch.zeros(1, 16 * 512, dtype=torch.bfloat16, device=DEV), torch.zeros(1, 1024, dtype=torch.bfloat16, device=DEV)
+    lout, lnw = torch.zeros(1, 4096, dtype=torch.bfloat16, device=DEV), torch.zeros(256, dtype=torch.bfloat16, device=DEV)
+    lpos = torch.tensor([long - 1], dtype=torch.int32, device=DEV)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for it in range(4):
+        for h, _, _, _ in runs:
+            h.copy_(c["hidden"])
+        torch.cuda.synchronize()
+        monkeypatch.setenv("SUPERSONIC_DECODE_TARGET_WGS", "64")
+        for _ in range(4):
+            K.fused_decode(0, lq, lkv, lkv, lnw, lnw, None, None, lpos, K.KvCache(lk, lk), lout, q_heads=16, kv_heads=4,
+                           head_dim=256, rotary_dim=0, max_kv_len=long, stream=side.cuda_stream)
+        monkeypatch.delenv("SUPERSONIC_DECODE_TARGET_WGS")
+        for h, cache, ws, st in runs:
+            K.decode_layer(0, h, *w, pos, cache, ws, q_heads=c["Hq"], kv_heads=c["Hkv"], head_dim=c["D"],
+                           rotary_dim=c["rot"], max_kv_len=max(c["lens"]) + 1, stream=st.cuda_stream)
+        torch.cuda.synchronize()
+        assert K.wait_status() == 0
+        for h, cache, ws, _ in runs:
+            check_layer(c, h.float().cpu(), cache, ref, v_ref)
+            assert int(ws[:256 + 4 * 1024].count_nonzero()) == 0, "barrier words or ids not reset"
