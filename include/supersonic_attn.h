@@ -297,7 +297,9 @@ int supersonic_attn_gfx950_prefill(
  * share one block-paged cache (different sequences).  workspace: NULL
  * (library-owned) or caller device memory of at least
  * supersonic_attn_gfx950_mixed_workspace_size() bytes, zero-filled before its
- * first use and not written between calls.  Calls sharing the library
+ * first use and not written between calls (without the room for the chunk's key
+ * split, which shorter chunks ask for and longer ones do not, the chunk runs
+ * unsplit).  Calls sharing the library
  * stream of a device must not overlap.  The library stream and its two events
  * are created by the first CU-split call on a device: make that call outside
  * stream capture (later calls can be captured with a caller workspace). */

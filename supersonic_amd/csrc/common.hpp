@@ -385,6 +385,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
                    const void* k_norm_w, const void* cos_table, const void* sin_table,
                    const supersonic_kv_cache* cache, void* out, void* workspace, size_t workspace_bytes,
                    unsigned* claims, int free_wgs = 0);
+size_t prefill_stage_bytes(int kv_dtype, size_t kv_heads, size_t head_dim, size_t chunk_len, size_t chunk_start);
 constexpr size_t kClaimBytes = 16 * 128;
 
 // Row repack with cast and zero padding (elementwise.hip): dst row

@@ -125,15 +125,18 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
     void* pws = nullptr;
     size_t dbytes = 0, pbytes = 0;
     if (workspace) {
-        const size_t need =
-            supersonic_attn_gfx950_mixed_workspace_size(kv_dtype, q_heads, kv_heads, head_dim, chunk, decode);
-        if (workspace_bytes < need) return SUPERSONIC_ERR_WORKSPACE;
+        if (has_d)
+            dbytes = align256(supersonic_attn_gfx950_decode_workspace_size(decode->batch, q_heads, kv_heads,
+                                                                           head_dim, decode->max_kv_len));
+        // The chunk needs its staging; room for a key split's sums is what is
+        // left behind it, and a chunk without that runs unsplit.
+        const size_t stage =
+            has_c ? align256(prefill_stage_bytes(kv_dtype, kv_heads, head_dim, chunk->chunk_len, chunk->chunk_start)) : 0;
+        if (workspace_bytes < kClaimBytes + dbytes + stage) return SUPERSONIC_ERR_WORKSPACE;
         uint8_t* w = static_cast<uint8_t*>(workspace);
         claims = reinterpret_cast<unsigned*>(w);
         size_t o = kClaimBytes;
         if (has_d) {
-            dbytes = align256(supersonic_attn_gfx950_decode_workspace_size(decode->batch, q_heads, kv_heads,
-                                                                           head_dim, decode->max_kv_len));
             dws = w + o;
             o += dbytes;
         }

@@ -1471,15 +1471,21 @@ extern "C" int supersonic_qwen35_4b_hip_full_attention_prefill(
                           num_kv_groups, scale, seqlen_offset, query, key, value, out);
 }
 
+// The part of a prefill workspace that a call cannot do without: the V^T
+// staging, and the bf16 K rows of an fp8 cache.
+size_t ssa::prefill_stage_bytes(int kv_dtype, size_t kv_heads, size_t head_dim, size_t chunk_len, size_t chunk_start) {
+    const size_t L = chunk_start + chunk_len;
+    if (L > 0x7FFFFFFF || kv_heads > 4096 || head_dim > 512) return 0;
+    const size_t stage = kv_heads * head_dim * ((L + 63) / 64 * 64) * 2;
+    return kv_dtype == SUPERSONIC_KV_FP8_E4M3 ? 2 * stage : stage;
+}
+
 extern "C" size_t supersonic_attn_gfx950_prefill_workspace_size(int kv_dtype, size_t kv_heads, size_t head_dim,
                                                                 size_t chunk_len, size_t chunk_start) {
     const size_t L = chunk_start + chunk_len;
-    if (L > 0x7FFFFFFF || kv_heads > 4096 || head_dim > 512) return 0;
-    const size_t ld = (L + 63) / 64 * 64;
-    const size_t stage = kv_heads * head_dim * ld * 2;  // V^T staging
-    const size_t stages = kv_dtype == SUPERSONIC_KV_FP8_E4M3 ? 2 * stage : stage;  // + the bf16 K rows of an fp8 cache
+    const size_t stages = prefill_stage_bytes(kv_dtype, kv_heads, head_dim, chunk_len, chunk_start);
     // + a key split's sums
-    return stages + (prefill_may_split(chunk_len, L, kv_heads) ? prefill_part_bytes(static_cast<int>(head_dim), 256) : 0);
+    return stages + (stages && prefill_may_split(chunk_len, L, kv_heads) ? prefill_part_bytes(static_cast<int>(head_dim), 256) : 0);
 }
 
 namespace ssa {

@@ -185,3 +185,40 @@ def test_mixed_key_split_chunk(S, start, batch, Hq, Hkv, own_ws):
         check(chunk["out"], ref_c.float().cpu(), TOL_BF16, "mixed split chunk")
         check(dec["out"], ref_d.float().cpu(), TOL_BF16, "mixed split decode")
     assert torch.equal(c1.k, c2.k) and torch.equal(c1.v, c2.v) and torch.equal(d1.k, d2.k) and torch.equal(d1.v, d2.v)
+
+
+def test_mixed_workspace_of_a_larger_chunk():
+    """A workspace sized for a long chunk, which has no key split, takes a short chunk behind a prefix with fewer tokens in
+    all: with the key split's sums the short one's size is the larger, but it runs without them."""
+    S, start, batch, Hq, Hkv, D, rot = 60, 1000, 3, 8, 2, 256, 64
+    announce("mixed step in a workspace sized for a larger chunk")
+    g = torch.Generator(device=DEV).manual_seed(92)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, start + S + 1, 1.0e7))
+    qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
+    lens = [100, 7, 350]
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    kc, vc = rnd(1, Hkv, start + S, D), rnd(1, Hkv, start + S, D)
+    kd, vd = rnd(batch, Hkv, max(lens) + 1, D), rnd(batch, Hkv, max(lens) + 1, D)
+    xc = [rnd(S, Hq * 2 * D), rnd(S, Hkv * D), rnd(S, Hkv * D)]
+    xd = [rnd(batch, Hq * 2 * D), rnd(batch, Hkv * D), rnd(batch, Hkv * D)]
+    shape = dict(q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot)
+    nan = lambda n: torch.full((n, Hq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ref_c, ref_d = nan(S), nan(batch)
+    K.fused_prefill(0, *xc, qw, kw, cos, sin, K.KvCache(kc.clone(), vc.clone()), ref_c, chunk_start=start, **shape)
+    K.fused_decode(0, *xd, qw, kw, cos, sin, pos, K.KvCache(kd.clone(), vd.clone()), ref_d, max_kv_len=max(lens) + 1, **shape)
+    chunk = dict(zip(("q_proj", "k_new", "v_new"), xc), cache=K.KvCache(kc.clone(), vc.clone()), out=nan(S), chunk_start=start)
+    dec = dict(zip(("q_proj", "k_new", "v_new"), xd), cache=K.KvCache(kd.clone(), vd.clone()), out=nan(batch),
+               positions=pos, max_kv_len=max(lens) + 1)
+    long = dict(chunk, q_proj=torch.empty(4200, 1, dtype=torch.bfloat16), chunk_start=0)  # 4200 rows of 2 kv heads: never split
+    size = K.mixed_workspace_size(False, Hq, Hkv, D, long, dec)
+    assert size < K.mixed_workspace_size(False, Hq, Hkv, D, chunk, dec)
+    K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, decode=dec,
+                  workspace=torch.zeros(size, dtype=torch.uint8, device=DEV), **shape)
+    torch.cuda.synchronize()
+    check(chunk["out"], ref_c.float().cpu(), TOL_BF16, "mixed chunk, small workspace")
+    check(dec["out"], ref_d.float().cpu(), TOL_BF16, "mixed decode, small workspace")
+    # less than the staging is still refused
+    with pytest.raises(K.GpuError):
+        K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, decode=dec,
+                      workspace=torch.zeros(1 << 19, dtype=torch.uint8, device=DEV), **shape)
