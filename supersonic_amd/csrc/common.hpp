@@ -387,6 +387,7 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
                    unsigned* claims, int free_wgs = 0);
 size_t prefill_stage_bytes(int kv_dtype, size_t kv_heads, size_t head_dim, size_t chunk_len, size_t chunk_start);
 constexpr size_t kClaimBytes = 16 * 128;
+constexpr size_t kDecodeArrivalBytes = 64 * 1024;  // a decode workspace's counters, zero between calls, at its start
 
 // Row repack with cast and zero padding (elementwise.hip): dst row
 // (o, i) of dout elements = src[o * so + i * si + 0 .. din) cast from dtype

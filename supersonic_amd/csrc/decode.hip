@@ -115,7 +115,7 @@ static size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255);
 // counters sit at a fixed offset so they never overlap partials of a call
 // with another shape; they are zero before the first call (a fresh library
 // workspace is zero-filled) and every call leaves them zero.
-constexpr size_t kArrivalBytes = 64 * 1024;
+constexpr size_t kArrivalBytes = kDecodeArrivalBytes;
 constexpr int kMaxArrivals = static_cast<int>(kArrivalBytes / sizeof(unsigned));
 
 static size_t workspace_bytes_for(size_t rows, int D) {

@@ -102,6 +102,8 @@ extern "C" size_t supersonic_attn_gfx950_mixed_workspace_size(int kv_dtype, size
     if (decode && decode->batch)
         n += align256(supersonic_attn_gfx950_decode_workspace_size(decode->batch, q_heads, kv_heads, head_dim,
                                                                    decode->max_kv_len));
+    else
+        n += kDecodeArrivalBytes;
     if (chunk && chunk->chunk_len)
         n += align256(supersonic_attn_gfx950_prefill_workspace_size(kv_dtype, kv_heads, head_dim, chunk->chunk_len,
                                                                     chunk->chunk_start));
@@ -119,7 +121,7 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
     const bool has_c = chunk && chunk->chunk_len > 0;
     const bool has_d = decode && decode->batch > 0;
     const int dev = static_cast<int>(device_ordinal);
-    // Workspace: [claim counters][decode][prefill], or the library's buffers.
+    // Workspace: [claim counters][decode, its arrival counters first][prefill], or the library's buffers.
     unsigned* claims = nullptr;
     void* dws = nullptr;
     void* pws = nullptr;
@@ -139,6 +141,9 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
         if (has_d) {
             dws = w + o;
             o += dbytes;
+        } else if (workspace_bytes >= o + kDecodeArrivalBytes + stage) {
+            // a step without decodes leaves the counters of the steps with them alone
+            o += kDecodeArrivalBytes;
         }
         if (has_c) {
             pws = w + o;

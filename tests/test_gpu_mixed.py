@@ -222,3 +222,34 @@ def test_mixed_workspace_of_a_larger_chunk():
     with pytest.raises(K.GpuError):
         K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, decode=dec,
                       workspace=torch.zeros(1 << 19, dtype=torch.uint8, device=DEV), **shape)
+
+
+def test_mixed_step_without_decodes_leaves_their_counters():
+    """One workspace for a step with a chunk only (its staging holds NaNs) and then steps with decodes, whose splits count
+    their arrivals in it."""
+    S, batch, Hq, Hkv, D, rot = 300, 2, 8, 2, 256, 64
+    announce("mixed step without decodes, then with them, one workspace")
+    g = torch.Generator(device=DEV).manual_seed(93)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, 4001, 1.0e7))
+    qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
+    lens = [4000, 1500]
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    kd, vd = rnd(batch, Hkv, max(lens) + 1, D), rnd(batch, Hkv, max(lens) + 1, D)
+    xc = [rnd(S, Hq * 2 * D), rnd(S, Hkv * D), torch.full((S, Hkv * D), float("nan"), dtype=torch.bfloat16, device=DEV)]
+    xd = [rnd(batch, Hq * 2 * D), rnd(batch, Hkv * D), rnd(batch, Hkv * D)]
+    shape = dict(q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot)
+    ref = torch.empty(batch, Hq * D, dtype=torch.bfloat16, device=DEV)
+    K.fused_decode(0, *xd, qw, kw, cos, sin, pos, K.KvCache(kd.clone(), vd.clone()), ref, max_kv_len=max(lens) + 1, **shape)
+    zero = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16, device=DEV)
+    chunk = dict(zip(("q_proj", "k_new", "v_new"), xc), cache=K.KvCache(zero(1, Hkv, S, D), zero(1, Hkv, S, D)),
+                 out=zero(S, Hq * D), chunk_start=0)
+    dec = dict(zip(("q_proj", "k_new", "v_new"), xd), cache=K.KvCache(kd.clone(), vd.clone()), out=zero(batch, Hq * D),
+               positions=pos, max_kv_len=max(lens) + 1)
+    ws = torch.zeros(K.mixed_workspace_size(False, Hq, Hkv, D, chunk, dec), dtype=torch.uint8, device=DEV)
+    K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, workspace=ws, **shape)
+    for part in (dict(chunk=chunk, decode=dec), dict(decode=dec)):
+        dec["out"].fill_(float("nan"))
+        K.fused_mixed(0, qw, kw, cos, sin, workspace=ws, **part, **shape)
+        torch.cuda.synchronize()
+        check(dec["out"], ref.float().cpu(), TOL_BF16, "decodes after a step without them")
