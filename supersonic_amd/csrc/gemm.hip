@@ -1,6 +1,6 @@
-// bf16 GEMM out = a . w^T for the prefill-sized projections: the plan of every
-// tiled product (gemm_plan) and its 256 x 256 kernel; the smaller tiles are
-// gemm_tile.hip's.  The reference's matmul_rhs_transposed_tiled
+// bf16 GEMM out = a . w^T for the prefill-sized projections: the launch of every
+// tiled product as gemm_plan.cpp plans it, and its 256 x 256 kernel; the
+// smaller tiles are gemm_tile.hip's.  The reference's matmul_rhs_transposed_tiled
 // (kernels/full_attention_4b.hip:2513-2575) and the hipBLASLt calls the
 // projection entry points used before, as one MFMA kernel for gfx950.
 //
@@ -368,111 +368,17 @@ __global__ void gemm_bt_simple_kernel(GemmKParams p) {
     }
 }
 
-// Picks the tiles and the k split by an estimate of the time in microseconds:
-// rounds of workgroups (one a CU; two for the 32- and 64-row tiles, whose
-// LDS allows it) of `KT` 64-deep steps each, a constant a round for filling
-// the pipeline and the epilogue, a term for the partials of a split, and no
-// less than the HBM time of the operands.  The step times (s0 with few
-// workgroups, s0 + s1 with every CU busy) were fitted to 2900 timings of the
-// Q/K/V and output projections of the 8/2-, 16/4- and 16/2-head layers at 13 to
-// 8192 rows (one MI355X); over those the pick is within 0.5% of the best
-// plan on average and 9% at worst.  256 x 256 tiles stay where one round of
-// them holds the whole product and k is short (k = 1024, 2000 rows x 5120:
-// 37.7 us against 41.6 for 128 x 128).
-namespace {
-struct TileCost {
-    int bm, bn, max_m, slots;
-    double s0, s1, round;
-};
-constexpr int kPlanCus = 256;
-constexpr TileCost kTileCosts[] = {
-    {256, 256, 0x7fffffff, 1, 1.437, 0.361, 4.32}, {256, 128, 0x7fffffff, 1, 0.617, 0.217, 4.77},
-    {128, 128, 0x7fffffff, 1, 0.489, 0.060, 1.74}, {128, 64, 0x7fffffff, 1, 0.336, 0.073, 1.25},
-    {64, 64, 600, 2, 0.290, 0.248, 1.25},          {32, 64, 200, 2, 0.192, 0.210, 1.25},
-};
-// `wgs` workgroups of n steps
-double rounds_us(const TileCost& c, int64_t wgs, double n) {
-    const int64_t slots = static_cast<int64_t>(kPlanCus) * c.slots, r = wgs / slots, rem = wgs % slots;
-    double t = static_cast<double>(r) * (n * (c.s0 + c.s1) + c.round);
-    if (rem) {
-        const double busy = c.slots > 1 ? (rem > kPlanCus ? 1.0 : 0.0) : static_cast<double>(rem) / kPlanCus;
-        t += n * (c.s0 + c.s1 * busy) + c.round;
-    }
-    return t;
-}
-}  // namespace
-
-GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch) {
-    GemmPlan best;
-    double best_t = 1e30;
-    const int KT = (k + 63) / 64;
-    double nsum = 0;
-    for (int s = 0; s < nseg; ++s) nsum += n[s];
-    const double hbm = 2.0 * batch * (nsum * k + static_cast<double>(m) * k + m * nsum) / 5.64e6;
-    auto take = [&](const TileCost& c, int ks, int64_t split, double t, double handicap) {
-        t = (std::max(t, hbm) + 1.85) * handicap;
-        if (t < best_t) {
-            best_t = t;
-            best = GemmPlan{c.bm, c.bn, ks, static_cast<int>(split)};
-        }
-    };
-    for (const TileCost& c : kTileCosts) {
-        if (m > c.max_m) continue;
-        int64_t nt = 0;
-        for (int s = 0; s < nseg; ++s) nt += (n[s] + c.bn - 1) / c.bn;
-        const int64_t tiles = nt * ((m + c.bm - 1) / c.bm) * batch;
-        const int64_t tail = tiles > kPlanCus ? tiles % kPlanCus : 0;
-        if (c.bn == 256) {
-            double t = rounds_us(c, tiles, KT);
-            if (batch == 1 && tail > 0 && 2 * tail <= kPlanCus && KT >= 4)  // gemm_bt's tail split
-                t = rounds_us(c, tiles - tail, KT) + rounds_us(c, 2 * tail, 0.5 * KT) + 7.5;
-            take(c, 1, 0, t, 1.0);
-            continue;
-        }
-        // Whole tiles, then a split of every tile, then of the last partial
-        // round's; a split has to win 4%, the smaller tiles 2%.
-        take(c, 1, 0, rounds_us(c, tiles, KT), 1.02);
-        if (batch > 1) continue;
-        for (int all = 1; all >= 0; --all) {
-            const int64_t split = all ? tiles : tail;
-            for (int ks = 2; ks <= (all ? 16 : 8) && split > 0 && KT / ks >= 3 && split * ks <= (all ? 1600 : 600); ++ks) {
-                const int kper = (KT + ks - 1) / ks, kk = (KT + kper - 1) / kper;
-                const double kb = c.bm * c.bn * 4.0 / 1024.0;  // one slice's partials
-                double t = rounds_us(c, split * kk, kper) + 1.4 + 0.0212 * kk * kb + split * kk * kb * 2048.0 / 11.6e6;
-                if (!all) t += rounds_us(c, tiles - split, KT);
-                take(c, ks, split, t, 1.02 * 1.04);
-            }
-        }
-    }
-    return best;
-}
-
-size_t gemm_ws_bytes(int m, int k, int nseg, const int* n) {
-    const GemmPlan p = gemm_plan(m, k, nseg, n);
-    if (p.bn != 256) return gemm_split_bytes(p);
-    int64_t nt = 0;
-    for (int s = 0; s < nseg; ++s) nt += (n[s] + 255) / 256;
-    const int64_t tiles = static_cast<int64_t>((m + 255) / 256) * nt;
-    const int tail = static_cast<int>(tiles % kPlanCus);
-    return tiles > kPlanCus && tail > 0 && 2 * tail <= kPlanCus ? gemm_tail_bytes(tail) : 0;
-}
-
 int gemm_bt(hipStream_t st, const GemmArgs& g) {
     if (g.batch <= 0 || g.m <= 0 || g.k < 0 || g.nseg < 1 || g.nseg > 3) return 1;
     if (g.lda < g.k || g.batch > 65535) return 1;
     // 32-bit per-lane copy offsets: 256 rows of lda elements stay below the
     // buffer range (2^31 - 16 bytes)
     const bool tiled = g.k % 8 == 0 && g.lda % 8 == 0 && g.lda < (1 << 22);
-    if (tiled && g.k > 0) {
-        int ntot = 0;
-        for (int s = 0; s < g.nseg; ++s) ntot += g.n[s] > 0;
-        GemmPlan plan = gemm_plan(g.m, g.k, g.nseg, g.n, g.batch);
-        if (ntot > 0 && plan.bn != 256) {
-            // a workspace too small for the split: every tile runs whole
-            if (!g.ws || g.ws_bytes < gemm_split_bytes(plan)) plan.ks = 1;
-            return gemm_tile(st, g, plan);
-        }
-    }
+    int ntot = 0;
+    for (int s = 0; s < g.nseg; ++s) ntot += g.n[s] > 0;
+    if (ntot == 0) return 0;
+    if (g.plan.bytes > 0 && !g.ws) return 1;
+    if (tiled && g.k > 0 && g.plan.bn != 256) return gemm_tile(st, g);
     GemmKParams p{};
     p.a = g.a;
     p.lda = g.lda;
@@ -494,7 +400,6 @@ int gemm_bt(hipStream_t st, const GemmArgs& g) {
         p.nt_end[s] = nt;
     }
     p.nt = nt;
-    if (nt == 0) return 0;
     const int64_t tiles = static_cast<int64_t>(p.mt) * nt;
     if (tiles > 0x7fffffff) return 1;
     p.tiles = static_cast<int>(tiles);
@@ -502,16 +407,11 @@ int gemm_bt(hipStream_t st, const GemmArgs& g) {
     {
         // Tail split: with whole rounds of one workgroup a CU, the last
         // partial round's tiles run as two half-k workgroups each.
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
-        const int tail = p.tiles % cus;
-        const int KT = (g.k + kGBK - 1) / kGBK;
-        if (g.batch == 1 && p.tiles > cus && tail > 0 && 2 * tail <= cus && KT >= 4 &&
-            g.ws && g.ws_bytes >= gemm_tail_bytes(tail)) {
+        const int tail = g.plan.tail;
+        if (tiled && tail > 0) {
             p.full = p.tiles - tail;
             p.tail = tail;
-            p.khalf = KT / 2;
+            p.khalf = (g.k + kGBK - 1) / kGBK / 2;
             p.flags = static_cast<unsigned*>(g.ws);
             p.tail_polls = wait_polls(1 << 22);
             p.part = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(g.ws) + kGemmPartOff);

@@ -1,0 +1,92 @@
+// The plan of a tiled product: which tiles, and how k is split.
+#include "gemm_plan.hpp"
+
+#include <algorithm>
+
+namespace ssa {
+
+// Picks the tiles and the k split by an estimate of the time in microseconds:
+// rounds of workgroups (one a CU; two for the 32- and 64-row tiles, whose
+// LDS allows it) of `KT` 64-deep steps each, a constant a round for filling
+// the pipeline and the epilogue, a term for the partials of a split, and no
+// less than the HBM time of the operands.  The step times (s0 with few
+// workgroups, s0 + s1 with every CU busy) were fitted to 2900 timings of the
+// Q/K/V and output projections of the 8/2-, 16/4- and 16/2-head layers at 13 to
+// 8192 rows (one MI355X); over those the pick is within 0.5% of the best
+// plan on average and 9% at worst.  256 x 256 tiles stay where one round of
+// them holds the whole product and k is short (k = 1024, 2000 rows x 5120:
+// 37.7 us against 41.6 for 128 x 128).
+namespace {
+struct TileCost {
+    int bm, bn, max_m, slots;
+    double s0, s1, round;
+};
+constexpr int kPlanCus = 256;
+constexpr TileCost kTileCosts[] = {
+    {256, 256, 0x7fffffff, 1, 1.437, 0.361, 4.32}, {256, 128, 0x7fffffff, 1, 0.617, 0.217, 4.77},
+    {128, 128, 0x7fffffff, 1, 0.489, 0.060, 1.74}, {128, 64, 0x7fffffff, 1, 0.336, 0.073, 1.25},
+    {64, 64, 600, 2, 0.290, 0.248, 1.25},          {32, 64, 200, 2, 0.192, 0.210, 1.25},
+};
+// `wgs` workgroups of n steps
+double rounds_us(const TileCost& c, int64_t wgs, double n) {
+    const int64_t slots = static_cast<int64_t>(kPlanCus) * c.slots, r = wgs / slots, rem = wgs % slots;
+    double t = static_cast<double>(r) * (n * (c.s0 + c.s1) + c.round);
+    if (rem) {
+        const double busy = c.slots > 1 ? (rem > kPlanCus ? 1.0 : 0.0) : static_cast<double>(rem) / kPlanCus;
+        t += n * (c.s0 + c.s1 * busy) + c.round;
+    }
+    return t;
+}
+}  // namespace
+
+GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch, size_t room) {
+    GemmPlan best;
+    best.us = 1e30;
+    if (k <= 0 || k % 8 != 0) return best;  // not a tiled product
+    const int KT = (k + 63) / 64;
+    double nsum = 0;
+    for (int s = 0; s < nseg; ++s) nsum += n[s];
+    const double hbm = 2.0 * batch * (nsum * k + static_cast<double>(m) * k + m * nsum) / 5.64e6;
+    // split: tiles over ks slices of k, tail: 256 x 256 tiles in two halves
+    auto take = [&](const TileCost& c, int ks, int64_t split, int64_t tail, double t, double handicap) {
+        t = (std::max(t, hbm) + 1.85) * handicap;
+        if (t >= best.us) return;
+        const size_t bytes = tail > 0 ? gemm_tail_bytes(static_cast<int>(tail))
+                             : ks > 1 ? kGemmPartOff + static_cast<size_t>(split) * ks * c.bm * c.bn * sizeof(float) : 0;
+        if (bytes > room) return;
+        best = GemmPlan{c.bm, c.bn, ks, static_cast<int>(split), static_cast<int>(tail), bytes, t};
+    };
+    for (const TileCost& c : kTileCosts) {
+        if (m > c.max_m) continue;
+        int64_t nt = 0;
+        for (int s = 0; s < nseg; ++s) nt += (n[s] + c.bn - 1) / c.bn;
+        const int64_t tiles = nt * ((m + c.bm - 1) / c.bm) * batch;
+        const int64_t tail = tiles > kPlanCus ? tiles % kPlanCus : 0;
+        if (c.bn == 256) {
+            // the last partial round in two halves of k where that is possible, whole
+            // where the workspace has no room for it
+            if (batch == 1 && tail > 0 && 2 * tail <= kPlanCus && KT >= 4 && gemm_tail_bytes(static_cast<int>(tail)) <= room)
+                take(c, 1, 0, tail, rounds_us(c, tiles - tail, KT) + rounds_us(c, 2 * tail, 0.5 * KT) + 7.5, 1.0);
+            else
+                take(c, 1, 0, 0, rounds_us(c, tiles, KT), 1.0);
+            continue;
+        }
+        // Whole tiles, then a split of every tile, then of the last partial
+        // round's; a split has to win 4%, the smaller tiles 2%.
+        take(c, 1, 0, 0, rounds_us(c, tiles, KT), 1.02);
+        if (batch > 1) continue;
+        for (int all = 1; all >= 0; --all) {
+            const int64_t split = all ? tiles : tail;
+            for (int ks = 2; ks <= (all ? 16 : 8) && split > 0 && KT / ks >= 3 && split * ks <= (all ? 1600 : 600); ++ks) {
+                const int kper = (KT + ks - 1) / ks, kk = (KT + kper - 1) / kper;
+                const double kb = c.bm * c.bn * 4.0 / 1024.0;  // one slice's partials
+                double t = rounds_us(c, split * kk, kper) + 1.4 + 0.0212 * kk * kb + split * kk * kb * 2048.0 / 11.6e6;
+                if (!all) t += rounds_us(c, tiles - split, KT);
+                take(c, ks, split, 0, t, 1.02 * 1.04);
+            }
+        }
+    }
+    return best;
+}
+
+}  // namespace ssa

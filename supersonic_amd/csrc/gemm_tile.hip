@@ -312,7 +312,8 @@ static int launch_tile(hipStream_t st, const GemmTileParams& p, int batch, int e
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-int gemm_tile(hipStream_t st, const GemmArgs& g, const GemmPlan& plan) {
+int gemm_tile(hipStream_t st, const GemmArgs& g) {
+    const GemmPlan& plan = g.plan;
     GemmTileParams p{};
     p.a = g.a;
     p.lda = g.lda;

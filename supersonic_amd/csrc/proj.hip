@@ -552,11 +552,34 @@ bool use_hipblaslt() {
     return v && std::strcmp(v, "hipblaslt") == 0;
 }
 size_t lt_ws_bytes() { return use_hipblaslt() ? kLtWorkspace : 0; }
-// The three projections (or one) as one hand-written GEMM launch.  ws: the
-// caller's region for the tail split (gemm_ws_bytes()), or null for the
-// library's own.
-int gemm_segments(int dev, hipStream_t st, int m, int k, const void* a, int nseg, const void* const* w,
-                  void* const* out, const int* n, int epilogue, uint8_t* ws, size_t ws_bytes) {
+// A hand-written GEMM call's plan and the workspace it takes: of the caller's
+// region (ws), or the library's own.
+struct GemmCall {
+    GemmPlan plan;
+    uint8_t* ws = nullptr;
+};
+// A tail split's region that the caller's is too small for is an error (a
+// status); a k split without room leaves the call to the best plan that fits.
+int plan_gemm(int dev, int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, GemmCall* call) {
+    GemmPlan& plan = call->plan;
+    plan = gemm_plan(m, k, nseg, n);
+    if (plan.bytes == 0) return 0;
+    if (ws) {
+        if (plan.bytes > ws_bytes) {
+            if (plan.tail > 0) return SUPERSONIC_ERR_LAUNCH;
+            plan = gemm_plan(m, k, nseg, n, 1, ws_bytes);
+        }
+        call->ws = ws;
+    } else {
+        call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceGemm));
+        if (!call->ws) plan = gemm_plan(m, k, nseg, n, 1, 0);
+    }
+    return 0;
+}
+
+// The three projections (or one) as one hand-written GEMM launch.
+int gemm_segments(hipStream_t st, int m, int k, const void* a, int nseg, const void* const* w, void* const* out,
+                  const int* n, int epilogue, const GemmCall& call) {
     GemmArgs g;
     g.m = m;
     g.k = k;
@@ -569,30 +592,17 @@ int gemm_segments(int dev, hipStream_t st, int m, int k, const void* a, int nseg
         g.n[i] = n[i];
     }
     g.epilogue = epilogue;
-    const size_t need = gemm_ws_bytes(m, k, nseg, n);
-    if (need > 0) {
-        if (ws) {
-            // a tail split's region that is missing is the caller's error; a
-            // k split without room runs its tiles whole
-            if (gemm_plan(m, k, nseg, n).bn == 256 && ws_bytes < need) return 1;
-            g.ws = ws;
-            g.ws_bytes = ws_bytes;
-        } else {
-            g.ws = device_workspace(dev, need, kWorkspaceGemm);
-            g.ws_bytes = g.ws ? need : 0;
-        }
-    }
+    g.plan = call.plan;
+    g.ws = call.ws;
     return gemm_bt(st, g);
 }
 
-// Arrival counters that the GEMM of this shape takes in the caller's region
-// (NULL: none of the caller's): their number, and where they are.
-int split_counters(int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, unsigned** at) {
-    if (!ws || use_hipblaslt()) return 0;
-    const GemmPlan plan = gemm_plan(m, k, nseg, n);
-    if (plan.ks == 1 || ws_bytes < gemm_split_bytes(plan)) return 0;
-    *at = reinterpret_cast<unsigned*>(ws + kGemmFlagBytes);
-    return plan.split_tiles;
+// The arrival counters that a call takes in the caller's region (NULL: none of
+// the caller's): their number, and where they are.
+int split_counters(const uint8_t* ws, const GemmCall& call, unsigned** at) {
+    if (!ws || call.ws != ws || call.plan.ks == 1) return 0;
+    *at = reinterpret_cast<unsigned*>(call.ws + kGemmFlagBytes);
+    return call.plan.split_tiles;
 }
 
 bool make_layout(hipblasLtMatrixLayout_t* l, uint64_t rows, uint64_t cols, int64_t ld, int batch, int64_t stride) {
@@ -704,9 +714,12 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
             g.w_bs = static_cast<int64_t>(n) * k;
             g.o_bs = static_cast<int64_t>(m) * n;
             if (batch == 1) {
-                g.ws_bytes = gemm_ws_bytes(m, k, 1, &n);
-                if (g.ws_bytes > 0) g.ws = device_workspace(dev, g.ws_bytes, kWorkspaceGemm);
-                if (!g.ws) g.ws_bytes = 0;
+                GemmCall call;
+                if (plan_gemm(dev, m, k, 1, &n, nullptr, 0, &call) != 0) return 270;
+                g.plan = call.plan;
+                g.ws = call.ws;
+            } else {
+                g.plan = gemm_plan(m, k, 1, &n, batch);
             }
             if (gemm_bt(nullptr, g) != 0) return 270;
         }
@@ -753,7 +766,7 @@ size_t o_proj_ws_bytes(int m, int n, int k) {
     // the streaming kernels' region or the tiled GEMM's (which adds into the
     // hidden rows in place), whichever the call takes
     const size_t stream = m <= skinny_max_m() ? skinny_ws_bytes(m, k, (n + kSkinnyCols - 1) / kSkinnyCols) : 0;
-    if (!use_hipblaslt()) return std::max(stream, (m > skinny_max_m() ? 256 : 0) + gemm_ws_bytes(m, k, 1, &n));
+    if (!use_hipblaslt()) return std::max(stream, (m > skinny_max_m() ? 256 : 0) + gemm_plan(m, k, 1, &n).bytes);
     return align256(static_cast<size_t>(m) * n * 2) + kLtWorkspace;
 }
 // Workspace of the qkv entry point: the normed rows, then the streaming
@@ -762,7 +775,7 @@ size_t qkv_ws_bytes(int m, int k, int nq, int nkv) {
     const size_t normed = align256(static_cast<size_t>(m) * k * 2);
     const int ns[3] = {nq, nkv, nkv};
     const size_t stream = m <= skinny_max_m() ? skinny_ws_bytes(m, k, nq / kSkinnyCols + 2 * (nkv / kSkinnyCols)) : 0;
-    return normed + (use_hipblaslt() ? std::max(stream, lt_ws_bytes()) : std::max(stream, gemm_ws_bytes(m, k, 3, ns)));
+    return normed + (use_hipblaslt() ? std::max(stream, lt_ws_bytes()) : std::max(stream, gemm_plan(m, k, 3, ns).bytes));
 }
 }  // namespace ssa
 
@@ -816,9 +829,9 @@ extern "C" int supersonic_attn_gfx950_o_proj_residual(size_t device_ordinal, voi
         if (k == 0) return 0;  // nothing to add
         const void* w1[1] = {o_proj_w};
         void* o1[1] = {hidden};
-        const int n1[1] = {n};
-        if (gemm_segments(dev, st, m, k, attn, 1, w1, o1, n1, f32 ? kGemmResidualF32 : kGemmResidualBf16, ws,
-                          workspace_bytes) != 0)
+        GemmCall call;
+        if (const int rc = plan_gemm(dev, m, k, 1, &n, ws, workspace_bytes, &call)) return rc;
+        if (gemm_segments(st, m, k, attn, 1, w1, o1, &n, f32 ? kGemmResidualF32 : kGemmResidualBf16, call) != 0)
             return SUPERSONIC_ERR_LAUNCH;
     } else {
         const size_t total = rows * hidden_dim;
@@ -894,8 +907,11 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
     const int ns[3] = {nq, nkv, nkv};
     const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
                         nkv % kSkinnyCols == 0 && stream_columns(dev, (nq + 2 * nkv) / kSkinnyCols);
+    GemmCall call;
+    if (!skinny && !use_hipblaslt())
+        if (const int rc = plan_gemm(dev, m, k, 3, ns, rest, rest_bytes, &call)) return rc;
     unsigned* clear = nullptr;
-    const int n_clear = skinny ? 0 : split_counters(m, k, 3, ns, rest, rest_bytes, &clear);
+    const int n_clear = split_counters(rest, call, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {
@@ -934,8 +950,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
         const void* wts[3] = {q_proj_w, k_proj_w, v_proj_w};
         void* os[3] = {q_proj_out, k_out, v_out};
         if (!use_hipblaslt()) {
-            if (gemm_segments(dev, st, m, k, normed, 3, wts, os, ns, kGemmStore, ws ? rest : nullptr, rest_bytes) != 0)
-                return SUPERSONIC_ERR_LAUNCH;
+            if (gemm_segments(st, m, k, normed, 3, wts, os, ns, kGemmStore, call) != 0) return SUPERSONIC_ERR_LAUNCH;
         } else {
             if (ws && rest_bytes < kLtWorkspace) return SUPERSONIC_ERR_WORKSPACE;
             for (int i = 0; i < 3; ++i) {
@@ -1049,8 +1064,12 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
                         nkv % kSkinnyCols == 0 && stream_columns(dev, ncb);
     const int ns[3] = {nq, nkv, nkv};
+    uint8_t* const own = workspace ? pws : nullptr;
+    GemmCall call;
+    if (!fused && !skinny && !use_hipblaslt())
+        if (const int rc = plan_gemm(dev, m, k, 3, ns, own, pws_bytes, &call)) return rc;
     unsigned* clear = nullptr;
-    const int n_clear = fused || skinny ? 0 : split_counters(m, k, 3, ns, workspace ? pws : nullptr, pws_bytes, &clear);
+    const int n_clear = split_counters(own, call, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {
@@ -1104,9 +1123,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
             const void* wts[3] = {q_proj_w, k_proj_w, v_proj_w};
             void* os[3] = {qp, kr, vr};
             if (!use_hipblaslt()) {
-                if (gemm_segments(dev, st, m, k, normed, 3, wts, os, ns, kGemmStore, workspace ? pws : nullptr,
-                                  pws_bytes) != 0)
-                    return SUPERSONIC_ERR_LAUNCH;
+                if (gemm_segments(st, m, k, normed, 3, wts, os, ns, kGemmStore, call) != 0) return SUPERSONIC_ERR_LAUNCH;
             } else {
                 if (workspace && pws_bytes < kLtWorkspace) return SUPERSONIC_ERR_WORKSPACE;
                 for (int i = 0; i < 3; ++i)
