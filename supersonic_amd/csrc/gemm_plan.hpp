@@ -10,7 +10,8 @@ namespace ssa {
 // Workspace of a projection's split work: a header of counts at fixed places,
 // whatever the shape, then the partials.  Every call leaves the tail's two
 // counts of a tile equal and the arrival counters at zero, so calls of
-// different shapes can follow each other on one workspace.
+// different shapes can follow each other on one workspace.  (Where the header
+// itself moves, behind the normed rows of a Q/K/V call, the call clears its counts.)
 constexpr size_t kGemmFlagBytes = 8192;         // tail counts, two per tile (<= 1024 tail tiles)
 constexpr size_t kGemmArrivalBytes = 64 << 10;  // split-k arrival counters, one per tile or column block
 constexpr size_t kGemmPartOff = kGemmFlagBytes + kGemmArrivalBytes;

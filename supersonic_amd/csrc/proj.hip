@@ -195,9 +195,8 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_kernel(SkinnyParams 
 // workgroup per row, 8 elements (16 or 32 bytes) per thread and chunk, every
 // chunk's load issued before the reduction (k <= 8192 in one pass of
 // registers; longer rows re-read their chunks from cache).  Also clears the
-// arrival counters of the split-k GEMM that follows: in the Q/K/V workspace
-// they sit behind the normed rows, so a call with another row count may have
-// written there.
+// counts of the projection that follows where they are in the Q/K/V workspace
+// (moving_counts).
 template <typename XT>
 __global__ __launch_bounds__(256) void input_norm_kernel(int rows, int k, float eps, const XT* x, const uint16_t* w,
                                                          uint16_t* out, unsigned* clear, int n_clear) {
@@ -456,6 +455,13 @@ size_t skinny_ws_bytes(int m, int k, int64_t wgs) {
     return kGemmPartOff + static_cast<size_t>(wgs) * ks * kSkinnyCB * MB * 256 * sizeof(float);
 }
 
+// Arrival counters that the streaming kernels of a Q/K/V call of ncb column
+// blocks use.
+int stream_counts(int dev, int m, int k, int ncb) {
+    const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
+    return !lds_path(dev, m, k, 1, ncb) && skinny_k_split(cus, ncb, k) > 1 ? ncb : 0;
+}
+
 // ws: the skinny_ws_bytes() region (arrival counters zero between calls), or
 // NULL for the library's own.
 template <typename OT, bool RES>
@@ -597,12 +603,15 @@ int gemm_segments(hipStream_t st, int m, int k, const void* a, int nseg, const v
     return gemm_bt(st, g);
 }
 
-// The arrival counters that a call takes in the caller's region (NULL: none of
-// the caller's): their number, and where they are.
-int split_counters(const uint8_t* ws, const GemmCall& call, unsigned** at) {
-    if (!ws || call.ws != ws || call.plan.ks == 1) return 0;
-    *at = reinterpret_cast<unsigned*>(call.ws + kGemmFlagBytes);
-    return call.plan.split_tiles;
+// The counts that a call takes in the caller's region behind its normed rows
+// (NULL: none of the caller's): their number, and where they are.  The region
+// moves with the row count, so a call with more rows may have left its normed
+// rows there, and the norm kernel clears them.
+int moving_counts(uint8_t* region, const GemmCall& call, int stream_wgs, unsigned** at) {
+    if (!region) return 0;
+    const bool tail = call.plan.tail > 0;
+    *at = reinterpret_cast<unsigned*>(region + (tail ? 0 : kGemmFlagBytes));
+    return tail ? 2 * call.plan.tail : (call.plan.ks > 1 ? call.plan.split_tiles : stream_wgs);
 }
 
 bool make_layout(hipblasLtMatrixLayout_t* l, uint64_t rows, uint64_t cols, int64_t ld, int batch, int64_t stride) {
@@ -911,7 +920,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
     if (!skinny && !use_hipblaslt())
         if (const int rc = plan_gemm(dev, m, k, 3, ns, rest, rest_bytes, &call)) return rc;
     unsigned* clear = nullptr;
-    const int n_clear = split_counters(rest, call, &clear);
+    const int n_clear = moving_counts(rest, call, skinny ? stream_counts(dev, m, k, (nq + 2 * nkv) / kSkinnyCols) : 0, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {
@@ -1069,7 +1078,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     if (!fused && !skinny && !use_hipblaslt())
         if (const int rc = plan_gemm(dev, m, k, 3, ns, own, pws_bytes, &call)) return rc;
     unsigned* clear = nullptr;
-    const int n_clear = split_counters(own, call, &clear);
+    const int n_clear = moving_counts(own, call, skinny && !fused ? stream_counts(dev, m, k, ncb) : 0, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {

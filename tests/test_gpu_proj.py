@@ -14,6 +14,7 @@ import torch
 
 from gpu_util import DEV, announce, gen
 from oracle import attn_oracle as O
+from plan_util import gemm_plan
 from supersonic_amd import kernel_ffi as K
 
 pytestmark = pytest.mark.gpu
@@ -479,6 +480,54 @@ def test_projections_share_a_workspace_over_row_counts():
         big = torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())
         assert_ulps(h.float().cpu(), ref, 2 * ulp(big) + 1e-6, f"o_proj shared ws rows={r}")
     assert K.wait_status() == 0
+
+
+# More rows first: their normed rows lie where the fewer rows' counts are.  8192 and 8000 rows of 1024 -> 4096 + 2 x 512
+# take 256 x 256 tiles with a tail split, 12 and 4 rows of 4096 -> 512 + 2 x 128 the streaming kernel over two k slices,
+# 600 and 300 rows of 4096 -> 1024 + 2 x 256 tiles over slices of k.
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("counts,hid,Hq,Hkv,D,plan", [((8000, 8192, 8000), 1024, 8, 2, 256, "tail"),
+                                                      ((4, 12, 4), 4096, 2, 1, 128, None),
+                                                      ((300, 600, 300), 4096, 2, 1, 256, "split")])
+def test_qkv_projections_share_a_workspace_over_row_counts(counts, hid, Hq, Hkv, D, plan, rope):
+    announce(f"qkv one workspace, rows {counts}, rope {rope}")
+    g = gen(94)
+    nq, nkv = Hq * 2 * D, Hkv * D
+    for r in set(counts) if plan else ():
+        p = gemm_plan(r, hid, (nq, nkv, nkv))
+        assert (p.tail if plan == "tail" else p.ks > 1), p
+    nw = O.randn_bf16(g, hid, std=0.1)
+    wq, wk, wv = (O.randn_bf16(g, n, hid, std=hid ** -0.5) for n in (nq, nkv, nkv))
+    wts = [t.to(DEV) for t in (nw, wq, wk, wv)]
+    size = lambda r: K.qkv_proj_rope_workspace_size(r, hid, Hq, Hkv, D) if rope else K.qkv_proj_workspace_size(r, hid, nq, nkv)
+    ws = torch.zeros(max(size(r) for r in counts), dtype=torch.uint8, device=DEV)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(64, 64, 1.0e7))
+    hidden = O.randn_bf16(g, max(counts), hid)
+    cases = {}
+    for r in counts:
+        # against the call on a workspace of its own
+        x = hidden[:r].to(DEV)
+        dims = (Hq * D, Hq * D, nkv, nkv) if rope else (nq, nkv, nkv)
+        outs = [[torch.full((r, n), float("nan"), dtype=torch.bfloat16, device=DEV) for n in dims] for _ in range(2)]
+        pos = torch.arange(r, dtype=torch.int32, device=DEV) % 64
+        for o, w in zip(outs, (torch.zeros(size(r), dtype=torch.uint8, device=DEV), ws)):
+            if rope:
+                qk = [torch.zeros(D, dtype=torch.bfloat16, device=DEV)] * 2
+                K.qkv_proj_rope(0, x, *wts, *qk, cos, sin, pos, *o, workspace=w, q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=64)
+            else:
+                K.qkv_proj(0, x, *wts, *o, workspace=w)
+        torch.cuda.synchronize()
+        assert K.wait_status() == 0
+        for own, shared in zip(*outs):
+            assert torch.equal(own, shared), f"rows {r}"
+        if not rope and r not in cases:
+            cases[r] = outs[1]
+    for r, out in cases.items():
+        if r > 1000:
+            continue  # (the oracle's product takes long)
+        for o, ref in zip(out, O.qkv_proj(hidden[:r].float(), nw, wq, wk, wv)):
+            big = torch.maximum(o.float().cpu().abs(), ref.float().abs())
+            assert_ulps(o.float().cpu(), ref, 2 * ulp(big) + 2.0 ** -7, f"qkv shared ws rows={r}")
 
 
 def test_gemm_tail_expired_handover_is_reported(monkeypatch):
