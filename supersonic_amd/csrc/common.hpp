@@ -324,11 +324,18 @@ constexpr int kWorkspacePrefill = 1;
 constexpr int kWorkspaceProj = 2;    // scratch rows: the o_proj GEMM output (hipBLASLt path), qkv_proj normed rows
 constexpr int kWorkspaceProjLt = 3;  // hipBLASLt workspace
 constexpr int kWorkspaceSkinny = 4;  // split-k partials and arrival counters of the o_proj kernel
-constexpr int kWorkspaceGemm = 5;    // split partials and counts of the hand-written GEMMs
+constexpr int kWorkspaceGemm = 5;    // tail-split partials and counts of the 256 x 256 GEMM
 constexpr int kWorkspaceRope = 6;    // qkv_proj_rope: per-head counters (zero between calls), then rows
 constexpr int kWorkspaceMixed = 7;   // mixed step: the prefill's claim counters (zero between calls)
-constexpr int kWorkspaceSlots = 8;
+constexpr int kWorkspaceSplit = 8;   // k-split partials and counts of the smaller GEMM tiles
+constexpr int kWorkspacePieces = 9;  // a prefill key split's sums (one size, so it never moves)
+constexpr int kWorkspaceSlots = 10;
 void* device_workspace(int device, size_t bytes, int slot);
+// The slot's buffer if it holds `bytes` as it is, else NULL: what a call may
+// take while `stream` is being captured, when nothing can be allocated, for
+// work that it can do without.
+void* device_workspace_held(int device, size_t bytes, int slot);
+bool stream_capturing(hipStream_t stream);
 
 // Compute units of `device` (cached; 256 on MI355X), 0 if the query fails.
 int device_cu_count(int device);

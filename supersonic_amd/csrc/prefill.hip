@@ -1231,14 +1231,12 @@ __global__ __launch_bounds__(64 * kKvStageWaves) void kv_stage_kernel(KvStagePar
 
 // Stages V^T for `B` sequences of `L` keys into the prefill workspace slot of
 // `device` and points `p` at it.  Returns hipSuccess or the failing error.
-// `part_bytes` more are kept for a key split, at *part.
 static hipError_t stage_vt(int device, hipStream_t st, const KvView& kv, int B, int Hkv, int L, int D,
-                           PrefillParams& p, size_t part_bytes, void** part) {
+                           PrefillParams& p) {
     const int ld = (L + 63) / 64 * 64;
-    const size_t bytes = (static_cast<size_t>(B) * Hkv * D * ld * 2 + 255) & ~static_cast<size_t>(255);
-    void* ws = device_workspace(device, bytes + part_bytes, kWorkspacePrefill);
+    const size_t bytes = static_cast<size_t>(B) * Hkv * D * ld * 2;
+    void* ws = device_workspace(device, bytes, kWorkspacePrefill);
     if (!ws) return hipErrorOutOfMemory;
-    *part = part_bytes ? static_cast<uint8_t*>(ws) + bytes : nullptr;
     p.vt = static_cast<const uint16_t*>(ws);
     p.vt_ld = ld;
     const dim3 grid(ld / 64, Hkv, B);
@@ -1264,6 +1262,16 @@ static size_t prefill_part_bytes(int D, int n_wg) { return static_cast<size_t>(n
 // pieces that win more than their merge costs.
 static bool prefill_may_split(size_t S, size_t L, size_t Hkv) {
     return S * Hkv <= 8192 && L > 2 * 64 * kSplitMinTiles;
+}
+
+// Room for a key split's sums where the caller gave none (NULL: the chunk runs
+// whole): a library buffer of one size, so that it never moves, apart from the
+// staging's, so that the split never makes that one move.  While `st` is captured
+// only a buffer that is there already.
+static void* pieces_workspace(int device, hipStream_t st, size_t* bytes) {
+    *bytes = prefill_part_bytes(256, std::max(device_cu_count(device), 256));
+    return stream_capturing(st) ? device_workspace_held(device, *bytes, kWorkspacePieces)
+                                : device_workspace(device, *bytes, kWorkspacePieces);
 }
 
 // Fills in p's split (piece 0: none) for n workgroups.  The estimates are in
@@ -1439,10 +1447,10 @@ int prefill_dropin(int dtype, size_t device, size_t B, size_t Hq, size_t Hkv, si
     p.B = static_cast<int>(B);
     const int dev = static_cast<int>(device);
     void* part = nullptr;
-    const size_t part_bytes = prefill_may_split(q_len * B, kv_len, Hkv)
-                                  ? prefill_part_bytes(static_cast<int>(D), std::max(device_cu_count(dev), 256)) : 0;
+    size_t part_bytes = 0;
+    if (prefill_may_split(q_len * B, kv_len, Hkv)) part = pieces_workspace(dev, nullptr, &part_bytes);
     if (kv_len > 0 && stage_vt(dev, nullptr, p.kv, static_cast<int>(B), static_cast<int>(Hkv), static_cast<int>(kv_len),
-                               static_cast<int>(D), p, part_bytes, &part) != hipSuccess)
+                               static_cast<int>(D), p) != hipSuccess)
         return 11;
     const hipError_t e = dtype == 0 ? launch_prefill<f16_t, false>(dev, static_cast<int>(D), nullptr, p, part, part_bytes)
                                     : launch_prefill<bf16_t, false>(dev, static_cast<int>(D), nullptr, p, part, part_bytes);
@@ -1547,18 +1555,20 @@ int prefill_native(size_t device_ordinal, void* stream, int kv_dtype, size_t q_h
         // V^T staging, then (fp8 cache) the bf16 K rows the attention reads
         const size_t stage_bytes = static_cast<size_t>(p.Hkv) * head_dim * ld * 2;
         const size_t need = fp8 ? 2 * stage_bytes : stage_bytes;
-        // (stage_bytes is a multiple of 128)
-        if (prefill_may_split(chunk_len, p.L, kv_heads))
-            part_bytes = prefill_part_bytes(static_cast<int>(head_dim), std::max(device_cu_count(static_cast<int>(device_ordinal)), 256));
+        const bool may_split = prefill_may_split(chunk_len, p.L, kv_heads);
         void* ws = workspace;
         if (ws) {
             if (workspace_bytes < need) return SUPERSONIC_ERR_WORKSPACE;
-            part_bytes = std::min(part_bytes, workspace_bytes - need);
+            // (need is a multiple of 128)
+            if (may_split && workspace_bytes > need) {
+                part = static_cast<uint8_t*>(ws) + need;
+                part_bytes = workspace_bytes - need;
+            }
         } else {
-            ws = device_workspace(static_cast<int>(device_ordinal), need + part_bytes, kWorkspacePrefill);
+            ws = device_workspace(static_cast<int>(device_ordinal), need, kWorkspacePrefill);
+            if (ws && may_split) part = pieces_workspace(static_cast<int>(device_ordinal), st, &part_bytes);
         }
         if (!ws) return SUPERSONIC_ERR_WORKSPACE;
-        if (part_bytes) part = static_cast<uint8_t*>(ws) + need;
         p.vt = static_cast<const uint16_t*>(ws);
         p.vt_ld = ld;
         uint16_t* kst = fp8 ? reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(ws) + stage_bytes) : nullptr;

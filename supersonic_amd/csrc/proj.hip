@@ -566,7 +566,10 @@ struct GemmCall {
 };
 // A tail split's region that the caller's is too small for is an error (a
 // status); a k split without room leaves the call to the best plan that fits.
-int plan_gemm(int dev, int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, GemmCall* call) {
+// Nor does a call without a workspace split k while `st` is captured: the
+// library's buffer cannot be allocated then, and a graph that held it would
+// keep its address when a larger call moves it.
+int plan_gemm(int dev, hipStream_t st, int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, GemmCall* call) {
     GemmPlan& plan = call->plan;
     plan = gemm_plan(m, k, nseg, n);
     if (plan.bytes == 0) return 0;
@@ -577,7 +580,10 @@ int plan_gemm(int dev, int m, int k, int nseg, const int* n, uint8_t* ws, size_t
         }
         call->ws = ws;
     } else {
-        call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceGemm));
+        if (plan.tail > 0)
+            call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceGemm));
+        else if (!stream_capturing(st))
+            call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceSplit));
         if (!call->ws) plan = gemm_plan(m, k, nseg, n, 1, 0);
     }
     return 0;
@@ -724,7 +730,7 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
             g.o_bs = static_cast<int64_t>(m) * n;
             if (batch == 1) {
                 GemmCall call;
-                if (plan_gemm(dev, m, k, 1, &n, nullptr, 0, &call) != 0) return 270;
+                if (plan_gemm(dev, nullptr, m, k, 1, &n, nullptr, 0, &call) != 0) return 270;
                 g.plan = call.plan;
                 g.ws = call.ws;
             } else {
@@ -779,12 +785,15 @@ size_t o_proj_ws_bytes(int m, int n, int k) {
     return align256(static_cast<size_t>(m) * n * 2) + kLtWorkspace;
 }
 // Workspace of the qkv entry point: the normed rows, then the streaming
-// kernel's [counters | partials] or the hipBLASLt workspace.
-size_t qkv_ws_bytes(int m, int k, int nq, int nkv) {
+// kernel's [counters | partials] or the hipBLASLt workspace.  split: with the
+// room for a k split of the tiled GEMM, which a call can do without.
+size_t qkv_ws_bytes(int m, int k, int nq, int nkv, bool split = true) {
     const size_t normed = align256(static_cast<size_t>(m) * k * 2);
     const int ns[3] = {nq, nkv, nkv};
     const size_t stream = m <= skinny_max_m() ? skinny_ws_bytes(m, k, nq / kSkinnyCols + 2 * (nkv / kSkinnyCols)) : 0;
-    return normed + (use_hipblaslt() ? std::max(stream, lt_ws_bytes()) : std::max(stream, gemm_plan(m, k, 3, ns).bytes));
+    if (use_hipblaslt()) return normed + std::max(stream, lt_ws_bytes());
+    const GemmPlan plan = gemm_plan(m, k, 3, ns);
+    return normed + std::max(stream, split || plan.tail > 0 ? plan.bytes : 0);
 }
 }  // namespace ssa
 
@@ -839,7 +848,7 @@ extern "C" int supersonic_attn_gfx950_o_proj_residual(size_t device_ordinal, voi
         const void* w1[1] = {o_proj_w};
         void* o1[1] = {hidden};
         GemmCall call;
-        if (const int rc = plan_gemm(dev, m, k, 1, &n, ws, workspace_bytes, &call)) return rc;
+        if (const int rc = plan_gemm(dev, st, m, k, 1, &n, ws, workspace_bytes, &call)) return rc;
         if (gemm_segments(st, m, k, attn, 1, w1, o1, &n, f32 ? kGemmResidualF32 : kGemmResidualBf16, call) != 0)
             return SUPERSONIC_ERR_LAUNCH;
     } else {
@@ -918,7 +927,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
                         nkv % kSkinnyCols == 0 && stream_columns(dev, (nq + 2 * nkv) / kSkinnyCols);
     GemmCall call;
     if (!skinny && !use_hipblaslt())
-        if (const int rc = plan_gemm(dev, m, k, 3, ns, rest, rest_bytes, &call)) return rc;
+        if (const int rc = plan_gemm(dev, st, m, k, 3, ns, rest, rest_bytes, &call)) return rc;
     unsigned* clear = nullptr;
     const int n_clear = moving_counts(rest, call, skinny ? stream_counts(dev, m, k, (nq + 2 * nkv) / kSkinnyCols) : 0, &clear);
     const ProfileEvents ev = take_profile_events();
@@ -981,11 +990,10 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
 namespace ssa {
 constexpr size_t kRopeCounterBytes = 64 << 10;  // per-head arrival counters (Hq + Hkv <= 16384)
 
-size_t qkv_rope_ws_bytes(int m, int k, int Hq, int Hkv, int D) {
-    const size_t normed = align256(static_cast<size_t>(m) * k * 2);
+size_t qkv_rope_ws_bytes(int m, int k, int Hq, int Hkv, int D, bool split = true) {
     // unfused path: q_proj and the raw k / v rows, then the projection's own workspace
     const size_t raw = align256(static_cast<size_t>(m) * Hq * 2 * D * 2) + 2 * align256(static_cast<size_t>(m) * Hkv * D * 2);
-    return kRopeCounterBytes + normed + raw + qkv_ws_bytes(m, k, Hq * 2 * D, Hkv * D) - align256(static_cast<size_t>(m) * k * 2);
+    return kRopeCounterBytes + raw + qkv_ws_bytes(m, k, Hq * 2 * D, Hkv * D, split);
 }
 }  // namespace ssa
 
@@ -1027,7 +1035,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     const int m = static_cast<int>(rows), k = static_cast<int>(hidden_dim);
     const int Hq = static_cast<int>(q_heads), Hkv = static_cast<int>(kv_heads), D = static_cast<int>(head_dim);
     const int nq = Hq * 2 * D, nkv = Hkv * D;
-    const size_t need = qkv_rope_ws_bytes(m, k, Hq, Hkv, D);
+    const size_t need = qkv_rope_ws_bytes(m, k, Hq, Hkv, D, false);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     if (ws) {
         if (workspace_bytes < need) return SUPERSONIC_ERR_WORKSPACE;
@@ -1066,7 +1074,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     uint16_t* kr = reinterpret_cast<uint16_t*>(rest + align256(static_cast<size_t>(m) * nq * 2));
     uint16_t* vr = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(kr) + align256(static_cast<size_t>(m) * nkv * 2));
     uint8_t* pws = reinterpret_cast<uint8_t*>(vr) + align256(static_cast<size_t>(m) * nkv * 2);
-    const size_t pws_bytes = ws + need > pws ? static_cast<size_t>(ws + need - pws) : 0;
+    const size_t pws_bytes = (workspace ? workspace_bytes : need) - static_cast<size_t>(pws - ws);  // need reaches up to pws
     const int ncb = (nq + 2 * nkv) / kSkinnyCols;
     const bool fused = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
                        Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4) && stream_columns(dev, ncb);
@@ -1076,7 +1084,7 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     uint8_t* const own = workspace ? pws : nullptr;
     GemmCall call;
     if (!fused && !skinny && !use_hipblaslt())
-        if (const int rc = plan_gemm(dev, m, k, 3, ns, own, pws_bytes, &call)) return rc;
+        if (const int rc = plan_gemm(dev, st, m, k, 3, ns, own, pws_bytes, &call)) return rc;
     unsigned* clear = nullptr;
     const int n_clear = moving_counts(own, call, skinny && !fused ? stream_counts(dev, m, k, ncb) : 0, &clear);
     const ProfileEvents ev = take_profile_events();

@@ -51,6 +51,19 @@ void* device_workspace(int device, size_t bytes, int slot) {
     return w.ptr;
 }
 
+void* device_workspace_held(int device, size_t bytes, int slot) {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    if (device < 0 || slot < 0 || slot >= kWorkspaceSlots) return nullptr;
+    const size_t idx = static_cast<size_t>(device) * kWorkspaceSlots + slot;
+    return idx < g_ws.size() && g_ws[idx].bytes >= bytes ? g_ws[idx].ptr : nullptr;
+}
+
+// (The legacy stream cannot be captured.)
+bool stream_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return stream && hipStreamIsCapturing(stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
 int device_cu_count(int device) {
     static std::mutex m;
     static std::vector<int> counts;

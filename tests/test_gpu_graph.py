@@ -16,6 +16,7 @@ import torch
 
 from gpu_util import DEV, announce, gen
 from oracle import attn_oracle as O
+from plan_util import gemm_plan
 from supersonic_amd import kernel_ffi as K
 
 pytestmark = pytest.mark.gpu
@@ -277,3 +278,78 @@ def test_mixed_call_graph_replays_match_eager(monkeypatch):
         assert torch.equal(out_c, eager_c), f"replay {r}: chunk"
         assert torch.equal(out_d, eager_d), f"replay {r}: decodes"
         assert int(ws[:2048].count_nonzero()) == 0, f"replay {r}: claim counters"
+
+
+def replays_equal(graph, reset, out, want):
+    for _ in range(3):
+        reset()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
+def test_o_proj_without_workspace_is_captured_cold():
+    """The first call of its size, without a workspace, under capture: nothing is allocated then, so it does not split k."""
+    rows, adim, hid = 1000, 16384, 5120
+    announce(f"o_proj without a workspace captured cold: {rows} rows {adim}->{hid}")
+    plan = gemm_plan(rows, adim, (hid,))
+    assert plan.ks > 1 and plan.bytes > 48 << 20, plan  # more than any other test leaves in the library's buffer
+    g = torch.Generator(device=DEV).manual_seed(95)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    attn, w, hidden = rnd(rows, adim), rnd(hid, adim) * adim ** -0.5, rnd(rows, hid)
+    h, s = hidden.clone(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        K.o_proj_residual(0, attn, w, h, stream=s)
+    y = (attn.float() @ w.float().t()).bfloat16().float()
+    ref = hidden.float() + y
+    graph.replay()
+    torch.cuda.synchronize()
+    # the product's bf16 rounding may be its neighbour (another order of the sum), then the sum's rounding
+    ulp = lambda x: torch.exp2(torch.floor(torch.log2(x.abs().clamp_min(2.0 ** -100))) - 7)
+    assert bool(((h.float() - ref).abs() <= ulp(y) + ulp(ref) + 1e-6).all())
+    want = h.clone()
+    K.o_proj_residual(0, attn, w, hidden.clone())  # eager: now the library's buffer is there
+    replays_equal(graph, lambda: h.copy_(hidden), h, want)
+    # and a call captured while it is there does not hold on to it
+    graph2 = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph2, stream=s):
+        K.o_proj_residual(0, attn, w, h, stream=s)
+    replays_equal(graph2, lambda: h.copy_(hidden), h, want)
+
+
+def test_prefill_without_workspace_is_captured_behind_a_longer_one():
+    """A long chunk first, which is not split and leaves its staging's buffer; then a short one of as many keys, without a
+    workspace, under capture: it fits that buffer as it is."""
+    Hq, Hkv, D, rot, L, S = 16, 4, 256, 64, 30000, 64
+    announce("prefill without a workspace captured behind a longer one")
+    g = torch.Generator(device=DEV).manual_seed(96)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, L, 1.0e7))
+    qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
+    k0, v0 = rnd(1, Hkv, L, D), rnd(1, Hkv, L, D)
+    cache = K.KvCache(k0.clone(), v0.clone())
+    shape = dict(q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot)
+    s = torch.cuda.Stream()
+
+    def chunk(rows):
+        x = (rnd(rows, Hq * 2 * D), rnd(rows, Hkv * D), rnd(rows, Hkv * D))
+        out = torch.zeros(rows, Hq * D, dtype=torch.bfloat16, device=DEV)
+        return out, lambda **kw_: K.fused_prefill(0, *x, qw, kw, cos, sin, cache, out, chunk_start=L - rows, **kw_, **shape)
+
+    chunk(2100)[1](stream=s)
+    out, call = chunk(S)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call(stream=s)
+    graph.replay()
+    torch.cuda.synchronize()
+    want = out.clone()
+    # as a workspace with room for the staging alone
+    call(workspace=torch.zeros(Hkv * D * ((L + 63) // 64 * 64) * 2, dtype=torch.uint8, device=DEV))
+    torch.cuda.synchronize()
+    d = (out.float() - want.float()).abs()
+    assert d.max().item() <= 2e-2 and d.mean().item() <= 2e-3  # (split or not, whichever the capture found room for)
+    replays_equal(graph, out.zero_, out, want)
