@@ -43,7 +43,7 @@ GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch, size_t room)
     GemmPlan best;
     best.us = 1e30;
     if (k <= 0 || k % 8 != 0) return best;  // not a tiled product
-    const int KT = (k + 63) / 64;
+    const int KT_steps = (k + 63) / 64;
     double nsum = 0;
     for (int s = 0; s < nseg; ++s) nsum += n[s];
     const double hbm = 2.0 * batch * (nsum * k + static_cast<double>(m) * k + m * nsum) / 5.64e6;
@@ -62,10 +62,16 @@ GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch, size_t room)
         for (int s = 0; s < nseg; ++s) nt += (n[s] + c.bn - 1) / c.bn;
         const int64_t tiles = nt * ((m + c.bm - 1) / c.bm) * batch;
         const int64_t tail = tiles > kPlanCus ? tiles % kPlanCus : 0;
+        // Rows of a and w that do not begin on 64 bytes: the copies, which set the
+        // pace of the smaller tiles, straddle cache lines.  33 products of k % 32 != 0
+        // took 1.19 times these tiles' estimate and 1.07 times the 256 x 256 ones' (5977
+        // rows, 3112 -> 7184: 321 us in 256 x 128 tiles, 291 in 256 x 256; the other way
+        // round 1134 rows, 6152 -> 20528: 349 and 366).
+        const double KT = KT_steps * (c.bn != 256 && k % 32 != 0 ? 1.12 : 1.0);
         if (c.bn == 256) {
             // the last partial round in two halves of k where that is possible, whole
             // where the workspace has no room for it
-            if (batch == 1 && tail > 0 && 2 * tail <= kPlanCus && KT >= 4 && gemm_tail_bytes(static_cast<int>(tail)) <= room)
+            if (batch == 1 && tail > 0 && 2 * tail <= kPlanCus && KT_steps >= 4 && gemm_tail_bytes(static_cast<int>(tail)) <= room)
                 take(c, 1, 0, tail, rounds_us(c, tiles - tail, KT) + rounds_us(c, 2 * tail, 0.5 * KT) + 7.5, 1.0);
             else
                 take(c, 1, 0, 0, rounds_us(c, tiles, KT), 1.0);
@@ -77,10 +83,10 @@ GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch, size_t room)
         if (batch > 1) continue;
         for (int all = 1; all >= 0; --all) {
             const int64_t split = all ? tiles : tail;
-            for (int ks = 2; ks <= (all ? 16 : 8) && split > 0 && KT / ks >= 3 && split * ks <= (all ? 1600 : 600); ++ks) {
-                const int kper = (KT + ks - 1) / ks, kk = (KT + kper - 1) / kper;
+            for (int ks = 2; ks <= (all ? 16 : 8) && split > 0 && KT_steps / ks >= 3 && split * ks <= (all ? 1600 : 600); ++ks) {
+                const int kper = (KT_steps + ks - 1) / ks, kk = (KT_steps + kper - 1) / kper;
                 const double kb = c.bm * c.bn * 4.0 / 1024.0;  // one slice's partials
-                double t = rounds_us(c, split * kk, kper) + 1.4 + 0.0212 * kk * kb + split * kk * kb * 2048.0 / 11.6e6;
+                double t = rounds_us(c, split * kk, kper * KT / KT_steps) + 1.4 + 0.0212 * kk * kb + split * kk * kb * 2048.0 / 11.6e6;
                 if (!all) t += rounds_us(c, tiles - split, KT);
                 take(c, ks, split, 0, t, 1.02 * 1.04);
             }
