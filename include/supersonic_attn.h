@@ -154,9 +154,9 @@ int supersonic_qwen35_hip_split_qgate(
  * rhs [batch, n, k], out [batch, m, n], bf16 only (the projections, o_proj
  * included, of prefill_engine.rs:356-414).  Replaces
  * kernels/full_attention_bridge_4b.cpp:3683-3704 (kernel full_attention_4b.hip:2513-2575),
- * bound at prefill_ffi.rs:782-792.  m <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M) and at
- * most one 16-column block a CU: HBM-streaming MFMA kernel; otherwise the
- * hand-written tiled MFMA GEMM (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt).
+ * bound at prefill_ffi.rs:782-792.  m <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M) with at
+ * most one 16-column block a CU, or more where that is estimated the faster:
+ * HBM-streaming MFMA kernel; otherwise the hand-written tiled MFMA GEMM (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt).
  * Status: 272 bad dtype, 270 launch, 271 sync. */
 int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(
     int dtype, size_t device_ordinal, size_t batch_elems, int m, int n, int k,
@@ -347,9 +347,10 @@ int supersonic_attn_gfx950_mixed(
  * the megakernel's input norm and projections (full_attention_4b.hip:4942-4967,
  * :5019-5101) and rms_norm_rows_model + matmul_proj of prefill_engine.rs:1951-2117.
  * A norm kernel writes the normed rows once (workspace), then rows <= 12
- * (SUPERSONIC_PROJ_SKINNY_MAX_M) with q/kv_out_dim % 16 == 0 and at most one
- * 16-column block a CU take one weight-streaming launch over the three
- * matrices; otherwise one launch of the hand-written MFMA GEMM over the three matrices as column segments
+ * (SUPERSONIC_PROJ_SKINNY_MAX_M; setting it, to whatever value, keeps up to that
+ * many rows on the streaming kernels) with q/kv_out_dim % 16 == 0 and at most one
+ * 16-column block a CU, or more where that is estimated the faster, take one
+ * weight-streaming launch over the three matrices; otherwise one launch of the hand-written MFMA GEMM over the three matrices as column segments
  * (SUPERSONIC_PROJ_GEMM=hipblaslt: one hipBLASLt GEMM per matrix instead).
  * hidden_dim % 8 == 0.  Asynchronous on `stream`.  workspace: caller device
  * memory of at least supersonic_attn_gfx950_qkv_proj_workspace_size() bytes,
@@ -379,7 +380,8 @@ int supersonic_attn_gfx950_qkv_proj(
  * of row r at slot positions[r] of sequence r.  The outputs feed
  * supersonic_attn_gfx950_decode_attend (q, gate, kv_lens = positions + 1).
  * Rows <= 12 with rows * hidden_dim <= 32768, head_dim 128/256 and at most one
- * 16-column block a CU: one weight-streaming launch whose epilogue normalises
+ * 16-column block a CU (or more where that is estimated the faster): one
+ * weight-streaming launch whose epilogue normalises
  * and rotates each head as its last column block completes; otherwise the
  * projections, then one wave per (row, head).  workspace: at least
  * supersonic_attn_gfx950_qkv_proj_rope_workspace_size() bytes, zero-filled
@@ -437,7 +439,8 @@ int supersonic_attn_gfx950_decode_layer(
  * (hidden_dtype 1, the megakernel's hidden_f32).  Replaces the megakernel's
  * step G (full_attention_4b.hip:5481-5577) and matmul_proj + residual_add of
  * prefill_engine.rs:2308-2334.  rows <= 12 (SUPERSONIC_PROJ_SKINNY_MAX_M, at most 64) with attn_dim % 8 == 0 and at
- * most one 16-column block a CU: one HBM-streaming MFMA kernel with the residual fused; otherwise the hand-written
+ * most one 16-column block a CU (or more where that is estimated the faster): one
+ * HBM-streaming MFMA kernel with the residual fused; otherwise the hand-written
  * MFMA GEMM with the residual add in its epilogue, in place
  * (SUPERSONIC_PROJ_GEMM=hipblaslt: hipBLASLt and a residual kernel).
  * Asynchronous on `stream`.  workspace: split-k partials and arrival counters,

@@ -367,28 +367,11 @@ inline unsigned stride_blocks(size_t n) {
 }
 
 // Largest row count the streaming kernel takes (SUPERSONIC_PROJ_SKINNY_MAX_M,
-// default 12, at most 64, read per call); more rows go to hipBLASLt.
+// default 12, at most 64, read per call); more rows go to the tiled GEMM.
 int skinny_max_m() {
     const char* e = getenv("SUPERSONIC_PROJ_SKINNY_MAX_M");
     const int x = e ? atoi(e) : kSkinnyDefaultM;
     return x < 0 ? 0 : (x > kSkinnyMaxM ? kSkinnyMaxM : x);
-}
-
-// Whether the streaming kernels' few rows go to them rather than to the tiled
-// GEMM: with at most one 16-column block a CU.  More blocks come in uneven
-// rounds, and short rows of W leave a wave too few loads in flight (one
-// MI355X, 8 rows: o_proj 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled;
-// norm + Q/K/V 1024 -> 5120, 320 blocks, 13.0 against 11.4; 2048 -> 9216, 576
-// blocks, 20.0 against 12.0; 4096 -> 10240, 640 blocks, 23.2 against 19.7).  So
-// too with the QK norm and RoPE in the streaming kernel's epilogue, which the
-// tiled GEMM leaves to a kernel of their own (1 / 8 / 12 rows: 4096 -> 10240
-// 25.7 / 27.6 / 35.5 against 24.3 / 25.4 / 26.0; 2048 -> 9216 21.4 / 23.0 / 24.1
-// against 17.4 / 18.2 / 18.3; 1024 -> 5120 15.7 / 16.5 / 17.7 against 14.7 /
-// 14.6 / 15.1).
-// A row limit or a GEMM in the environment asks for the streaming kernels.
-bool stream_columns(int dev, int64_t ncb) {
-    const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
-    return ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM");
 }
 
 bool skinny_fits(int m, int k, const void* x, const void* w) {
@@ -564,6 +547,29 @@ struct GemmCall {
     GemmPlan plan;
     uint8_t* ws = nullptr;
 };
+// Whether few rows that the streaming kernels can take (fits) go to them
+// rather than to the tiled GEMM: always with at most one 16-column block a CU (8
+// rows of 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled), else by the two
+// estimates.  More blocks come in uneven rounds, and short rows of W leave a wave
+// too few loads in flight: 8 rows, 1024 -> 320 blocks 10.7 against 6.3 tiled,
+// 2048 -> 576 15.1 against 10.0, 4096 -> 640 18.1 against 17.0; but long rows of
+// W in full rounds are streamed faster: 1 row, 8192 -> 1024 blocks 41.1 against
+// 50.3, 12288 -> 512 30.9 against 43.4, 4096 -> 512 14.2 against 15.8.  Over 968
+// such calls the choice is 0.5% slower than the better one on average, 14% slower
+// than streaming at worst.  rope: the streaming kernel norms and rotates the heads
+// in its epilogue (3 us and 1.1 a round more), the tiled GEMM leaves them to a
+// kernel of their own (5.5).
+// A row limit or a GEMM in the environment asks for the streaming kernels.
+bool rows_stream(int dev, int m, int k, int nseg, const int* n, int64_t ncb, bool fits, bool rope, GemmCall* call) {
+    if (!fits) return false;
+    const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
+    if (k <= 0 || ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM")) return true;
+    call->plan = gemm_plan(m, k, nseg, n);
+    const double stream = stream_us(k, ncb, lds_path(dev, m, k, 1, static_cast<int>(ncb)));
+    return rope ? stream + 3.0 + 1.1 * static_cast<double>((ncb + 255) / 256 - 2) <= call->plan.us + 5.5
+                : stream <= call->plan.us;
+}
+
 // A tail split's region that the caller's is too small for is an error (a
 // status); a k split without room leaves the call to the best plan that fits.
 // Nor does a call without a workspace split k while `st` is captured: the
@@ -571,7 +577,7 @@ struct GemmCall {
 // keep its address when a larger call moves it.
 int plan_gemm(int dev, hipStream_t st, int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, GemmCall* call) {
     GemmPlan& plan = call->plan;
-    plan = gemm_plan(m, k, nseg, n);
+    if (plan.us == 0) plan = gemm_plan(m, k, nseg, n);  // (rows_stream may have made it)
     if (plan.bytes == 0) return 0;
     if (ws) {
         if (plan.bytes > ws_bytes) {
@@ -696,8 +702,9 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
     ScopedDevice scoped(dev);
     if (batch_elems > 0 && m > 0 && n > 0) {
         const int batch = static_cast<int>(batch_elems);
-        if (k <= 0 || (skinny_fits(m, k, lhs, rhs) &&
-                       (batch > 1 || stream_columns(dev, (n + kSkinnyCols - 1) / kSkinnyCols)))) {
+        GemmCall call;
+        const bool fits = k <= 0 || skinny_fits(m, k, lhs, rhs);
+        if (batch > 1 ? fits : rows_stream(dev, m, k, 1, &n, (n + kSkinnyCols - 1) / kSkinnyCols, fits, false, &call)) {
             SkinnyParams p{};
             p.x = static_cast<const uint16_t*>(lhs);
             one_segment(p, rhs, out, n);
@@ -729,7 +736,6 @@ extern "C" int supersonic_qwen35_4b_hip_matmul_rhs_transposed_tiled(int dtype, s
             g.w_bs = static_cast<int64_t>(n) * k;
             g.o_bs = static_cast<int64_t>(m) * n;
             if (batch == 1) {
-                GemmCall call;
                 if (plan_gemm(dev, nullptr, m, k, 1, &n, nullptr, 0, &call) != 0) return 270;
                 g.plan = call.plan;
                 g.ws = call.ws;
@@ -828,7 +834,8 @@ extern "C" int supersonic_attn_gfx950_o_proj_residual(size_t device_ordinal, voi
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
-    if (skinny_fits(m, k, attn, o_proj_w) && stream_columns(dev, (n + kSkinnyCols - 1) / kSkinnyCols)) {
+    GemmCall call;
+    if (rows_stream(dev, m, k, 1, &n, (n + kSkinnyCols - 1) / kSkinnyCols, skinny_fits(m, k, attn, o_proj_w), false, &call)) {
         SkinnyParams p{};
         p.x = static_cast<const uint16_t*>(attn);
         one_segment(p, o_proj_w, hidden, n);
@@ -847,7 +854,6 @@ extern "C" int supersonic_attn_gfx950_o_proj_residual(size_t device_ordinal, voi
         if (k == 0) return 0;  // nothing to add
         const void* w1[1] = {o_proj_w};
         void* o1[1] = {hidden};
-        GemmCall call;
         if (const int rc = plan_gemm(dev, st, m, k, 1, &n, ws, workspace_bytes, &call)) return rc;
         if (gemm_segments(st, m, k, attn, 1, w1, o1, &n, f32 ? kGemmResidualF32 : kGemmResidualBf16, call) != 0)
             return SUPERSONIC_ERR_LAUNCH;
@@ -923,9 +929,10 @@ extern "C" int supersonic_attn_gfx950_qkv_proj(size_t device_ordinal, void* stre
     // the three matrices as one column space of the weight-streaming kernel, or
     // as column segments of one GEMM
     const int ns[3] = {nq, nkv, nkv};
-    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
-                        nkv % kSkinnyCols == 0 && stream_columns(dev, (nq + 2 * nkv) / kSkinnyCols);
     GemmCall call;
+    const bool skinny = rows_stream(dev, m, k, 3, ns, (nq + 2 * nkv) / kSkinnyCols,
+                                    skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
+                                        nkv % kSkinnyCols == 0, false, &call);
     if (!skinny && !use_hipblaslt())
         if (const int rc = plan_gemm(dev, st, m, k, 3, ns, rest, rest_bytes, &call)) return rc;
     unsigned* clear = nullptr;
@@ -1076,17 +1083,20 @@ extern "C" int supersonic_attn_gfx950_qkv_proj_rope(
     uint8_t* pws = reinterpret_cast<uint8_t*>(vr) + align256(static_cast<size_t>(m) * nkv * 2);
     const size_t pws_bytes = (workspace ? workspace_bytes : need) - static_cast<size_t>(pws - ws);  // need reaches up to pws
     const int ncb = (nq + 2 * nkv) / kSkinnyCols;
-    const bool fused = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
-                       Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4) && stream_columns(dev, ncb);
-    const bool skinny = skinny_fits(m, k, normed, q_proj_w) && aligned && nq % kSkinnyCols == 0 &&
-                        nkv % kSkinnyCols == 0 && stream_columns(dev, ncb);
     const int ns[3] = {nq, nkv, nkv};
-    uint8_t* const own = workspace ? pws : nullptr;
     GemmCall call;
+    const bool one_launch = aligned && (D == 128 || D == 256) && lds_path(dev, m, k, 1, ncb) && m <= skinny_max_m() &&
+                            Hq + Hkv <= static_cast<int>(kRopeCounterBytes / 4);
+    const bool streams = rows_stream(dev, m, k, 3, ns, ncb,
+                                     one_launch || (skinny_fits(m, k, normed, q_proj_w) && aligned &&
+                                                    nq % kSkinnyCols == 0 && nkv % kSkinnyCols == 0), one_launch, &call);
+    const bool fused = streams && one_launch;
+    const bool skinny = streams && !one_launch;
+    uint8_t* const own = workspace ? pws : nullptr;
     if (!fused && !skinny && !use_hipblaslt())
         if (const int rc = plan_gemm(dev, st, m, k, 3, ns, own, pws_bytes, &call)) return rc;
     unsigned* clear = nullptr;
-    const int n_clear = moving_counts(own, call, skinny && !fused ? stream_counts(dev, m, k, ncb) : 0, &clear);
+    const int n_clear = moving_counts(own, call, skinny ? stream_counts(dev, m, k, ncb) : 0, &clear);
     const ProfileEvents ev = take_profile_events();
     if (ev.before) (void)hipEventRecord(ev.before, st);
     {

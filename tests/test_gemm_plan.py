@@ -3,7 +3,7 @@ import random
 
 import pytest
 
-from plan_util import gemm_plan
+from plan_util import gemm_plan, stream_us
 
 
 def test_plans_fit_their_room_and_the_kernels():
@@ -37,3 +37,14 @@ def test_unaligned_rows_keep_the_large_tiles(m, k, n):
                                    (3932, 1664, (4592, 592, 592)), (890, 4008, (2328,)), (2040, 9520, (856,))])
 def test_smaller_tiles_where_they_were_faster(m, k, n):
     assert gemm_plan(m, k, n).bn < 256
+
+
+# rows, k, 16-column blocks, us streamed, us tiled (output projections, one MI355X): the estimates take the faster
+@pytest.mark.parametrize("m,k,ncb,streamed,tiled", [
+    (1, 12288, 512, 30.9, 43.4), (1, 8192, 512, 22.7, 28.2), (4, 8192, 512, 23.5, 28.2), (1, 8192, 1024, 41.1, 50.3),
+    (4, 12288, 512, 35.4, 43.5), (1, 4096, 512, 14.2, 15.8), (1, 4096, 1280, 28.2, 33.5), (8, 6144, 512, 22.3, 18.6),
+    (1, 512, 1792, 30.1, 7.1), (8, 1024, 320, 10.7, 6.3), (8, 2048, 576, 15.1, 10.0), (8, 4096, 640, 18.1, 17.0),
+    (8, 4096, 272, 11.7, 10.1), (12, 8192, 640, 41.0, 29.2), (1, 16384, 800, 109.9, 71.7), (1, 5120, 1280, 47.0, 40.3),
+])
+def test_few_rows_take_the_faster_kernel(m, k, ncb, streamed, tiled):
+    assert (stream_us(m, k, ncb) <= gemm_plan(m, k, (16 * ncb,)).us) == (streamed < tiled)
