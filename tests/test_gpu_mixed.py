@@ -253,3 +253,50 @@ def test_mixed_step_without_decodes_leaves_their_counters():
         K.fused_mixed(0, qw, kw, cos, sin, workspace=ws, **part, **shape)
         torch.cuda.synchronize()
         check(dec["out"], ref.float().cpu(), TOL_BF16, "decodes after a step without them")
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_mixed_key_split_chunk_paged(fp8):
+    """The key pieces of a mixed step's chunk in one block-paged cache that the decodes share, bf16 and fp8."""
+    S, start, batch, Hq, Hkv, D, rot, ps = 60, 2000, 3, 8, 2, 256, 64, 64
+    announce(f"mixed key split, one paged cache, fp8={fp8}")
+    g = torch.Generator(device=DEV).manual_seed(94)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, start + S + 1, 1.0e7))
+    qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
+    lens = [100, 700, 1400]
+    pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    per = [-(-n // ps) for n in [start + S] + [n + 1 for n in lens]]
+    order = torch.randperm(sum(per), generator=torch.Generator().manual_seed(5)).tolist()
+    table = torch.zeros(len(per), max(per), dtype=torch.int32)
+    for i, n in enumerate(per):
+        table[i, :n] = torch.tensor([order.pop() for _ in range(n)], dtype=torch.int32)
+    k, v = rnd(sum(per), Hkv, ps, D), rnd(sum(per), Hkv, ps, D)
+    if fp8:
+        (kq, ks), (vq, vs) = fp8_rows(k.float().cpu()), fp8_rows(v.float().cpu())
+        pool = [t.to(DEV) for t in (kq, vq, ks, vs)]
+    else:
+        pool = [k, v]
+    table = table.to(DEV)
+    views = lambda: (lambda p: (K.KvCache(*p, block_table=table[:1].contiguous()), K.KvCache(*p, block_table=table[1:].contiguous()), p))(
+        [t.clone() for t in pool])
+    xc = [rnd(S, Hq * 2 * D), rnd(S, Hkv * D), rnd(S, Hkv * D)]
+    xd = [rnd(batch, Hq * 2 * D), rnd(batch, Hkv * D), rnd(batch, Hkv * D)]
+    shape = dict(q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot)
+    nan = lambda n: torch.full((n, Hq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    mine, theirs, one = views()
+    ref_c, ref_d = nan(S), nan(batch)
+    staging = Hkv * D * ((start + S + 63) // 64 * 64) * (4 if fp8 else 2)
+    K.fused_prefill(0, *xc, qw, kw, cos, sin, mine, ref_c, chunk_start=start,
+                    workspace=torch.zeros(staging, dtype=torch.uint8, device=DEV), **shape)  # unsplit
+    K.fused_decode(0, *xd, qw, kw, cos, sin, pos, theirs, ref_d, max_kv_len=max(lens) + 1, **shape)
+    mine, theirs, two = views()
+    chunk = dict(zip(("q_proj", "k_new", "v_new"), xc), cache=mine, out=nan(S), chunk_start=start)
+    dec = dict(zip(("q_proj", "k_new", "v_new"), xd), cache=theirs, out=nan(batch), positions=pos, max_kv_len=max(lens) + 1)
+    ws = torch.zeros(K.mixed_workspace_size(fp8, Hq, Hkv, D, chunk, dec), dtype=torch.uint8, device=DEV)
+    K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, decode=dec, workspace=ws, **shape)
+    torch.cuda.synchronize()
+    check(chunk["out"], ref_c.float().cpu(), TOL_BF16, "mixed split chunk, paged")
+    assert not torch.equal(chunk["out"], ref_c), "the chunk ran unsplit"
+    check(dec["out"], ref_d.float().cpu(), TOL_BF16, "mixed split decode, paged")
+    assert all(torch.equal(a, b) for a, b in zip(one, two))

@@ -178,6 +178,64 @@ def test_fused_prefill_key_split(S, Hq, Hkv, D, rot, start):
     check(outs[0], outs[2].float().cpu(), TOL_BF16, "split against whole")
 
 
+def cache_of(k, v, fp8, page, seed):
+    """[Hkv, cap, D] rows as one sequence's cache: bf16 or e4m3 codes with scales, contiguous or in shuffled pages."""
+    parts = [k, v]
+    if fp8:
+        (kq, ks), (vq, vs) = fp8_rows(k), fp8_rows(v)
+        parts = [kq, vq, ks, vs]
+    bt = None
+    if page:
+        n = -(-k.shape[1] // page)
+        perm = torch.randperm(n + 3, generator=gen(seed))[:n].to(torch.int32)
+        pools = []
+        for t in parts:
+            pool = torch.zeros((n + 3, t.shape[0], page) + tuple(t.shape[2:]), dtype=t.dtype)
+            for i in range(n):
+                rows = t[:, i * page:(i + 1) * page]
+                pool[int(perm[i]), :, :rows.shape[1]] = rows
+            pools.append(pool)
+        parts, bt = pools, perm.reshape(1, -1).to(DEV)
+    else:
+        parts = [t[None] for t in parts]
+    return K.KvCache(*(t.to(DEV) for t in parts), **({"block_table": bt} if page else {}))
+
+
+# Pieces that begin inside the sequence, where a paged cache's tiles lie in other pages and an fp8 cache's keys come from
+# the dequantised rows.
+@pytest.mark.parametrize("fp8,page", [(False, 64), (True, None), (True, 64), (False, 128)])
+@pytest.mark.parametrize("S,Hq,Hkv,D,rot,start", [(60, 16, 2, 256, 64, 2001), (130, 8, 4, 128, 32, 1531),
+                                                  (1, 16, 4, 256, 64, 3000)])
+def test_fused_prefill_key_split_paged_and_fp8(S, Hq, Hkv, D, rot, start, fp8, page):
+    announce(f"prefill key split S={S} {Hq}/{Hkv} D={D} start={start} fp8={fp8} page={page}")
+    c = fused_case(76, S, Hq, Hkv, D, rot, start)
+    rows = lambda t: torch.cat([t, torch.zeros(Hkv, S, D, dtype=t.dtype)], dim=1)
+    size = K.prefill_workspace_size(fp8, Hkv, D, S, start)
+    plain = Hkv * D * ((start + S + 63) // 64 * 64) * (4 if fp8 else 2)  # the staging alone: no room for the pieces
+    assert size > plain
+    outs, caches = [], []
+    for n in (size, plain):
+        cache = cache_of(rows(c["prefix_k"]), rows(c["prefix_v"]), fp8, page, 11)
+        out = torch.full((S, Hq * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.fused_prefill(0, *(c[k].to(DEV) for k in ("q_proj", "k_new", "v_new", "qw", "kw", "cos", "sin")), cache, out,
+                        q_heads=Hq, kv_heads=Hkv, head_dim=D, rotary_dim=rot, chunk_start=start,
+                        workspace=torch.full((n,), 255, dtype=torch.uint8, device=DEV))
+        torch.cuda.synchronize()
+        outs.append(out)
+        caches.append(cache)
+    pk, pv = c["prefix_k"], c["prefix_v"]
+    if fp8:
+        deq = lambda q, sc: (torch.from_numpy(fp8_codec.decode(q.numpy())) * sc[..., None]).bfloat16().float()
+        pk, pv = deq(*fp8_rows(pk)), deq(*fp8_rows(pv))
+    ref, _, _ = O.prefill_layer(c["shape"], c["q_proj"], c["k_new"], c["v_new"], c["qw"], c["kw"], c["cos"], c["sin"],
+                                start, pk, pv)
+    for out in outs:
+        check(out, ref, TOL_BF16, "prefill key split")
+    assert not torch.equal(*outs), "the chunk ran unsplit both times"
+    check(outs[0], outs[1].float().cpu(), TOL_BF16, "split against whole")
+    assert torch.equal(caches[0].k, caches[1].k) and torch.equal(caches[0].v, caches[1].v)
+
+
 @pytest.mark.parametrize("dtype", [K.ScalarType.BF16, K.ScalarType.F16])
 @pytest.mark.parametrize("B,Hq,Hkv,S,L,off,D", [(2, 8, 2, 65, 2065, 2000, 128), (1, 4, 4, 130, 1500, 2000, 256),
                                                 (3, 6, 3, 20, 3020, 3000, 64), (1, 8, 1, 100, 900, 850, 256)])

@@ -67,10 +67,8 @@ def test_matmul_matches_oracle(batch, m, n, k):
 
 
 def test_matmul_tail_split():
-    """More tiles than CUs with a short last round: the tail tiles run as two
-    half-k workgroups whose fp32 partials meet through the workspace.  Two calls
-    in a row (the second of another shape and tail) check that each call leaves
-    the hand-over flags cleared; the partial last k-tile sits in the second half."""
+    """More 256 x 256 tiles than CUs with a short last round: 128 x 128 tiles, the
+    partial last k-tile among them.  (test_matmul_tail_split_planned has the shapes whose last round runs in halves.)"""
     for seed, (m, n, k) in enumerate([(4096, 4608, 512), (4100, 4608, 520), (4096, 4608, 512)]):
         announce(f"matmul tail split m={m} n={n} k={k}")
         g = gen(90 + seed)
@@ -463,7 +461,7 @@ def test_qkv_proj_rope_many_columns(rows, hid, Hq, Hkv):
 
 
 def test_projections_share_a_workspace_over_row_counts():
-    """One o_proj workspace for calls of different row counts, a tail split among them."""
+    """One o_proj workspace for calls of different row counts, without a split."""
     announce("o_proj one workspace, many row counts")
     g = gen(93)
     hid, adim = 4608, 512
@@ -530,10 +528,111 @@ def test_qkv_projections_share_a_workspace_over_row_counts(counts, hid, Hq, Hkv,
             assert_ulps(o.float().cpu(), ref, 2 * ulp(big) + 2.0 ** -7, f"qkv shared ws rows={r}")
 
 
+# Every tile whole, split along k, and with the last round's tiles split (halved: the 256 x 256 tail), at its cheapest.
+PLANNED = {
+    "32x64 split": (16, 1280, 256), "64x64 split": (257, 1024, 256), "128x64 split": (601, 1280, 256),
+    "128x128 split": (129, 5888, 4096), "128x128 split tail": (2600, 1792, 3080), "256x128 split": (1000, 4864, 2056),
+    "256x128 split tail": (3000, 2560, 3080), "256x256 halved tail": (8200, 512, 4608),
+    "256x256 whole": (2600, 256, 3080), "256x128 whole": (1300, 512, 3080), "128x128 whole": (1300, 256, 1536),
+}
+
+
+def planned_path(rows, adim, hid):
+    p = gemm_plan(rows, adim, (hid,))
+    tiles = -(-rows // p.bm) * -(-hid // p.bn)
+    how = "halved tail" if p.tail else "whole" if p.ks == 1 else "split" if p.split_tiles == tiles else "split tail"
+    return f"{p.bm}x{p.bn} {how}"
+
+
+@pytest.mark.parametrize("path", list(PLANNED))
+def test_o_proj_planned_paths(path):
+    rows, adim, hid = PLANNED[path]
+    announce(f"o_proj {path}: {rows} rows {adim}->{hid}")
+    assert planned_path(rows, adim, hid) == path
+    g = gen(97)
+    attn = O.randn_bf16(g, rows, adim)
+    w = O.randn_bf16(g, hid, adim, std=adim ** -0.5)
+    hidden = O.randn_bf16(g, rows, hid)
+    ref = O.o_proj_residual(attn.float(), w, hidden)
+    slack = 2 * ulp(torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())) + 1e-6
+    ad, wd = attn.to(DEV), w.to(DEV)
+    ws = torch.zeros(K.o_proj_workspace_size(rows, hid, adim), dtype=torch.uint8, device=DEV)
+    got = []
+    for _ in range(2):  # twice: the counts are left as they were
+        h = hidden.to(DEV)
+        K.o_proj_residual(0, ad, wd, h, workspace=ws)
+        torch.cuda.synchronize()
+        assert_ulps(h.float().cpu(), ref, slack, path)
+        got.append(h)
+    assert torch.equal(*got) and K.wait_status() == 0
+
+
+def test_matmul_tail_split_planned():
+    """The drop-in's tail hand-over (test_matmul_tail_split's shapes take smaller tiles now), twice around another tail."""
+    for seed, (m, n, k) in enumerate([(8200, 4608, 512), (8200, 4608, 264), (8200, 4608, 512)]):
+        announce(f"matmul halved tail m={m} n={n} k={k}")
+        assert planned_path(m, k, n) == "256x256 halved tail"
+        g = gen(98 + seed)
+        lhs, rhs = O.randn_bf16(g, 1, m, k), O.randn_bf16(g, 1, n, k, std=k ** -0.5)
+        out = dropin_matmul(lhs, rhs)
+        ref = O.matmul_rhs_transposed(lhs, rhs)
+        assert_ulps(out, ref, ulp(ref) + 1e-6, f"matmul halved tail {m}x{n}x{k}")
+
+
+def test_o_proj_shapes_share_a_workspace():
+    """One o_proj workspace for calls that split in every way: streamed over two k slices, tiles over slices of k, a halved
+    tail, the partials of each lying where the others' were."""
+    announce("o_proj one workspace, every split")
+    calls = [("64x64 split",), ("256x256 halved tail",), (8, 4096, 1024), ("128x128 split",), ("256x128 split tail",),
+             ("256x256 halved tail",), (8, 4096, 1024), ("64x64 split",)]
+    calls = [PLANNED[c[0]] if len(c) == 1 else c for c in calls]
+    for c, path in ((calls[0], "64x64 split"), (calls[1], "256x256 halved tail")):
+        assert planned_path(*c) == path
+    ws = torch.zeros(max(K.o_proj_workspace_size(r, h, a) for r, a, h in calls), dtype=torch.uint8, device=DEV)
+    g = gen(99)
+    for r, a, h in calls:
+        attn, w, hidden = O.randn_bf16(g, r, a), O.randn_bf16(g, h, a, std=a ** -0.5), O.randn_bf16(g, r, h)
+        hd = hidden.to(DEV)
+        K.o_proj_residual(0, attn.to(DEV), w.to(DEV), hd, workspace=ws)
+        torch.cuda.synchronize()
+        ref = O.o_proj_residual(attn.float(), w, hidden)
+        big = torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())
+        assert_ulps(hd.float().cpu(), ref, 2 * ulp(big) + 1e-6, f"o_proj shared ws {r} rows {a}->{h}")
+    assert K.wait_status() == 0
+
+
+def test_o_proj_tail_expired_handover_is_reported(monkeypatch):
+    """As test_gemm_tail_expired_handover_is_reported, where nothing clears the counts ahead of the product: the host
+    presets one tile's consumed count ahead, and a short poll bound lets its wait give up."""
+    rows, adim, hid = PLANNED["256x256 halved tail"]
+    assert planned_path(rows, adim, hid) == "256x256 halved tail"
+    g = gen(100)
+    attn, w, hidden = O.randn_bf16(g, rows, adim), O.randn_bf16(g, hid, adim, std=adim ** -0.5), O.randn_bf16(g, rows, hid)
+    ws = torch.zeros(K.o_proj_workspace_size(rows, hid, adim), dtype=torch.uint8, device=DEV)
+    counts = ws[:8192].view(torch.int32)
+    counts[1] = 1  # tile 0: consumed 1, produced 0
+    ad, wd = attn.to(DEV), w.to(DEV)
+    assert K.wait_status() == 0
+    monkeypatch.setenv("SUPERSONIC_WAIT_POLLS", "256")
+    announce("o_proj tail hand-over held (forced give-up)")
+    K.o_proj_residual(0, ad, wd, hidden.to(DEV), workspace=ws)
+    assert K.wait_status() & K.WAIT_GEMM_TAIL
+    monkeypatch.delenv("SUPERSONIC_WAIT_POLLS")
+    ws.zero_()
+    hd = hidden.to(DEV)
+    K.o_proj_residual(0, ad, wd, hd, workspace=ws)
+    assert K.wait_status() == 0
+    c = counts.cpu().view(-1, 2)
+    assert bool((c[:, 0] == c[:, 1]).all()) and int(c[:, 0].max()) == 1
+    ref = O.o_proj_residual(attn.float(), w, hidden)
+    big = torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())
+    assert_ulps(hd.float().cpu(), ref, 2 * ulp(big) + 1e-6, "o_proj after the forced give-up")
+
+
 def test_gemm_tail_expired_handover_is_reported(monkeypatch):
-    """The host presets one tail tile's consumed count ahead of its produced count,
-    so that tile's second k half never sees its first half, and shortens the
-    poll bound: the wait gives up, the kernel exits normally and the error word
+    """The host shortens the poll bound below the time that a tail tile's first k
+    half takes to arrive (the preset count is cleared ahead of the product): the
+    wait gives up, the kernel exits normally and the error word
     reports it.  A normal call on the re-zeroed workspace is then correct,
     reports nothing and leaves every tile's two counts equal."""
     rows, hid, nq, nkv = 4096, 1024, 8192, 1024
