@@ -555,10 +555,10 @@ struct GemmCall {
 // 2048 -> 576 15.1 against 10.0, 4096 -> 640 18.1 against 17.0; but long rows of
 // W in full rounds are streamed faster: 1 row, 8192 -> 1024 blocks 41.1 against
 // 50.3, 12288 -> 512 30.9 against 43.4, 4096 -> 512 14.2 against 15.8.  Over 968
-// such calls the choice is 0.5% slower than the better one on average, 14% slower
+// such calls the choice is 0.1% slower than the better one on average, 13% slower
 // than streaming at worst.  rope: the streaming kernel norms and rotates the heads
 // in its epilogue (3 us and 1.1 a round more), the tiled GEMM leaves them to a
-// kernel of their own (5.5).
+// kernel of their own (4.4).
 // A row limit or a GEMM in the environment asks for the streaming kernels.
 bool rows_stream(int dev, int m, int k, int nseg, const int* n, int64_t ncb, bool fits, bool rope, GemmCall* call) {
     if (!fits) return false;
@@ -566,7 +566,7 @@ bool rows_stream(int dev, int m, int k, int nseg, const int* n, int64_t ncb, boo
     if (k <= 0 || ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM")) return true;
     call->plan = gemm_plan(m, k, nseg, n);
     const double stream = stream_us(k, ncb, lds_path(dev, m, k, 1, static_cast<int>(ncb)));
-    return rope ? stream + 3.0 + 1.1 * static_cast<double>((ncb + 255) / 256 - 2) <= call->plan.us + 5.5
+    return rope ? stream + 3.0 + 1.1 * static_cast<double>((ncb + 255) / 256 - 2) <= call->plan.us + 4.4
                 : stream <= call->plan.us;
 }
 
