@@ -33,7 +33,8 @@ SSA_HOST_DEVICE inline int64_t ragged_round_chunk(int64_t c) {
 template <typename Items, typename Longest>
 SSA_HOST_DEVICE inline int ragged_chunk(int64_t tot, int Hkv, int target, int min_chunk, bool strict,
                                         const Items& items_of, const Longest& longest) {
-    int64_t c = ragged_round_chunk((tot * Hkv + target - 1) / target);
+    // (far below the bound: tot is what a cache holds)
+    int64_t c = ((tot * Hkv + target - 1) / target + 15) / 16 * 16;
     c = c > min_chunk ? c : min_chunk;
     bool fits = false;
     for (int pass = 0; pass < 5; ++pass) {
