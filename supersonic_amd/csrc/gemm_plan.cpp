@@ -95,18 +95,17 @@ GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch, size_t room)
     return best;
 }
 
-// A constant and a time a round of 256 column blocks: with staged rows 3.9 us
-// and 4.6 more for each load batch of 4096 k after the first, or, past the two
-// rounds that are resident at once, the HBM time of a full round's weights;
-// otherwise in proportion to k.  No less than the
-// weights at the rate that the kernels reach.  Fitted to the output projections of
-// 1 to 12 rows, k 512 to 16384, 272 to 1792 blocks (one MI355X).
-double stream_us(int k, int64_t ncb, bool staged) {
-    const double rounds = static_cast<double>((ncb + 255) / 256);
-    const double round = staged ? std::max(3.9 + 4.6 * ((k + 4095) / 4096 - 1), ncb > 512 ? 0.00118 * k : 0.0)
-                                : 1.0 + 0.00138 * k;
-    const double rate = k > 8192 && ncb > 512 ? (k > 12288 ? 4.6e6 : 5.9e6) : 6.2e6;
-    return std::max(3.0 + rounds * round, 32.0 * static_cast<double>(ncb) * k / rate + 2.0);
+// A constant and a time a round of 256 column blocks.  Staged rows: a time a
+// load batch of 4096 k and a little for the length, or the HBM time of a round's
+// weights, and the staging of the rows; otherwise in proportion to k.  Past k =
+// 12288 more than two rounds take 1.35 times that (1 row, 16384 -> 1024 blocks:
+// 121 us).  Fitted to the output projections of 1 to 12 rows, k 1024 to 12288, 272
+// to 1792 blocks, with weights that come from HBM (copies of them in turn; one
+// MI355X).
+double stream_us(int m, int k, int64_t ncb, bool staged) {
+    const double round = staged ? std::max(3.8 + 4.3 * ((k + 4095) / 4096 - 1) + 0.00027 * k, 0.0013 * k) + 2e-5 * k * (m - 1)
+                                : (0.0016 * k + 0.6) * (1.0 + 0.025 * (m - 8));
+    return 3.0 + static_cast<double>((ncb + 255) / 256) * round * (k > 12288 && ncb > 512 ? 1.35 : 1.0);
 }
 
 }  // namespace ssa

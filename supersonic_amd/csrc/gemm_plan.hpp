@@ -30,8 +30,8 @@ struct GemmPlan {
 // takes more than `room` bytes of workspace.
 GemmPlan gemm_plan(int m, int k, int nseg, const int* n, int batch = 1, size_t room = SIZE_MAX);
 
-// The weight-streaming kernels' time for few rows against ncb 16-column blocks
+// The weight-streaming kernels' time for m <= 12 rows against ncb 16-column blocks
 // of W (staged: the rows fit in LDS, the LDS-staged kernel), as GemmPlan::us.
-double stream_us(int k, int64_t ncb, bool staged);
+double stream_us(int m, int k, int64_t ncb, bool staged);
 
 }  // namespace ssa

@@ -551,21 +551,21 @@ struct GemmCall {
 // rather than to the tiled GEMM: always with at most one 16-column block a CU (8
 // rows of 4096 -> 4096, 256 blocks, 9.7 us against 11.0 tiled), else by the two
 // estimates.  More blocks come in uneven rounds, and short rows of W leave a wave
-// too few loads in flight: 8 rows, 1024 -> 320 blocks 10.7 against 6.3 tiled,
-// 2048 -> 576 15.1 against 10.0, 4096 -> 640 18.1 against 17.0; but long rows of
-// W in full rounds are streamed faster: 1 row, 8192 -> 1024 blocks 41.1 against
-// 50.3, 12288 -> 512 30.9 against 43.4, 4096 -> 512 14.2 against 15.8.  Over 968
-// such calls the choice is 0.1% slower than the better one on average, 13% slower
-// than streaming at worst.  rope: the streaming kernel norms and rotates the heads
-// in its epilogue (3 us and 1.1 a round more), the tiled GEMM leaves them to a
-// kernel of their own (4.4).
+// too few loads in flight: 8 rows, 1024 -> 320 blocks 11.1 us against 6.4 tiled,
+// 2048 -> 576 17.4 against 10.4, 4096 -> 640 20.2 against 16.9; but long rows of
+// W in full rounds are streamed faster: 1 row, 8192 -> 1024 blocks 46.7 against
+// 52.0, 12288 -> 512 36.2 against 44.2, 4096 -> 512 14.5 against 17.0 (weights from
+// HBM).  Over 432 such calls the choice is 0.2% slower than the better one on
+// average and 18% at worst, where it tiles; one that streams was never the
+// slower.  rope: the streaming kernel norms and rotates the heads in its epilogue (3
+// us and 1.1 a round more), the tiled GEMM leaves them to a kernel of their own (4.4).
 // A row limit or a GEMM in the environment asks for the streaming kernels.
 bool rows_stream(int dev, int m, int k, int nseg, const int* n, int64_t ncb, bool fits, bool rope, GemmCall* call) {
     if (!fits) return false;
     const int cus = device_cu_count(dev) > 0 ? device_cu_count(dev) : 256;
     if (k <= 0 || ncb <= cus || getenv("SUPERSONIC_PROJ_SKINNY_MAX_M") || getenv("SUPERSONIC_PROJ_GEMM")) return true;
     call->plan = gemm_plan(m, k, nseg, n);
-    const double stream = stream_us(k, ncb, lds_path(dev, m, k, 1, static_cast<int>(ncb)));
+    const double stream = stream_us(m, k, ncb, lds_path(dev, m, k, 1, static_cast<int>(ncb)));
     return rope ? stream + 3.0 + 1.1 * static_cast<double>((ncb + 255) / 256 - 2) <= call->plan.us + 4.4
                 : stream <= call->plan.us;
 }

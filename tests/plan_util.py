@@ -17,7 +17,7 @@ extern "C" void plan_of(int m, int k, int nseg, const int* n, int batch, size_t 
     const ssa::GemmPlan p = ssa::gemm_plan(m, k, nseg, n, batch, room);
     o[0] = p.bm; o[1] = p.bn; o[2] = p.ks; o[3] = p.split_tiles; o[4] = p.tail; o[5] = static_cast<double>(p.bytes); o[6] = p.us;
 }
-extern "C" double stream_of(int k, long ncb, int staged) { return ssa::stream_us(k, ncb, staged != 0); }
+extern "C" double stream_of(int m, int k, long ncb, int staged) { return ssa::stream_us(m, k, ncb, staged != 0); }
 """
 _lib = None
 
@@ -43,7 +43,7 @@ def _load():
 
 
 def stream_us(m, k, ncb):
-    return _load().stream_of(k, ctypes.c_long(ncb), int(m <= 16 and m * k <= 32768))
+    return _load().stream_of(m, k, ctypes.c_long(ncb), int(m <= 16 and m * k <= 32768))
 
 
 def gemm_plan(m, k, n, batch=1, room=2 ** 62):
