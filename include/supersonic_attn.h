@@ -358,8 +358,9 @@ int supersonic_attn_gfx950_mixed(
  * (split-k arrival counters, which every call leaves at zero, and the GEMM's
  * tail hand-over counts, which every call leaves pairwise equal; a workspace
  * below the size leaves a k split out, but not the tail's);
- * calls sharing it must not overlap.  NULL: library-owned buffers per device
- * (grown on demand; overlapping calls on one device then race). */
+ * calls sharing it must not overlap, and may have different row counts.  NULL:
+ * library-owned buffers per device (grown on demand; overlapping calls on one
+ * device then race; no k split while `stream` is captured). */
 size_t supersonic_attn_gfx950_qkv_proj_workspace_size(
     size_t rows, size_t hidden_dim, size_t q_out_dim, size_t kv_out_dim);
 int supersonic_attn_gfx950_qkv_proj(

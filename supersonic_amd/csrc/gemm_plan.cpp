@@ -12,8 +12,9 @@ namespace ssa {
 // less than the HBM time of the operands.  The step times (s0 with few
 // workgroups, s0 + s1 with every CU busy) were fitted to 2900 timings of the
 // Q/K/V and output projections of the 8/2-, 16/4- and 16/2-head layers at 13 to
-// 8192 rows (one MI355X); over those the pick is within 0.5% of the best
-// plan on average and 9% at worst.  256 x 256 tiles stay where one round of
+// 8192 rows (one MI355X), before the copies of weights that one workgroup reads
+// passed the caches by; 240 output projections of 1 to 12 rows take 0.85 to 1.28
+// times the estimate since.  256 x 256 tiles stay where one round of
 // them holds the whole product and k is short (k = 1024, 2000 rows x 5120:
 // 37.7 us against 41.6 for 128 x 128).
 namespace {
