@@ -396,6 +396,9 @@ size_t prefill_stage_bytes(int kv_dtype, size_t kv_heads, size_t head_dim, size_
 constexpr size_t kClaimBytes = 16 * 128;
 constexpr size_t kDecodeArrivalBytes = 64 * 1024;  // a decode workspace's counters, zero between calls, at its start
 
+// Zero words, by a kernel (proj.hip): captured graphs take no memset.
+hipError_t clear_words(hipStream_t st, void* p, size_t words);
+
 // Row repack with cast and zero padding (elementwise.hip): dst row
 // (o, i) of dout elements = src[o * so + i * si + 0 .. din) cast from dtype
 // code tin to tout (0 f16, 1 f32, 2 bf16), zero past din.  Asynchronous on st.

@@ -102,8 +102,6 @@ extern "C" size_t supersonic_attn_gfx950_mixed_workspace_size(int kv_dtype, size
     if (decode && decode->batch)
         n += align256(supersonic_attn_gfx950_decode_workspace_size(decode->batch, q_heads, kv_heads, head_dim,
                                                                    decode->max_kv_len));
-    else
-        n += kDecodeArrivalBytes;
     if (chunk && chunk->chunk_len)
         n += align256(supersonic_attn_gfx950_prefill_workspace_size(kv_dtype, kv_heads, head_dim, chunk->chunk_len,
                                                                     chunk->chunk_start));
@@ -125,6 +123,7 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
     unsigned* claims = nullptr;
     void* dws = nullptr;
     void* pws = nullptr;
+    uint8_t* counters = nullptr;  // the decodes' counters, under a chunk's staging
     size_t dbytes = 0, pbytes = 0;
     if (workspace) {
         if (has_d)
@@ -142,8 +141,11 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
             dws = w + o;
             o += dbytes;
         } else if (workspace_bytes >= o + kDecodeArrivalBytes + stage) {
-            // a step without decodes leaves the counters of the steps with them alone
+            // a step without decodes leaves the counters of the steps with them
+            // alone, or, where its staging does not fit behind them, at zero
             o += kDecodeArrivalBytes;
+        } else {
+            counters = w + o;
         }
         if (has_c) {
             pws = w + o;
@@ -173,11 +175,16 @@ extern "C" int supersonic_attn_gfx950_mixed(size_t device_ordinal, void* stream,
                              decode->max_kv_len, eps, scale, decode->q_proj, decode->k_new, decode->v_new, q_norm_w,
                              k_norm_w, cos_table, sin_table, decode->positions, decode->cache, decode->out, dws,
                              dbytes, 0);
-    if (!has_d)
-        return prefill_native(device_ordinal, stream, kv_dtype, q_heads, kv_heads, head_dim, rotary_dim,
-                              chunk->chunk_len, chunk->chunk_start, eps, scale, chunk->q_proj, chunk->k_new,
-                              chunk->v_new, q_norm_w, k_norm_w, cos_table, sin_table, chunk->cache, chunk->out, pws,
-                              pbytes, nullptr);
+    if (!has_d) {
+        const int rc = prefill_native(device_ordinal, stream, kv_dtype, q_heads, kv_heads, head_dim, rotary_dim,
+                                      chunk->chunk_len, chunk->chunk_start, eps, scale, chunk->q_proj, chunk->k_new,
+                                      chunk->v_new, q_norm_w, k_norm_w, cos_table, sin_table, chunk->cache, chunk->out,
+                                      pws, pbytes, nullptr);
+        if (rc || !counters) return rc;
+        ScopedDevice scoped(dev);
+        return clear_words(static_cast<hipStream_t>(stream), counters, std::min(kDecodeArrivalBytes, pbytes) / 4) == hipSuccess
+                   ? 0 : SUPERSONIC_ERR_LAUNCH;
+    }
 
     ScopedDevice scoped(dev);
     if (!workspace) {

@@ -366,6 +366,12 @@ inline unsigned stride_blocks(size_t n) {
     return static_cast<unsigned>(b < 8192 ? (b ? b : 1) : 8192);
 }
 
+hipError_t clear_words(hipStream_t st, void* p, size_t words) {
+    hipLaunchKernelGGL(fill_u16_kernel, dim3(stride_blocks(2 * words)), dim3(256), 0, st, 2 * words,
+                       static_cast<uint16_t*>(p));
+    return hipGetLastError();
+}
+
 // Largest row count the streaming kernel takes (SUPERSONIC_PROJ_SKINNY_MAX_M,
 // default 12, at most 64, read per call); more rows go to the tiled GEMM.
 int skinny_max_m() {

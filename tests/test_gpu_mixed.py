@@ -224,14 +224,15 @@ def test_mixed_workspace_of_a_larger_chunk():
                       workspace=torch.zeros(1 << 19, dtype=torch.uint8, device=DEV), **shape)
 
 
-def test_mixed_step_without_decodes_leaves_their_counters():
+@pytest.mark.parametrize("tight", [False, True])
+def test_mixed_step_without_decodes_leaves_their_counters(tight):
     """One workspace for a step with a chunk only (its staging holds NaNs) and then steps with decodes, whose splits count
-    their arrivals in it."""
-    S, batch, Hq, Hkv, D, rot = 300, 2, 8, 2, 256, 64
+    their arrivals in it; tight: the chunk's staging takes all of it."""
+    S, batch, Hq, Hkv, D, rot = 4200 if tight else 300, 2, 8, 2, 256, 64
     announce("mixed step without decodes, then with them, one workspace")
     g = torch.Generator(device=DEV).manual_seed(93)
     rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
-    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, 4001, 1.0e7))
+    cos, sin = (t.to(DEV) for t in O.rope_tables(rot, 4201, 1.0e7))
     qw, kw = rnd(D) * 0.1, rnd(D) * 0.1
     lens = [4000, 1500]
     pos = torch.tensor(lens, dtype=torch.int32, device=DEV)
@@ -246,9 +247,10 @@ def test_mixed_step_without_decodes_leaves_their_counters():
                  out=zero(S, Hq * D), chunk_start=0)
     dec = dict(zip(("q_proj", "k_new", "v_new"), xd), cache=K.KvCache(kd.clone(), vd.clone()), out=zero(batch, Hq * D),
                positions=pos, max_kv_len=max(lens) + 1)
-    ws = torch.zeros(K.mixed_workspace_size(False, Hq, Hkv, D, chunk, dec), dtype=torch.uint8, device=DEV)
+    size = K.mixed_workspace_size(False, Hq, Hkv, D, chunk, None if tight else dec)
+    ws = torch.zeros(size, dtype=torch.uint8, device=DEV)
     K.fused_mixed(0, qw, kw, cos, sin, chunk=chunk, workspace=ws, **shape)
-    for part in (dict(chunk=chunk, decode=dec), dict(decode=dec)):
+    for part in (dict(decode=dec),) if tight else (dict(chunk=chunk, decode=dec), dict(decode=dec)):
         dec["out"].fill_(float("nan"))
         K.fused_mixed(0, qw, kw, cos, sin, workspace=ws, **part, **shape)
         torch.cuda.synchronize()
