@@ -578,24 +578,27 @@ bool rows_stream(int dev, int m, int k, int nseg, const int* n, int64_t ncb, boo
 
 // A tail split's region that the caller's is too small for is an error (a
 // status); a k split without room leaves the call to the best plan that fits.
-// Nor does a call without a workspace split k while `st` is captured: the
-// library's buffer cannot be allocated then, and a graph that held it would
-// keep its address when a larger call moves it.
+// Nor does a call without a workspace split k while `st` is captured (a tail
+// only in a buffer that is there): the library's buffer cannot be allocated
+// then, and a graph that held it would keep its address when a larger call
+// moves it.
 int plan_gemm(int dev, hipStream_t st, int m, int k, int nseg, const int* n, uint8_t* ws, size_t ws_bytes, GemmCall* call) {
     GemmPlan& plan = call->plan;
     if (plan.us == 0) plan = gemm_plan(m, k, nseg, n);  // (rows_stream may have made it)
     if (plan.bytes == 0) return 0;
     if (ws) {
         if (plan.bytes > ws_bytes) {
-            if (plan.tail > 0) return SUPERSONIC_ERR_LAUNCH;
+            // (k % 32 != 0 takes a tail split where it once had whole smaller tiles)
+            if (plan.tail > 0 && k % 32 == 0) return SUPERSONIC_ERR_LAUNCH;
             plan = gemm_plan(m, k, nseg, n, 1, ws_bytes);
         }
         call->ws = ws;
     } else {
-        if (plan.tail > 0)
-            call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceGemm));
-        else if (!stream_capturing(st))
-            call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, kWorkspaceSplit));
+        const int slot = plan.tail > 0 ? kWorkspaceGemm : kWorkspaceSplit;
+        if (!stream_capturing(st))
+            call->ws = static_cast<uint8_t*>(device_workspace(dev, plan.bytes, slot));
+        else if (plan.tail > 0 && k % 32 == 0)
+            call->ws = static_cast<uint8_t*>(device_workspace_held(dev, plan.bytes, slot));
         if (!call->ws) plan = gemm_plan(m, k, nseg, n, 1, 0);
     }
     return 0;

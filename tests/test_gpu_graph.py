@@ -288,12 +288,14 @@ def replays_equal(graph, reset, out, want):
         assert torch.equal(out, want)
 
 
-def test_o_proj_without_workspace_is_captured_cold():
-    """The first call of its size, without a workspace, under capture: nothing is allocated then, so it does not split k."""
-    rows, adim, hid = 1000, 16384, 5120
+@pytest.mark.parametrize("rows,adim,hid", [(1000, 16384, 5120), (8200, 520, 6912)])
+def test_o_proj_without_workspace_is_captured_cold(rows, adim, hid):
+    """The first call of its size, without a workspace, under capture: nothing is allocated then, so it does not split k
+    (nor, with k % 32 != 0, its last round's tiles)."""
     announce(f"o_proj without a workspace captured cold: {rows} rows {adim}->{hid}")
     plan = gemm_plan(rows, adim, (hid,))
-    assert plan.ks > 1 and plan.bytes > 48 << 20, plan  # more than any other test leaves in the library's buffer
+    # more than any other test leaves in the library's buffers
+    assert (plan.ks > 1 and plan.bytes > 48 << 20) or (plan.tail > 120 and adim % 32), plan
     g = torch.Generator(device=DEV).manual_seed(95)
     rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV, dtype=torch.bfloat16)
     attn, w, hidden = rnd(rows, adim), rnd(hid, adim) * adim ** -0.5, rnd(rows, hid)
@@ -311,6 +313,7 @@ def test_o_proj_without_workspace_is_captured_cold():
     assert bool(((h.float() - ref).abs() <= ulp(y) + ulp(ref) + 1e-6).all())
     want = h.clone()
     K.o_proj_residual(0, attn, w, hidden.clone())  # eager: now the library's buffer is there
+    torch.cuda.synchronize()
     replays_equal(graph, lambda: h.copy_(hidden), h, want)
     # and a call captured while it is there does not hold on to it
     graph2 = torch.cuda.CUDAGraph()

@@ -567,6 +567,21 @@ def test_o_proj_planned_paths(path):
     assert torch.equal(*got) and K.wait_status() == 0
 
 
+def test_o_proj_unaligned_rows_without_room_for_a_tail():
+    """k % 32 != 0, a workspace of a call with fewer rows: the tail's tiles run whole."""
+    rows, adim, hid = 8200, 264, 4608
+    announce(f"o_proj small workspace {rows} rows {adim}->{hid}")
+    assert planned_path(rows, adim, hid) == "256x256 halved tail"
+    g = gen(101)
+    attn, w, hidden = O.randn_bf16(g, rows, adim), O.randn_bf16(g, hid, adim, std=adim ** -0.5), O.randn_bf16(g, rows, hid)
+    hd = hidden.to(DEV)
+    K.o_proj_residual(0, attn.to(DEV), w.to(DEV), hd, workspace=torch.zeros(256, dtype=torch.uint8, device=DEV))
+    torch.cuda.synchronize()
+    ref = O.o_proj_residual(attn.float(), w, hidden)
+    big = torch.maximum(ref.float().abs(), (ref.float() - hidden.float()).abs())
+    assert_ulps(hd.float().cpu(), ref, 2 * ulp(big) + 1e-6, "o_proj unaligned, small workspace")
+
+
 def test_matmul_tail_split_planned():
     """The drop-in's tail hand-over (test_matmul_tail_split's shapes take smaller tiles now), twice around another tail."""
     for seed, (m, n, k) in enumerate([(8200, 4608, 512), (8200, 4608, 264), (8200, 4608, 512)]):
