@@ -98,8 +98,8 @@ enum LayerWait { kLayerGo, kLayerMissing };
 constexpr int kArriveThread = kLayerThreads - 64;
 struct LayerShared {
     int mine;                        // this workgroup got the id it is working on
-    int res;                         // grid_wait's and take_over's result
-    int first, unfinished;           // take_over's scan
+    int res;                         // grid_wait's polls and take_over's id
+    int first;                       // free_id's result
     uint16_t taken[kLayerMaxGrid];   // [1 ..]: ids taken over
 };
 // Whether this workgroup has its id, known by the time the outputs go out.
@@ -125,63 +125,72 @@ __device__ __forceinline__ void grid_arrive(unsigned* ctr, unsigned* flag, unsig
         if (prev == n - 1) __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
-// Waits for barrier `which` (0 or 1).  kLayerMissing: it lasted while arrivals
-// were missing from barrier 0.  spent: polls of the waits that ended so, in all.
-__device__ __forceinline__ LayerWait grid_wait(const LayerParams& P, int which, unsigned nwg, int& spent,
-                                               LayerShared& sh) {
-    if (threadIdx.x == 0) {
-        unsigned* const ctr = P.bar + which;
-        unsigned* const flag = P.bar + 32 + 16 * which;
-        const int patience = spent ? 8 : min(P.polls, kLayerMissingPolls);
-        auto missing = [&](unsigned* c) { return static_cast<int>(load_agent_u32(c)) < static_cast<int>(nwg); };
-        // a wait expires after P.polls polls once every arrival has been counted
-        // for kLayerMissingPolls of them (the flag follows the count)
-        int r = 0, late = 0;
-        for (int it = 0;; ++it) {
-            if (load_agent_u32(flag) != 0u) break;
-            if (it >= patience && spent < kLayerSpin && load_agent_u32(P.bar + 32) == 0u && missing(P.bar)) {
-                r = it + 1;
-                break;
-            }
-            if (it >= P.polls && !missing(ctr)) ++late;
-            if (late >= kLayerMissingPolls || it >= kLayerSpin || spent >= kLayerSpin) {
-                wait_expired(kWaitLayerBarrier);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        sh.res = r;
-    }
+// The first id from w on that no workgroup has started, as its distance from
+// w; nwg: every id is taken, nwg + 1: and has its phase 1 done.
+__device__ __forceinline__ int free_id(const LayerParams& P, int w, int nwg, LayerShared& sh) {
     __syncthreads();
-    // (the next writer of res is behind another barrier)
-    const int r = __builtin_amdgcn_readfirstlane(sh.res);
-    spent += r;
-    return r ? kLayerMissing : kLayerGo;
-}
-// Takes the next id after w that no workgroup has started; -1: there is none
-// (or another workgroup was faster).  With every id's phase 1 done, barrier 0 opens
-// whatever its counter says.
-__device__ __forceinline__ int take_over(const LayerParams& P, int w, int nwg, LayerShared& sh) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        sh.first = nwg;
-        sh.unfinished = 0;
-    }
+    if (threadIdx.x == 0) sh.first = nwg + 1;
     __syncthreads();
     for (int i = threadIdx.x; i < nwg; i += kLayerThreads) {
-        const int v = w + i < nwg ? w + i : w + i - nwg;
-        const unsigned s = load_agent_u32(P.ids + v);
-        if (s == kIdFree) atomicMin(&sh.first, i);
-        if (s != kIdProjected) sh.unfinished = 1;
+        const unsigned s = load_agent_u32(P.ids + (w + i < nwg ? w + i : w + i - nwg));
+        if (s != kIdProjected) atomicMin(&sh.first, s == kIdFree ? i : nwg);
     }
     __syncthreads();
+    return __builtin_amdgcn_readfirstlane(sh.first);
+}
+// Waits for barrier `which` (0 or 1).  kLayerMissing: it lasted, arrivals are
+// missing from barrier 0 and an id is free.  (With every id taken the wait goes
+// on, so that a decode item is not planned again; with every id's phase 1 done
+// barrier 0 opens whatever its counter says.)  spent: polls of the waits that
+// found a free id, in all.
+__device__ __forceinline__ LayerWait grid_wait(const LayerParams& P, int which, int w, unsigned nwg, int& spent,
+                                               LayerShared& sh) {
+    int at = 0, look = spent ? 8 : min(P.polls, kLayerMissingPolls);
+    for (;;) {
+        if (threadIdx.x == 0) {
+            unsigned* const ctr = P.bar + which;
+            unsigned* const flag = P.bar + 32 + 16 * which;
+            auto missing = [&](unsigned* c) { return static_cast<int>(load_agent_u32(c)) < static_cast<int>(nwg); };
+            // a wait expires after P.polls polls once every arrival has been counted
+            // for kLayerMissingPolls of them (the flag follows the count)
+            int r = 0, late = 0;
+            for (int it = at;; ++it) {
+                if (load_agent_u32(flag) != 0u) break;
+                if (it >= look && spent < kLayerSpin && load_agent_u32(P.bar + 32) == 0u && missing(P.bar)) {
+                    r = it + 1;
+                    break;
+                }
+                if (it >= P.polls && !missing(ctr)) ++late;
+                if (late >= kLayerMissingPolls || it >= kLayerSpin || spent >= kLayerSpin) {
+                    wait_expired(kWaitLayerBarrier);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            sh.res = r;
+        }
+        __syncthreads();
+        at = __builtin_amdgcn_readfirstlane(sh.res);
+        if (at == 0) return kLayerGo;
+        const int f = free_id(P, w, static_cast<int>(nwg), sh);
+        if (f < static_cast<int>(nwg)) {
+            spent += at;
+            return kLayerMissing;
+        }
+        if (f > static_cast<int>(nwg) && threadIdx.x == 0)
+            __hip_atomic_store(P.bar + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        look = at + kLayerMissingPolls;
+    }
+}
+// Takes the next id after w that no workgroup has started; -1: there is none
+// any more.
+__device__ __forceinline__ int take_over(const LayerParams& P, int w, int nwg, LayerShared& sh) {
+    const int f = free_id(P, w, nwg, sh);
     if (threadIdx.x == 0) {
         int v = -1;
-        if (sh.first < nwg) {
-            v = w + sh.first < nwg ? w + sh.first : w + sh.first - nwg;
+        if (f < nwg) {
+            v = w + f < nwg ? w + f : w + f - nwg;
             if (atomicCAS(P.ids + v, static_cast<unsigned>(kIdFree), static_cast<unsigned>(kIdTaken)) != kIdFree) v = -1;
-        } else if (!sh.unfinished) {
-            __hip_atomic_store(P.bar + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         sh.res = v;
     }
@@ -191,7 +200,7 @@ __device__ __forceinline__ int take_over(const LayerParams& P, int w, int nwg, L
 
 // The kernel's arguments, read again where they are asked for: kept in scalar
 // registers around the loops below they spill (259 of them, and 39 vector
-// registers with them; 59 and none so).
+// registers with them; 57 and none so).
 __device__ __forceinline__ const LayerParams& layer_args() {
     typedef const __attribute__((address_space(4))) LayerParams* Kernarg;
     uint64_t a = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
@@ -271,7 +280,7 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
             const DecodeParams dec = P.dec;
             bool had_item = false;
             decode_split_body<bf16_t, FP8, D, 4, true>(dec, item_of(u), 0, 0, lds.d, [&]() {
-                res = grid_wait(P, 0, nwg, spent, sh);
+                res = grid_wait(P, 0, w, nwg, spent, sh);
                 had_item = true;
                 return res == kLayerGo;
             });
@@ -298,7 +307,7 @@ __global__ __launch_bounds__(kLayerThreads) void decode_layer_kernel(LayerParams
             stores_complete();
             grid_arrive(&P.bar[1], &P.bar[48], nwg);
         }
-        if (res == kLayerGo && has_op) res = grid_wait(P, 1, nwg, spent, sh);
+        if (res == kLayerGo && has_op) res = grid_wait(P, 1, w, nwg, spent, sh);
         if (res == kLayerGo) {
             // 3. output projection + residual
             for (int i = 0; i < n_ids; ++i) {
